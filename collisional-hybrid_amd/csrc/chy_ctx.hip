@@ -613,7 +613,7 @@ int chy_create(const chy_params *prm_in, int64_t np_capacity, chy_ctx **out)
     A(dalloc(ctx, &q, (int64_t)ts * 3 * nc)); ctx->pc_buf = q;
   }
   A(dalloc(ctx, &ctx->red, (int64_t)kRedBlocks * 32));
-  A(dalloc(ctx, &ctx->rpl, lhs_zsum_blocks(g, false)));
+  A(dalloc(ctx, &ctx->rpl, std::max(lhs_zsum_blocks(g, false), lhs_zsum_blocks(g, ctx->mixed))));
   ctx->red_out_n = 3 * (ctx->restart + 2) + 16;
   A(dalloc(ctx, &ctx->red_out, ctx->red_out_n));
   // the mirror is coherent host memory: device writes reach it without a copy

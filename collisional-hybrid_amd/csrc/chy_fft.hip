@@ -927,7 +927,7 @@ static H2 h2_layout(const chy_ctx *ctx, bool fp32)
   h.nb = nb2_of(nxy);
   h.nlb = lhs_zsum_blocks(ctx->g, fp32);
   h.part = ctx->pc2_h;
-  h.pl = h.part + (int64_t)lhs_zchunks(ctx->g) * nxy;
+  h.pl = h.part + (int64_t)lhs_zchunks(ctx->g, fp32) * nxy;
   h.pn = h.pl + h.nlb;
   h.p1 = h.pn + (int64_t)(kHm + 1) * h.nb;
   h.p2 = h.p1 + (int64_t)kHm * kHm * h.nb;
@@ -939,8 +939,8 @@ int64_t fft2_h_elems(const chy_ctx *ctx)
 {
   const int64_t nxy = (int64_t)ctx->g.nx * ctx->g.ny;
   const int nb = nb2_of(nxy);
-  const int64_t nlb = std::max(lhs_zsum_blocks(ctx->g, false), lhs_zsum_blocks(ctx->g, true));
-  return (int64_t)lhs_zchunks(ctx->g) * nxy + nlb + (int64_t)(kHm + 1) * nb +
+  const bool fp32 = ctx->mixed;
+  return (int64_t)lhs_zchunks(ctx->g, fp32) * nxy + lhs_zsum_blocks(ctx->g, fp32) + (int64_t)(kHm + 1) * nb +
          2 * (int64_t)kHm * kHm * nb + kHm;
 }
 
@@ -1233,7 +1233,7 @@ int fft2_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z, T *w3, b
   const int nb = h.nb;
   // z-averaged residual of the first level, mean removed, into V0
   launch_lhs_zsum<T>(ctx, ctx->prm.lhs_type, (const T *)ctx->mom[0], z, r, h.part, h.pl, fused ? w3 : nullptr);
-  hipLaunchKernelGGL((k2_r2<T>), nb, 256, 0, ctx->stream, nxy, nz, lhs_zchunks(ctx->g), (const double *)h.part,
+  hipLaunchKernelGGL((k2_r2<T>), nb, 256, 0, ctx->stream, nxy, nz, lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part,
                      (const double *)h.pl, h.nlb, V, h.pn);
   Symbol sym = make_symbol(ctx, v19);
   sym.inv_scale = 1.0 / (double)nxy;

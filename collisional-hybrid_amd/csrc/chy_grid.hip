@@ -7,6 +7,7 @@
 // shaped for coalesced x-fastest access; FP64 kernels use the oracle's
 // operation order (the library is built with -ffp-contract=off).
 #include <cmath>
+#include <utility>
 
 #include "chy_internal.h"
 
@@ -105,6 +106,21 @@ __device__ __forceinline__ void row_coeffs(const Grid &g, int lhs_type, const SC
 
 struct LapRow { double v[19]; };
 
+// kOff for compile-time indices, and f(q) for q = 0 .. 18 in order
+static constexpr int cOff[19][3] = {
+  {+1, 0, 0}, {-1, 0, 0}, {0, +1, 0}, {0, -1, 0}, {0, 0, +1}, {0, 0, -1},
+  {+1, +1, 0}, {+1, -1, 0}, {-1, +1, 0}, {-1, -1, 0},
+  {+1, 0, +1}, {+1, 0, -1}, {-1, 0, +1}, {-1, 0, -1},
+  {0, +1, +1}, {0, +1, -1}, {0, -1, +1}, {0, -1, -1},
+  {0, 0, 0}};
+template <typename F, int... Q>
+__device__ __forceinline__ void each_q(F &&f, std::integer_sequence<int, Q...>)
+{
+  (f(std::integral_constant<int, Q>()), ...);
+}
+// periodic index for i in [-2, n + 1], n >= 3
+__device__ __forceinline__ int wrap2(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
+
 // y = A x (FP64: oracle order sum_q v_q x_q; FP32: difference form
 // sum_q v_q (x_q - x_c), exact in exact arithmetic because rows sum to zero).
 template <typename TN, typename TX, typename TY, typename C, bool DIFF>
@@ -128,48 +144,49 @@ __global__ __launch_bounds__(256) void k_lhs_apply(Grid g, int lhs_type, SCoef s
   y[c] = (TY)acc;
 }
 
-// res = b - A x, one thread per node (grids too small for the tiled kernel's
-// tiles to fill the chip: the multigrid's coarse levels); the row sum as
-// k_lhs_apply forms it.
-template <typename T, typename C, bool DIFF>
-__global__ __launch_bounds__(256) void k_residual_node(Grid g, int lhs_type, SCoef s, LapRow lap,
-                                                       const T *__restrict__ n, const T *__restrict__ b,
-                                                       const T *__restrict__ x, T *__restrict__ res)
+// Entry Q of row r from the densities around it, nat(dx, dy, dz) relative to
+// r: row_from_star's entry alone.
+template <typename C, int Q, typename F>
+__device__ __forceinline__ C row_entry(const SCoef &s, F nat)
 {
-  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= g.nc) return;
-  const int i = (int)(c % g.nx), j = (int)((c / g.nx) % g.ny), k = (int)(c / ((int64_t)g.nx * g.ny));
   C v[19];
-  row_coeffs<C, T>(g, lhs_type, s, lap.v, n, i, j, k, v);
-  C acc = (C)0;
-  if (DIFF) {
-    const C xc = (C)x[c];
-#pragma unroll
-    for (int q = 0; q < 18; q++) acc += v[q] * ((C)x[lin(g, i + kOff[q][0], j + kOff[q][1], k + kOff[q][2])] - xc);
-  } else {
-#pragma unroll
-    for (int q = 0; q < 19; q++) acc += v[q] * (C)x[lin(g, i + kOff[q][0], j + kOff[q][1], k + kOff[q][2])];
-  }
-  res[c] = (T)((C)b[c] - acc);
+  const C n0 = nat(0, 0, 0);
+  const C xp = nat(1, 0, 0), xm = nat(-1, 0, 0), yp = nat(0, 1, 0), ym = nat(0, -1, 0), zp = nat(0, 0, 1),
+          zm = nat(0, 0, -1);
+  row_from_star<C>(s, n0, xp, xm, yp, ym, zp, zm, v);  // (the other entries are dead code)
+  return v[Q];
 }
 
 // y = A^T x: (A^T x)_c = sum_q A[c - o_q, c] x[c - o_q]; the coefficient of
 // column c in row r = c - o_q is that row's entry q.
-template <typename TN, typename TX, typename TY, typename C>
-__global__ __launch_bounds__(256) void k_lhs_apply_t(Grid g, int lhs_type, SCoef s, LapRow lap, const TN *__restrict__ n,
+template <typename TN, typename TX, typename TY, typename C, bool FULL>
+__global__ __launch_bounds__(256) void k_lhs_apply_t(Grid g, SCoef s, LapRow lap, const TN *__restrict__ n,
                                                      const TX *__restrict__ x, TY *__restrict__ y)
 {
   const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.nc) return;
-  const int i = (int)(c % g.nx), j = (int)((c / g.nx) % g.ny), k = (int)(c / ((int64_t)g.nx * g.ny));
-  C acc = (C)0;
-#pragma unroll 1
-  for (int q = 0; q < 19; q++) {
-    const int ri = i - kOff[q][0], rj = j - kOff[q][1], rk = k - kOff[q][2];
-    C v[19];
-    row_coeffs<C, TN>(g, lhs_type, s, lap.v, n, ri, rj, rk, v);
-    acc += v[q] * (C)x[lin(g, ri, rj, rk)];
+  int i, j, k;
+  split_cell(g, (int)c, i, j, k);
+  // indices of the two nodes on each side (a row's star reaches one past its node)
+  int64_t ox[5], oy[5], oz[5];
+#pragma unroll
+  for (int d = -2; d <= 2; d++) {
+    ox[d + 2] = wrap2(i + d, g.nx);
+    oy[d + 2] = (int64_t)g.nx * wrap2(j + d, g.ny);
+    oz[d + 2] = (int64_t)g.nx * g.ny * wrap2(k + d, g.nz);
   }
+  C acc = (C)0;
+  auto term = [&](auto q_) {
+    constexpr int q = decltype(q_)::value;
+    constexpr int rx = -cOff[q][0], ry = -cOff[q][1], rz = -cOff[q][2];  // row r = c + (rx, ry, rz)
+    C v;
+    if constexpr (FULL)
+      v = row_entry<C, q>(s, [&](int a, int b, int d) { return (C)n[ox[rx + a + 2] + oy[ry + b + 2] + oz[rz + d + 2]]; });
+    else
+      v = (C)lap.v[q];
+    acc += v * (C)x[ox[rx + 2] + oy[ry + 2] + oz[rz + 2]];
+  };
+  each_q(term, std::make_integer_sequence<int, 19>());
   y[c] = (TY)acc;
 }
 
@@ -448,6 +465,186 @@ void k_lhs_tiled(Grid g, int lhs_type, SCoef s, LapRow lap,
   }
 }
 
+// ---- column stencil --------------------------------------------------------------
+// One thread per (i, j) column of a chunk of planes, no LDS and no barriers:
+// each group of kColZ planes loads its stencil straight from the caches (the
+// x-y neighbours are other lanes' centres, so L1 and L2 serve them) with every
+// load of the group in flight at once, and the z neighbours are shared between
+// the group's planes in registers.
+//
+// On grids that fit the caches the tiled kernel below is bound by its serial
+// march through 16 planes (two barriers a plane) on few tiles: 8 blocks at
+// 32^3, 128 at 128^3.  Here a launch has 1024 blocks where the grid gives them
+// (chunks of 4 to 16 planes).  Measured, tiled -> column, us per pass of A x:
+// 32^3 FP64 25.7 -> 5.3, 64^3 FP32 20.5 -> 4.6, 128^3 FP32 21.6 -> 9.4, 128^3
+// FP64 28.4 -> 20.0, 256x256x64 FP32 22.9 -> 14.9; with B oblique 128^3 FP32
+// 35.0 -> 10.6.  Larger grids: 15 loads a node (FP64 twice the bytes) reach
+// the L1's rate before the tiles' LDS does: 256x256x64 FP64 30.3 -> 39.3,
+// 256x256x128 FP32 27.9 -> 28.6 (column sums 44.7 -> 30.0), 256^3 FP32 53 ->
+// 72 and FP64 99 -> 199.  col_stencil draws the line between them.  Four planes
+// a group measured best or level for both types (1, 2, 4 and 8 tried).
+constexpr int kColZ = 4;
+static inline bool col_stencil(const Grid &g, bool fp32) { return g.nc <= (fp32 ? (int64_t)1 << 23 : (int64_t)1 << 21); }
+
+// Planes per chunk: 1024 blocks of columns, in whole groups, at most kZChunk
+static inline int col_chunk(const Grid &g)
+{
+  const int64_t nb = ((int64_t)g.nx * g.ny + 255) / 256;
+  const int64_t zc = (g.nz * nb + 1023) / 1024;
+  return (int)std::min<int64_t>(kZChunk, (zc + kColZ - 1) / kColZ * kColZ);
+}
+
+static inline dim3 col_grid(const Grid &g)
+{
+  const int zc = col_chunk(g);
+  return dim3((unsigned)(((int64_t)g.nx * g.ny + 255) / 256), (unsigned)((g.nz + zc - 1) / zc));
+}
+
+enum { kOpKz, kOpFull, kOpConst };  // the full operator with B along z, any B, a constant row
+// base + a 32-bit byte offset within a plane (a plane of 4 GB does not fit
+// beside the solver's vectors), so that the plane's address stays scalar
+template <typename T>
+__device__ __forceinline__ T ld_off(const T *__restrict__ base, uint32_t byte_off)
+{
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + byte_off);
+}
+
+template <typename TN, typename TX, typename TY, typename C, bool DIFF, int OUT, typename TB, int OP>
+__global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow lap, const TN *__restrict__ n,
+                                                 const TX *__restrict__ x, const TB *__restrict__ b,
+                                                 TY *__restrict__ y, double *__restrict__ pl, TX *__restrict__ d3)
+{
+  constexpr bool ZS = OUT == 2 || OUT == 4, KZ = OP == kOpKz;
+  constexpr int ZR = kColZ;
+  uint32_t bx, by, bz;
+  const uint32_t tile = xcd_tile(bx, by, bz);
+  const int64_t pstride = (int64_t)g.nx * g.ny;
+  const int col = (int)(bx * 256 + threadIdx.x);
+  const bool live = col < (int)pstride;
+  int i, j, k_;
+  split_cell(g, live ? col : 0, i, j, k_);
+  const int ip = i + 1 == g.nx ? 0 : i + 1, im = i == 0 ? g.nx - 1 : i - 1;
+  const int jp = j + 1 == g.ny ? 0 : j + 1, jm = j == 0 ? g.ny - 1 : j - 1;
+  const uint32_t c0 = (uint32_t)(i + g.nx * j), cxp = (uint32_t)(ip + g.nx * j), cxm = (uint32_t)(im + g.nx * j),
+                 cyp = (uint32_t)(i + g.nx * jp), cym = (uint32_t)(i + g.nx * jm),
+                 cpp = (uint32_t)(ip + g.nx * jp), cpm = (uint32_t)(ip + g.nx * jm),
+                 cmp = (uint32_t)(im + g.nx * jp), cmm = (uint32_t)(im + g.nx * jm);
+  const int z0 = (int)by * zc, z1 = z0 + zc < g.nz ? z0 + zc : g.nz;
+  double zs = 0.0;
+  if (live) {
+    for (int k0 = z0; k0 < z1; k0 += ZR) {
+      // planes k0 - 1 .. k0 + ZR: the centre, and (unless KZ) the four face neighbours
+      C xc[ZR + 2], nc[ZR + 2], xf[ZR + 2][4], xe[ZR][4], nf[ZR][4];
+      TB rb[ZR];
+#pragma unroll
+      for (int u = 0; u < ZR + 2; u++) {
+        int k = k0 - 1 + u;
+        if (k > z1) k = z1;  // past the chunk: any plane in range
+        const int64_t pb = pstride * wrapi(k, g.nz);
+        const TX *xp = x + pb;
+        const TN *np = n + pb;
+        xc[u] = (C)ld_off(xp, c0 * (uint32_t)sizeof(TX));
+        if (OP != kOpConst) nc[u] = (C)ld_off(np, c0 * (uint32_t)sizeof(TN));
+        const bool inner = u >= 1 && u <= ZR;
+        if (inner || !KZ) {
+          xf[u][0] = (C)ld_off(xp, cxp * (uint32_t)sizeof(TX));
+          xf[u][1] = (C)ld_off(xp, cxm * (uint32_t)sizeof(TX));
+          xf[u][2] = (C)ld_off(xp, cyp * (uint32_t)sizeof(TX));
+          xf[u][3] = (C)ld_off(xp, cym * (uint32_t)sizeof(TX));
+        }
+        if (inner) {
+          const int v = u - 1;
+          xe[v][0] = (C)ld_off(xp, cpp * (uint32_t)sizeof(TX));
+          xe[v][1] = (C)ld_off(xp, cpm * (uint32_t)sizeof(TX));
+          xe[v][2] = (C)ld_off(xp, cmp * (uint32_t)sizeof(TX));
+          xe[v][3] = (C)ld_off(xp, cmm * (uint32_t)sizeof(TX));
+          if (OP != kOpConst) {
+            nf[v][0] = (C)ld_off(np, cxp * (uint32_t)sizeof(TN));
+            nf[v][1] = (C)ld_off(np, cxm * (uint32_t)sizeof(TN));
+            nf[v][2] = (C)ld_off(np, cyp * (uint32_t)sizeof(TN));
+            nf[v][3] = (C)ld_off(np, cym * (uint32_t)sizeof(TN));
+          }
+          if (OUT != 0) rb[v] = ld_off(b + pb, c0 * (uint32_t)sizeof(TB));
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < ZR; v++) {
+        const int u = v + 1, k = k0 + v;
+        if (k >= z1) break;
+        C acc = (C)0;
+        if constexpr (KZ) {
+          const C sxx = (C)s.sxx, syy = (C)s.syy, szz = (C)s.szz, sxy = (C)s.sxy, syx = (C)s.syx;
+          const C n0 = nc[u], nxp = nf[v][0], nxm = nf[v][1], nyp = nf[v][2], nym = nf[v][3], nzp = nc[u + 1],
+                  nzm = nc[u - 1];
+          // entries 0-9 and 18 of row_from_star with s_xz = s_yz = s_zx = s_zy = 0
+          const C a = nxp + n0, bq = n0 + nxm, cq = nyp + n0, dq = n0 + nym;
+          const C dy = nyp - nym, dx = nxp - nxm;
+          C w[10];
+          w[0] = mad(sxx, a, syx * dy);
+          w[1] = mad(sxx, bq, -(syx * dy));
+          w[2] = mad(syy, cq, sxy * dx);
+          w[3] = mad(syy, dq, -(sxy * dx));
+          w[4] = szz * (nzp + n0);
+          w[5] = szz * (n0 + nzm);
+          w[6] = mad(sxy, a, syx * cq);
+          w[7] = mad(-sxy, a, -(syx * dq));
+          w[8] = mad(-sxy, bq, -(syx * cq));
+          w[9] = mad(sxy, bq, syx * dq);
+          // -((sxx X + syy Y) + szz Z), the oracle's association
+          const C w18 = -(mad(szz, nzp + 2 * n0 + nzm, mad(sxx, nxp + 2 * n0 + nxm, syy * (nyp + 2 * n0 + nym))));
+          const C xv[10] = {xf[u][0], xf[u][1], xf[u][2], xf[u][3], xc[u + 1], xc[u - 1],
+                            xe[v][0], xe[v][1], xe[v][2], xe[v][3]};
+          if (DIFF) {
+#pragma unroll
+            for (int q = 0; q < 10; q++) acc = mad(w[q], xv[q] - xc[u], acc);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 10; q++) acc += w[q] * xv[q];
+            acc += w18 * xc[u];
+          }
+        } else {
+          C w[19];
+          if constexpr (OP == kOpFull) {
+            row_from_star<C>(s, nc[u], nf[v][0], nf[v][1], nf[v][2], nf[v][3], nc[u + 1], nc[u - 1], w);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 19; q++) w[q] = (C)lap.v[q];
+          }
+          const C xv[19] = {xf[u][0],     xf[u][1],     xf[u][2],     xf[u][3],     xc[u + 1],    xc[u - 1],    xe[v][0],
+                            xe[v][1],     xe[v][2],     xe[v][3],     xf[u + 1][0], xf[u - 1][0], xf[u + 1][1], xf[u - 1][1],
+                            xf[u + 1][2], xf[u - 1][2], xf[u + 1][3], xf[u - 1][3], xc[u]};
+          if (DIFF) {
+#pragma unroll
+            for (int q = 0; q < 18; q++) acc = mad(w[q], xv[q] - xv[18], acc);
+          } else {
+#pragma unroll
+            for (int q = 0; q < 19; q++) acc += w[q] * xv[q];
+          }
+        }
+        const int64_t c = (int64_t)c0 + pstride * k;
+        if (OUT == 0) y[c] = (TY)acc;
+        else {
+          const double rv = (double)rb[v] - (double)acc;
+          if (OUT == 1 || OUT == 3) y[c] = (TY)rv;
+          if (OUT == 4) d3[c] = (TX)rv;
+          if (ZS) zs += rv;
+          if (OUT == 3) zs += rv * rv;
+        }
+      }
+    }
+    if (ZS) y[(int64_t)by * pstride + c0] = (TY)zs;
+  }
+  if (ZS || OUT == 3) {
+    __shared__ double wsum[4];
+    double t = zs;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) pl[tile] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+  }
+}
+
 static inline dim3 tiled_grid(const Grid &g, int tw = kTX)
 {
   const int ty = tw == 256 ? 8 : kTY;
@@ -477,11 +674,22 @@ static inline bool kz_operator(int lhs_type, const SCoef &s)
   return lhs_type == CHY_LHS_FULL && s.sxz == 0.0 && s.syz == 0.0 && s.szx == 0.0 && s.szy == 0.0;
 }
 
-// One tiled stencil pass on grid g, the B-along-z instantiation when it applies.
+// One stencil pass on grid g: the column kernel on grids it suits, else the tiled
+// one; the B-along-z instantiation when it applies.
 template <typename TN, typename TX, typename TY, typename C, bool DIFF, int OUT, typename TB = double, int TW = kTX>
 static void launch_tiled_on(chy_ctx *ctx, const Grid &g, const SCoef &s, const LapRow &L, int lhs_type, const TN *n,
                             const TX *x, const TB *b, TY *y, double *pl, TX *d3 = nullptr)
 {
+  if (col_stencil(g, sizeof(C) == 4)) {
+#define COLK(OP)                                                                                                  \
+  hipLaunchKernelGGL((k_lhs_col<TN, TX, TY, C, DIFF, OUT, TB, OP>), col_grid(g), 256, 0, ctx->stream, g, col_chunk(g), \
+                     s, L, n, x, b, y, pl, d3)
+    if (kz_operator(lhs_type, s)) COLK(kOpKz);
+    else if (lhs_type == CHY_LHS_FULL) COLK(kOpFull);
+    else COLK(kOpConst);
+#undef COLK
+    return;
+  }
   if (kz_operator(lhs_type, s))
     hipLaunchKernelGGL((k_lhs_tiled<TN, TX, TY, C, DIFF, OUT, TB, TW, true>), tiled_grid(g, TW), kBlock, 0,
                        ctx->stream, g, lhs_type, s, L, n, x, b, y, pl, d3);
@@ -508,16 +716,25 @@ void launch_lhs_apply(chy_ctx *ctx, int lhs_type, bool transpose, const TN *n, c
   constexpr bool fp32 = sizeof(TX) == 4 && sizeof(TY) == 4;
   using C = typename std::conditional<fp32, float, double>::type;
   if (transpose)
-    hipLaunchKernelGGL((k_lhs_apply_t<TN, TX, TY, C>), nblocks(ctx->g.nc), kBlock, 0, ctx->stream, ctx->g,
-                       lhs_type, s, L, n, x, y);
+  {
+    if (lhs_type == CHY_LHS_FULL)
+      hipLaunchKernelGGL((k_lhs_apply_t<TN, TX, TY, C, true>), nblocks(ctx->g.nc), kBlock, 0, ctx->stream, ctx->g, s,
+                         L, n, x, y);
+    else
+      hipLaunchKernelGGL((k_lhs_apply_t<TN, TX, TY, C, false>), nblocks(ctx->g.nc), kBlock, 0, ctx->stream, ctx->g, s,
+                         L, n, x, y);
+  }
   else
     launch_tiled<TN, TX, TY, C, fp32, 0>(ctx, lhs_type, n, x, (const double *)nullptr, y, (double *)nullptr);
 }
 
-int lhs_zchunks(const Grid &g) { return (g.nz + kZChunk - 1) / kZChunk; }
+int lhs_zchunks(const Grid &g, bool fp32)
+{
+  return col_stencil(g, fp32) ? (int)col_grid(g).y : (g.nz + kZChunk - 1) / kZChunk;
+}
 int64_t lhs_zsum_blocks(const Grid &g, bool fp32)
 {
-  const dim3 d = tiled_grid(g, wide_rows(g, fp32) ? 256 : kTX);
+  const dim3 d = col_stencil(g, fp32) ? col_grid(g) : tiled_grid(g, wide_rows(g, fp32) ? 256 : kTX);
   return (int64_t)d.x * d.y * d.z;
 }
 
@@ -1974,11 +2191,6 @@ void launch_residual_g(chy_ctx *ctx, const Grid &g, const double d[3], int lhs_t
   uniform_row(lhs_type == CHY_LHS_FULL ? CHY_LHS_IDENTITY : lhs_type, d, ctx->prm.kappa_e, 0.0, L.v);
   constexpr bool fp32 = sizeof(T) == 4;
   using C = typename std::conditional<fp32, float, double>::type;
-  if ((int64_t)g.nx * g.ny <= 16384) {  // few x-y tiles: one thread per node fills the chip better
-    hipLaunchKernelGGL((k_residual_node<T, C, fp32>), nblocks(g.nc), kBlock, 0, ctx->stream, g, lhs_type, s, L, n,
-                       b, x, res);
-    return;
-  }
   launch_tiled_on<T, T, T, C, fp32, 1, T>(ctx, g, s, L, lhs_type, n, x, b, res, (double *)nullptr);
 }
 

@@ -278,8 +278,8 @@ int64_t launch_residual_sq(chy_ctx *ctx, int lhs_type, const T *n, const T *b, c
 template <typename T>
 void launch_lhs_zsum(chy_ctx *ctx, int lhs_type, const T *n, const T *x, const T *b, double *part, double *pl,
                      T *r = nullptr);
-int lhs_zchunks(const Grid &g);
-int64_t lhs_zsum_blocks(const Grid &g, bool fp32);  // FP32 or FP64 stencil's grid
+int lhs_zchunks(const Grid &g, bool fp32);          // of the FP32 or FP64 stencil
+int64_t lhs_zsum_blocks(const Grid &g, bool fp32);
 template <typename T>
 void launch_efield(chy_ctx *ctx, const double *phi, T *E4);
 template <typename T>

@@ -1,0 +1,35 @@
+"""Kernels at the sizes where their tiling can go wrong: block edges,
+remainders, the smallest grids and both sides of each dispatch rule."""
+import numpy as np
+import pytest
+
+import orc
+from gpu_cases import context, grid_of, opts, vlasov_from
+
+pytestmark = pytest.mark.gpu
+
+
+def _moments(g, rng, amp=0.2):
+    n = 1 + amp * rng.uniform(-1, 1, g.nc)
+    return [n] + [0.1 * rng.standard_normal(g.nc) for _ in range(3)]
+
+
+# one block of columns is 256, a group of planes 4; the 128-plane grid is the
+# largest of the FP64 column stencil, the 129-plane one goes to the tiles
+@pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5", "--lhs-type laplacian"])
+@pytest.mark.parametrize("N", [(3, 3, 3), (16, 16, 4), (17, 15, 9), (257, 3, 7), (40, 24, 33), (128, 128, 128),
+                               (128, 128, 129)])
+def test_stencil_is_the_oracles_bit_for_bit(N, extra):
+    rng = np.random.default_rng(11)
+    with context(opts(N, extra=extra)) as ctx:
+        g = grid_of(ctx.prm)
+        mom = _moments(g, rng)
+        ctx.set_moments(vlasov_from(mom))
+        x = rng.standard_normal(g.nc)
+        y = ctx.lhs_apply(x)
+        yt = ctx.lhs_apply(x, transpose=True)
+        K, lt = list(ctx.prm.kappa_e), ctx.prm.lhs_type
+    assert np.array_equal(y, orc.lhs_apply(g, K, mom[0], x, lhs_type=lt))
+    ref = orc.lhs_apply(g, K, mom[0], x, lhs_type=lt, transpose=True)
+    # the oracle scatters its rows: the same 19 products a node, in another order
+    assert np.abs(yt - ref).max() <= 19 * 2.0 ** -52 * np.abs(ref).max() * 19
