@@ -1117,6 +1117,46 @@ __global__ __launch_bounds__(256) void k2_gs_pass(int64_t nxy, int j, T *__restr
   if (threadIdx.x < nv) pout[(int64_t)threadIdx.x * nb + blockIdx.x] = o[threadIdx.x];
 }
 
+// Givens QR of the Hessenberg columns h[q][j] (q <= j) with subdiagonals
+// sub[j + 1] = |V_{j+1}|, sub[0] = beta, and back substitution: y[q], q < kHm
+// (zero past a breakdown).
+__device__ __forceinline__ void h2_lstsq(const double (&sub)[kHm + 1], const double (&hc)[kHm][kHm], double *y)
+{
+  double H[kHm][kHm], g[kHm + 1], cs[kHm], sn[kHm], yy[kHm];
+  for (int q = 0; q <= kHm; q++) g[q] = 0.0;
+  for (int q = 0; q < kHm; q++) yy[q] = 0.0;
+  int jm = 0;
+  if (sub[0] > 0.0) {
+    g[0] = sub[0];
+    for (int j = 0; j < kHm; j++) {
+      double h[kHm + 1];
+      for (int q = 0; q <= j; q++) h[q] = hc[q][j];
+      h[j + 1] = sub[j + 1];
+      const bool more = h[j + 1] > 0.0;
+      for (int q = 0; q < j; q++) {
+        const double t = cs[q] * h[q] + sn[q] * h[q + 1];
+        h[q + 1] = -sn[q] * h[q] + cs[q] * h[q + 1];
+        h[q] = t;
+      }
+      const double rr = sqrt(h[j] * h[j] + h[j + 1] * h[j + 1]);
+      cs[j] = rr > 0.0 ? h[j] / rr : 1.0;
+      sn[j] = rr > 0.0 ? h[j + 1] / rr : 0.0;
+      h[j] = rr;
+      g[j + 1] = -sn[j] * g[j];
+      g[j] = cs[j] * g[j];
+      for (int q = 0; q <= j; q++) H[q][j] = h[q];
+      jm = j + 1;
+      if (!more) break;
+    }
+    for (int q = jm - 1; q >= 0; q--) {
+      double s = g[q];
+      for (int r = q + 1; r < jm; r++) s -= H[q][r] * yy[r];
+      yy[q] = H[q][q] != 0.0 ? s / H[q][q] : 0.0;
+    }
+  }
+  for (int q = 0; q < kHm; q++) y[q] = yy[q];
+}
+
 // Hessenberg columns from the partials, Givens QR and back substitution
 // (one block): y[q], q < kHm (zero past a breakdown).
 // (Every sum is formed as sum_partials forms it, so the values are those the
@@ -1143,50 +1183,239 @@ __global__ __launch_bounds__(256) void k2_solve(const double *__restrict__ pn, c
   }
   block_sums<kNSums>(a, kNSums, red);
   if (threadIdx.x != 0) return;
-  double n2[kHm + 1], h1[kHm][kHm], h2[kHm][kHm];
-  {
-    int t = 0;
-    for (int j = 0; j <= kHm; j++) n2[j] = red[t++];
-    for (int j = 0; j < kHm; j++)
-      for (int q = 0; q <= j; q++) {
-        h1[j][q] = red[t++];
-        h2[j][q] = red[t++];
-      }
-  }
-  double H[kHm][kHm], g[kHm + 1], cs[kHm], sn[kHm], yy[kHm];
-  for (int q = 0; q <= kHm; q++) g[q] = 0.0;
-  for (int q = 0; q < kHm; q++) yy[q] = 0.0;
-  const double beta = sqrt(n2[0]);
-  int jm = 0;
-  if (beta > 0.0) {
-    g[0] = beta;
-    for (int j = 0; j < kHm; j++) {
-      double h[kHm + 1];
-      for (int q = 0; q <= j; q++) h[q] = h1[j][q] + h2[j][q];
-      h[j + 1] = sqrt(n2[j + 1]);
-      const bool more = h[j + 1] > 0.0;
-      for (int q = 0; q < j; q++) {
-        const double t = cs[q] * h[q] + sn[q] * h[q + 1];
-        h[q + 1] = -sn[q] * h[q] + cs[q] * h[q + 1];
-        h[q] = t;
-      }
-      const double rr = sqrt(h[j] * h[j] + h[j + 1] * h[j + 1]);
-      cs[j] = rr > 0.0 ? h[j] / rr : 1.0;
-      sn[j] = rr > 0.0 ? h[j + 1] / rr : 0.0;
-      h[j] = rr;
-      g[j + 1] = -sn[j] * g[j];
-      g[j] = cs[j] * g[j];
-      for (int q = 0; q <= j; q++) H[q][j] = h[q];
-      jm = j + 1;
-      if (!more) break;
+  double sub[kHm + 1], hc[kHm][kHm];
+  int t = 0;
+  for (int j = 0; j <= kHm; j++) sub[j] = sqrt(red[t++]);
+  for (int j = 0; j < kHm; j++)
+    for (int q = 0; q <= j; q++) {
+      hc[q][j] = red[t] + red[t + 1];
+      t += 2;
     }
-    for (int q = jm - 1; q >= 0; q--) {
-      double s = g[q];
-      for (int r = q + 1; r < jm; r++) s -= H[q][r] * yy[r];
-      yy[q] = H[q][q] != 0.0 ? s / H[q][q] : 0.0;
+  h2_lstsq(sub, hc, y);
+}
+
+// ---- the whole 2-D correction in one workgroup ------------------------------------
+// On a plane of at most kPlaneMax nodes every kernel of the correction is a
+// launch of a few microseconds of latency: fourteen of them, 4 to 5 us each.
+// One workgroup of 1024 threads does them all: the columns it owns (P per
+// thread) stay in registers, the plane being transformed sits in LDS, and the
+// global sums are block sums.  It takes 20 us at 32^2 and 38 (FP32) or 49 us
+// (FP64) at 64^2; the launches take about 60 us there, and 15 to 20 us of gaps
+// between them.  (One CU does this work: at 128^2 it would take longer than
+// the launches.)  What bounds it is the latency of some 60 barriers and the
+// LDS round trips of the transforms between them.
+constexpr int kPlaneMax = 4096, kPlaneT = 1024, kPlaneP = kPlaneMax / kPlaneT;
+constexpr int kPlanePad = 1024;  // most lines of a plane (axes of 4 nodes and more): one pad value each
+
+// Radix-4 butterflies on x[0..3] (span 4 q; w1, w2 the forward twiddles), as
+// dif_fwd and dit_inv form them.
+template <typename T>
+__device__ __forceinline__ void bf4_fwd(cpx<T> (&x)[4], cpx<T> w1, cpx<T> w2)
+{
+  const cpx<T> a0 = {x[0].x + x[2].x, x[0].y + x[2].y}, a1 = {x[1].x + x[3].x, x[1].y + x[3].y};
+  const cpx<T> d02 = {x[0].x - x[2].x, x[0].y - x[2].y}, d13 = {x[1].x - x[3].x, x[1].y - x[3].y};
+  const cpx<T> a2 = cmul<T>(d02, w1), a3 = cmul<T>({d13.y, -d13.x}, w1);
+  x[0] = {a0.x + a1.x, a0.y + a1.y};
+  x[1] = cmul<T>({a0.x - a1.x, a0.y - a1.y}, w2);
+  x[2] = {a2.x + a3.x, a2.y + a3.y};
+  x[3] = cmul<T>({a2.x - a3.x, a2.y - a3.y}, w2);
+}
+
+template <typename T>
+__device__ __forceinline__ void bf4_inv(cpx<T> (&x)[4], cpx<T> w1, cpx<T> w2)
+{
+  const cpx<T> W = {w1.x, -w1.y}, V = {w2.x, -w2.y};
+  const cpx<T> v1 = cmul<T>(x[1], V), v3 = cmul<T>(x[3], V);
+  const cpx<T> a0 = {x[0].x + v1.x, x[0].y + v1.y}, a1 = {x[0].x - v1.x, x[0].y - v1.y};
+  const cpx<T> a2 = {x[2].x + v3.x, x[2].y + v3.y}, a3 = {x[2].x - v3.x, x[2].y - v3.y};
+  const cpx<T> b2 = cmul<T>(a2, W), wa3 = cmul<T>(a3, W);
+  const cpx<T> b3 = {-wa3.y, wa3.x};
+  x[0] = {a0.x + b2.x, a0.y + b2.y};
+  x[2] = {a0.x - b2.x, a0.y - b2.y};
+  x[1] = {a1.x + b3.x, a1.y + b3.y};
+  x[3] = {a1.x - b3.x, a1.y - b3.y};
+}
+
+// dif_fwd (INV false) or dit_inv over the 2^lB lines at b * ls, elements es
+// apart.  ROWS: a wave's threads take consecutive butterflies of a line, else
+// the same butterfly of consecutive lines.  The innermost stage (spans of 4,
+// or 2 when log2 n is odd) is left to the caller when SKIP is set.
+template <typename T, bool ROWS, bool INV, bool SKIP>
+__device__ __forceinline__ void plane_fft(cpx<T> *s, int lB, int logn, int ls, int es, const cpx<T> *tw)
+{
+  const int n = 1 << logn;
+  auto radix2 = [&]() {
+    const int nb2 = 1 << (lB + logn - 1);
+    for (int m = threadIdx.x; m < nb2; m += kPlaneT) {
+      const int b = ROWS ? m >> (logn - 1) : m & ((1 << lB) - 1);
+      const int r = ROWS ? m & ((n >> 1) - 1) : m >> lB;
+      const int i0 = b * ls + 2 * r * es;
+      const cpx<T> u = s[i0], v = s[i0 + es];
+      s[i0] = {u.x + v.x, u.y + v.y};
+      s[i0 + es] = {u.x - v.x, u.y - v.y};
+    }
+    __syncthreads();
+  };
+  if (INV && !SKIP && (logn & 1)) radix2();
+  // forward stages shrink the span from n, inverse ones grow it back
+  for (int lq = INV ? (logn & 1) + (SKIP && !(logn & 1) ? 2 : 0) : logn - 2;
+       INV ? lq + 2 <= logn : lq >= (SKIP && !(logn & 1) ? 2 : 0); lq += INV ? 2 : -2) {
+    const int q = 1 << lq, step = n >> (lq + 2);
+    const int nb4 = 1 << (lB + logn - 2);
+    for (int m = threadIdx.x; m < nb4; m += kPlaneT) {
+      const int b = ROWS ? m >> (logn - 2) : m & ((1 << lB) - 1);
+      const int r = ROWS ? m & ((n >> 2) - 1) : m >> lB;
+      const int k = r & (q - 1);
+      const int i0 = b * ls + (((r >> lq) << (lq + 2)) + k) * es, dq = q * es;
+      cpx<T> x[4] = {s[i0], s[i0 + dq], s[i0 + 2 * dq], s[i0 + 3 * dq]};
+      if (INV) bf4_inv<T>(x, tw[k * step], tw[2 * k * step]);
+      else bf4_fwd<T>(x, tw[k * step], tw[2 * k * step]);
+#pragma unroll
+      for (int u = 0; u < 4; u++) s[i0 + u * dq] = x[u];
+    }
+    __syncthreads();
+  }
+  if (!INV && !SKIP && (logn & 1)) radix2();
+}
+
+template <typename T>
+__global__ __launch_bounds__(kPlaneT) void k2_plane(int lx, int ly, int nz, int nzc, const double *__restrict__ part,
+                                                    const T *__restrict__ C, T *__restrict__ Z,
+                                                    const double *__restrict__ twx, const double *__restrict__ twy,
+                                                    Symbol sym, const double *__restrict__ trx,
+                                                    const double *__restrict__ try_, const double *__restrict__ trz,
+                                                    double *__restrict__ y)
+{
+  __shared__ cpx<T> s[kPlaneMax + kPlanePad];
+  __shared__ cpx<T> tx[512], ty[512];
+  __shared__ double cs[4 * (kPlanePad + 4)];  // cos, sin of the x and y modes
+  __shared__ double red[kHm];
+  const int nx = 1 << lx, ny = 1 << ly, nxy = 1 << (lx + ly), ls = nx + 1;
+  load_twiddles<T>(tx, twx, nx);
+  load_twiddles<T>(ty, twy, ny);
+  double *csy = cs + 2 * nx;
+  for (int t = threadIdx.x; t < 2 * nx; t += kPlaneT) cs[t] = trx[t];
+  for (int t = threadIdx.x; t < 2 * ny; t += kPlaneT) csy[t] = try_[t];
+  // the kz = 0 symbol's factor at the slot of bit-reversed frequencies (px, py)
+  auto factor = [&](int px, int py) { return symbol_factor(sym, bitrev(px, lx), bitrev(py, ly), 0, cs, csy, trz); };
+  auto slot = [&](int col) { return (col >> lx) * ls + (col & (nx - 1)); };
+  T V[kHm + 1][kPlaneP], w[kPlaneP];
+  // r2 = the z-mean of the residual, its own mean removed
+  double r2[kPlaneP], a[kHm];
+  a[0] = 0.0;
+#pragma unroll
+  for (int p = 0; p < kPlaneP; p++) {
+    const int col = (int)threadIdx.x + kPlaneT * p;
+    r2[p] = 0.0;
+    if (col < nxy) {
+      double t = 0.0;
+#pragma unroll 8
+      for (int zc = 0; zc < nzc; zc++) t += part[(int64_t)zc * nxy + col];
+      r2[p] = t;
+    }
+    a[0] += r2[p];
+  }
+  block_sums<kHm>(a, 1, red);
+  const double inz = 1.0 / (double)nz, mean = red[0] * inz / (double)nxy;
+  a[0] = 0.0;
+#pragma unroll
+  for (int p = 0; p < kPlaneP; p++) {
+    const int col = (int)threadIdx.x + kPlaneT * p;
+    V[0][p] = col < nxy ? (T)(r2[p] * inz - mean) : (T)0;
+    a[0] += (double)V[0][p] * (double)V[0][p];
+  }
+  double sub[kHm + 1], hc[kHm][kHm];
+#pragma unroll
+  for (int j = 0; j < kHm; j++) {
+    block_sums<kHm>(a, 1, red);
+    sub[j] = sqrt(red[0]);
+    const double inv = sub[j] > 0.0 ? 1.0 / sub[j] : 0.0;
+#pragma unroll
+    for (int p = 0; p < kPlaneP; p++) {
+      const int col = (int)threadIdx.x + kPlaneT * p;
+      V[j][p] = (T)((double)V[j][p] * inv);
+      if (col < nxy) s[slot(col)] = {V[j][p], (T)0};
+    }
+    __syncthreads();
+    // Z_j = F2 V_j
+    plane_fft<T, true, false, false>(s, ly, lx, ls, 1, tx);
+    plane_fft<T, false, false, true>(s, lx, ly, 1, ls, ty);
+    // the innermost stages of both y transforms touch the same values: the last
+    // forward one, the symbol and the first inverse one in registers
+    if (ly & 1) {
+      for (int m = threadIdx.x; m < nxy / 2; m += kPlaneT) {
+        const int px = m & (nx - 1), r = m >> lx, i0 = px + 2 * r * ls;
+        const cpx<T> u = s[i0], v = s[i0 + ls];
+        const double f0 = factor(px, 2 * r), f1 = factor(px, 2 * r + 1);
+        const cpx<T> a0 = {(T)((double)(u.x + v.x) * f0), (T)((double)(u.y + v.y) * f0)};
+        const cpx<T> a1 = {(T)((double)(u.x - v.x) * f1), (T)((double)(u.y - v.y) * f1)};
+        s[i0] = {a0.x + a1.x, a0.y + a1.y};
+        s[i0 + ls] = {a0.x - a1.x, a0.y - a1.y};
+      }
+    } else {
+      const cpx<T> one = ty[0];
+      for (int m = threadIdx.x; m < nxy / 4; m += kPlaneT) {
+        const int px = m & (nx - 1), r = m >> lx, i0 = px + 4 * r * ls;
+        cpx<T> x[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) x[u] = s[i0 + u * ls];
+        bf4_fwd<T>(x, one, one);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const double f = factor(px, 4 * r + u);
+          x[u] = {(T)((double)x[u].x * f), (T)((double)x[u].y * f)};
+        }
+        bf4_inv<T>(x, one, one);
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[i0 + u * ls] = x[u];
+      }
+    }
+    __syncthreads();
+    plane_fft<T, false, true, true>(s, lx, ly, 1, ls, ty);
+    plane_fft<T, true, true, false>(s, ly, lx, ls, 1, tx);
+    // w = A2 Z_j less its parts along V_0 .. V_j (one classical Gram-Schmidt
+    // pass: with two directions a second one changes the last bits only)
+#pragma unroll
+    for (int p = 0; p < kPlaneP; p++) {
+      const int col = (int)threadIdx.x + kPlaneT * p;
+      w[p] = (T)0;
+      if (col < nxy) {
+        const int i = col & (nx - 1), jy = col >> lx;
+        const int xs[3] = {(i - 1) & (nx - 1), i, (i + 1) & (nx - 1)};
+        const int ys[3] = {(jy - 1) & (ny - 1), jy, (jy + 1) & (ny - 1)};
+        double acc = 0.0;
+#pragma unroll
+        for (int o = 0; o < 9; o++) acc += (double)C[o * nxy + col] * (double)s[ys[o / 3] * ls + xs[o % 3]].x;
+        w[p] = (T)acc;
+        Z[j * nxy + col] = s[slot(col)].x;
+      }
+    }
+#pragma unroll
+    for (int q = 0; q <= j; q++) {
+      a[q] = 0.0;
+#pragma unroll
+      for (int p = 0; p < kPlaneP; p++) a[q] += (double)V[q][p] * (double)w[p];
+    }
+    block_sums<kHm>(a, j + 1, red);
+#pragma unroll
+    for (int q = 0; q <= j; q++) hc[q][j] = red[q];
+#pragma unroll
+    for (int p = 0; p < kPlaneP; p++) {
+      double x = (double)w[p];
+#pragma unroll
+      for (int q = 0; q <= j; q++) x -= hc[q][j] * (double)V[q][p];
+      w[p] = (T)x;
+    }
+    a[0] = 0.0;
+#pragma unroll
+    for (int p = 0; p < kPlaneP; p++) {
+      V[j + 1][p] = w[p];
+      a[0] += (double)w[p] * (double)w[p];
     }
   }
-  for (int q = 0; q < kHm; q++) y[q] = yy[q];
+  block_sums<kHm>(a, 1, red);
+  sub[kHm] = sqrt(red[0]);
+  if (threadIdx.x == 0) h2_lstsq(sub, hc, y);
 }
 
 // z[k * nxy + col] += sum_q y_q Z_q[col] over kExtZ planes per block
@@ -1233,30 +1462,36 @@ int fft2_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z, T *w3, b
   const int nb = h.nb;
   // z-averaged residual of the first level, mean removed, into V0
   launch_lhs_zsum<T>(ctx, ctx->prm.lhs_type, (const T *)ctx->mom[0], z, r, h.part, h.pl, fused ? w3 : nullptr);
-  hipLaunchKernelGGL((k2_r2<T>), nb, 256, 0, ctx->stream, nxy, nz, lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part,
-                     (const double *)h.pl, h.nlb, V, h.pn);
   Symbol sym = make_symbol(ctx, v19);
   sym.inv_scale = 1.0 / (double)nxy;
-  const int Bx = fft2_batch<T>(nx, ny), By = fft2_batch<T>(ny, nx);
-  for (int j = 0; j < kFft2Its; j++) {
-    T *Vj = V + (int64_t)j * nxy, *Zj = Z + (int64_t)j * nxy;
-    // Zj = F2 Vj: 2-D FFT solve with the kz = 0 symbol
-    hipLaunchKernelGGL((k_fft2_x<T, 0>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
-                       ilog2(nx), ny, Bx, Vj, cb, ctx->tw[0], (const double *)(h.pn + (int64_t)j * nb), nb);
-    hipLaunchKernelGGL((k_fft_s<T, 3>), (unsigned)(nx / By), kBlock, fft_lds<T>(ny, By), ctx->stream, ilog2(ny),
-                       (int64_t)nx, (int64_t)nx, (int64_t)0, By, cb, ctx->tw[1], sym, ctx->trig[0], ctx->trig[1],
-                       ctx->trig[2]);
-    hipLaunchKernelGGL((k_fft2_x<T, 1>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
-                       ilog2(nx), ny, Bx, Zj, cb, ctx->tw[0], (const double *)nullptr, 0);
-    double *p1 = h.p1 + (int64_t)j * kHm * nb, *p2 = h.p2 + (int64_t)j * kHm * nb;
-    hipLaunchKernelGGL((k2_a2dots<T>), nb, 256, 0, ctx->stream, nx, ny, j, (const T *)C, (const T *)Zj,
-                       (const T *)V, w, p1, nb);
-    hipLaunchKernelGGL((k2_gs_pass<T, 1>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p1, p2, nb);
-    hipLaunchKernelGGL((k2_gs_pass<T, 2>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p2,
-                       h.pn + (int64_t)(j + 1) * nb, nb);
+  if (nxy <= kPlaneMax) {
+    hipLaunchKernelGGL((k2_plane<T>), 1, kPlaneT, 0, ctx->stream, ilog2(nx), ilog2(ny), nz,
+                       lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part, (const T *)C, Z, ctx->tw[0],
+                       ctx->tw[1], sym, ctx->trig[0], ctx->trig[1], ctx->trig[2], h.y);
+  } else {
+    hipLaunchKernelGGL((k2_r2<T>), nb, 256, 0, ctx->stream, nxy, nz, lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part,
+                       (const double *)h.pl, h.nlb, V, h.pn);
+    const int Bx = fft2_batch<T>(nx, ny), By = fft2_batch<T>(ny, nx);
+    for (int j = 0; j < kFft2Its; j++) {
+      T *Vj = V + (int64_t)j * nxy, *Zj = Z + (int64_t)j * nxy;
+      // Zj = F2 Vj: 2-D FFT solve with the kz = 0 symbol
+      hipLaunchKernelGGL((k_fft2_x<T, 0>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
+                         ilog2(nx), ny, Bx, Vj, cb, ctx->tw[0], (const double *)(h.pn + (int64_t)j * nb), nb);
+      hipLaunchKernelGGL((k_fft_s<T, 3>), (unsigned)(nx / By), kBlock, fft_lds<T>(ny, By), ctx->stream, ilog2(ny),
+                         (int64_t)nx, (int64_t)nx, (int64_t)0, By, cb, ctx->tw[1], sym, ctx->trig[0], ctx->trig[1],
+                         ctx->trig[2]);
+      hipLaunchKernelGGL((k_fft2_x<T, 1>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
+                         ilog2(nx), ny, Bx, Zj, cb, ctx->tw[0], (const double *)nullptr, 0);
+      double *p1 = h.p1 + (int64_t)j * kHm * nb, *p2 = h.p2 + (int64_t)j * kHm * nb;
+      hipLaunchKernelGGL((k2_a2dots<T>), nb, 256, 0, ctx->stream, nx, ny, j, (const T *)C, (const T *)Zj,
+                         (const T *)V, w, p1, nb);
+      hipLaunchKernelGGL((k2_gs_pass<T, 1>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p1, p2, nb);
+      hipLaunchKernelGGL((k2_gs_pass<T, 2>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p2,
+                         h.pn + (int64_t)(j + 1) * nb, nb);
+    }
+    hipLaunchKernelGGL(k2_solve, 1, 256, 0, ctx->stream, (const double *)h.pn, (const double *)h.p1,
+                       (const double *)h.p2, nb, h.y);
   }
-  hipLaunchKernelGGL(k2_solve, 1, 256, 0, ctx->stream, (const double *)h.pn, (const double *)h.p1,
-                     (const double *)h.p2, nb, h.y);
   if (fused) {
     launch_zline_apply_e2<T>(ctx, (const T *)ctx->zl_buf, ctx->zl_col, w3, z, (const T *)ctx->mom[0], (const T *)Z,
                              (const double *)h.y);

@@ -33,3 +33,28 @@ def test_stencil_is_the_oracles_bit_for_bit(N, extra):
     ref = orc.lhs_apply(g, K, mom[0], x, lhs_type=lt, transpose=True)
     # the oracle scatters its rows: the same 19 products a node, in another order
     assert np.abs(yt - ref).max() <= 19 * 2.0 ** -52 * np.abs(ref).max() * 19
+
+
+# the one-workgroup 2-D correction: planes of 16 to 4096 nodes with even and
+# odd log2 lengths, the longest lines it takes, and the first plane beyond it
+# (8192), which the separate launches take.  The symbol of the FFT stage is a
+# sum that cancels towards the weakest mode: lambda_min / A0 = (1 - cos(2 pi /
+# N)) / (2 + 1 + Kz^2), and its 8 roundings on each side, in another order,
+# bound the agreement with the oracle.
+@pytest.mark.parametrize("prec,base", [("fp64", 1e-12), ("mixed", 2e-5)])
+@pytest.mark.parametrize("N", [(4, 4, 4), (8, 4, 4), (4, 8, 8), (32, 16, 8), (16, 32, 4), (64, 64, 4), (4, 1024, 4),
+                               (1024, 4, 4), (128, 64, 4)])
+def test_two_level_correction_on_any_plane(N, prec, base):
+    rng = np.random.default_rng(12)
+    with context(opts(N, extra=f"-pc_type fft2 -precision {prec}")) as ctx:
+        g = grid_of(ctx.prm)
+        mom = [m.astype(np.float32).astype(np.float64) for m in _moments(g, rng, amp=0.1)]
+        ctx.set_moments(vlasov_from(mom))
+        r = rng.standard_normal(g.nc)
+        r -= r.mean()
+        z = ctx.pc_apply(r)
+        K = list(ctx.prm.kappa_e)
+    tol = base + 16 * 2.0 ** -52 * (3 + K[2] ** 2) / (1 - np.cos(2 * np.pi / max(N)))
+    ref = orc.pc_apply(g, K, mom[0], r, orc.PC_FFT2)
+    z, ref = z - z.mean(), ref - ref.mean()
+    assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
