@@ -501,6 +501,66 @@ static inline dim3 col_grid(const Grid &g)
 }
 
 enum { kOpKz, kOpFull, kOpConst };  // the full operator with B along z, any B, a constant row
+
+// Row c of A times x from the values around it.  Densities: the centre n0, the
+// faces nf = x+, x-, y+, y- and z+, z- (unused with kOpConst); x: the centre
+// x0, the faces xf, the x-y edges xe = ++, +-, -+, --, the z neighbours, and
+// their faces xfp, xfm (the x-z and y-z edges; unused with kOpKz).  The
+// oracle's order of operations in FP64; FP32 sums v_q (x_q - x_c) (DIFF).
+template <typename C, bool DIFF, int OP>
+__device__ __forceinline__ C row_apply(const SCoef &s, const LapRow &lap, C n0, const C (&nf)[4], C nzp, C nzm, C x0,
+                                       const C (&xf)[4], const C (&xe)[4], C xzp, C xzm, const C (&xfp)[4],
+                                       const C (&xfm)[4])
+{
+  C acc = (C)0;
+  if constexpr (OP == kOpKz) {
+    const C sxx = (C)s.sxx, syy = (C)s.syy, szz = (C)s.szz, sxy = (C)s.sxy, syx = (C)s.syx;
+    const C nxp = nf[0], nxm = nf[1], nyp = nf[2], nym = nf[3];
+    // entries 0-9 and 18 of row_from_star with s_xz = s_yz = s_zx = s_zy = 0
+    const C a = nxp + n0, bq = n0 + nxm, cq = nyp + n0, dq = n0 + nym;
+    const C dy = nyp - nym, dx = nxp - nxm;
+    C w[10];
+    w[0] = mad(sxx, a, syx * dy);
+    w[1] = mad(sxx, bq, -(syx * dy));
+    w[2] = mad(syy, cq, sxy * dx);
+    w[3] = mad(syy, dq, -(sxy * dx));
+    w[4] = szz * (nzp + n0);
+    w[5] = szz * (n0 + nzm);
+    w[6] = mad(sxy, a, syx * cq);
+    w[7] = mad(-sxy, a, -(syx * dq));
+    w[8] = mad(-sxy, bq, -(syx * cq));
+    w[9] = mad(sxy, bq, syx * dq);
+    // -((sxx X + syy Y) + szz Z), the oracle's association
+    const C w18 = -(mad(szz, nzp + 2 * n0 + nzm, mad(sxx, nxp + 2 * n0 + nxm, syy * (nyp + 2 * n0 + nym))));
+    const C xv[10] = {xf[0], xf[1], xf[2], xf[3], xzp, xzm, xe[0], xe[1], xe[2], xe[3]};
+    if (DIFF) {
+#pragma unroll
+      for (int q = 0; q < 10; q++) acc = mad(w[q], xv[q] - x0, acc);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 10; q++) acc += w[q] * xv[q];
+      acc += w18 * x0;
+    }
+  } else {
+    C w[19];
+    if constexpr (OP == kOpFull) {
+      row_from_star<C>(s, n0, nf[0], nf[1], nf[2], nf[3], nzp, nzm, w);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 19; q++) w[q] = (C)lap.v[q];
+    }
+    const C xv[19] = {xf[0],  xf[1],  xf[2],  xf[3],  xzp,    xzm,    xe[0],  xe[1],  xe[2], xe[3],
+                      xfp[0], xfm[0], xfp[1], xfm[1], xfp[2], xfm[2], xfp[3], xfm[3], x0};
+    if (DIFF) {
+#pragma unroll
+      for (int q = 0; q < 18; q++) acc = mad(w[q], xv[q] - xv[18], acc);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 19; q++) acc += w[q] * xv[q];
+    }
+  }
+  return acc;
+}
 // base + a 32-bit byte offset within a plane (a plane of 4 GB does not fit
 // beside the solver's vectors), so that the plane's address stays scalar
 template <typename T>
@@ -571,56 +631,8 @@ __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow
       for (int v = 0; v < ZR; v++) {
         const int u = v + 1, k = k0 + v;
         if (k >= z1) break;
-        C acc = (C)0;
-        if constexpr (KZ) {
-          const C sxx = (C)s.sxx, syy = (C)s.syy, szz = (C)s.szz, sxy = (C)s.sxy, syx = (C)s.syx;
-          const C n0 = nc[u], nxp = nf[v][0], nxm = nf[v][1], nyp = nf[v][2], nym = nf[v][3], nzp = nc[u + 1],
-                  nzm = nc[u - 1];
-          // entries 0-9 and 18 of row_from_star with s_xz = s_yz = s_zx = s_zy = 0
-          const C a = nxp + n0, bq = n0 + nxm, cq = nyp + n0, dq = n0 + nym;
-          const C dy = nyp - nym, dx = nxp - nxm;
-          C w[10];
-          w[0] = mad(sxx, a, syx * dy);
-          w[1] = mad(sxx, bq, -(syx * dy));
-          w[2] = mad(syy, cq, sxy * dx);
-          w[3] = mad(syy, dq, -(sxy * dx));
-          w[4] = szz * (nzp + n0);
-          w[5] = szz * (n0 + nzm);
-          w[6] = mad(sxy, a, syx * cq);
-          w[7] = mad(-sxy, a, -(syx * dq));
-          w[8] = mad(-sxy, bq, -(syx * cq));
-          w[9] = mad(sxy, bq, syx * dq);
-          // -((sxx X + syy Y) + szz Z), the oracle's association
-          const C w18 = -(mad(szz, nzp + 2 * n0 + nzm, mad(sxx, nxp + 2 * n0 + nxm, syy * (nyp + 2 * n0 + nym))));
-          const C xv[10] = {xf[u][0], xf[u][1], xf[u][2], xf[u][3], xc[u + 1], xc[u - 1],
-                            xe[v][0], xe[v][1], xe[v][2], xe[v][3]};
-          if (DIFF) {
-#pragma unroll
-            for (int q = 0; q < 10; q++) acc = mad(w[q], xv[q] - xc[u], acc);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 10; q++) acc += w[q] * xv[q];
-            acc += w18 * xc[u];
-          }
-        } else {
-          C w[19];
-          if constexpr (OP == kOpFull) {
-            row_from_star<C>(s, nc[u], nf[v][0], nf[v][1], nf[v][2], nf[v][3], nc[u + 1], nc[u - 1], w);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 19; q++) w[q] = (C)lap.v[q];
-          }
-          const C xv[19] = {xf[u][0],     xf[u][1],     xf[u][2],     xf[u][3],     xc[u + 1],    xc[u - 1],    xe[v][0],
-                            xe[v][1],     xe[v][2],     xe[v][3],     xf[u + 1][0], xf[u - 1][0], xf[u + 1][1], xf[u - 1][1],
-                            xf[u + 1][2], xf[u - 1][2], xf[u + 1][3], xf[u - 1][3], xc[u]};
-          if (DIFF) {
-#pragma unroll
-            for (int q = 0; q < 18; q++) acc = mad(w[q], xv[q] - xv[18], acc);
-          } else {
-#pragma unroll
-            for (int q = 0; q < 19; q++) acc += w[q] * xv[q];
-          }
-        }
+        const C acc = row_apply<C, DIFF, OP>(s, lap, nc[u], nf[v], nc[u + 1], nc[u - 1], xc[u], xf[u], xe[v], xc[u + 1],
+                                             xc[u - 1], xf[u + 1], xf[u - 1]);
         const int64_t c = (int64_t)c0 + pstride * k;
         if (OUT == 0) y[c] = (TY)acc;
         else {
@@ -1908,38 +1920,76 @@ __global__ __launch_bounds__(256) void k_zline_apply_e2(Grid g, const T *__restr
   }
 }
 
-// The same z-line solve with one wave per column, for grids of few columns
-// (the multigrid's coarse levels), where one thread per column leaves the
-// chip idle and each call costs the latency of walking the column three
-// times.  The forward and back substitutions are first-order linear
-// recurrences, y_k = alpha_k y_(k-1) + beta_k: each lane composes the affine
-// maps of its P consecutive planes, a wave scan (6 shuffle steps) gives every
-// lane the value entering its planes, and the lane then runs its planes with
-// the sequential kernel's formulas.  Intermediate values are rounded to T
-// where the sequential kernel stores them.  The scan reassociates the
-// products, so results agree with k_zline_apply to rounding, not bitwise.
-template <typename T, int P>
-__global__ __launch_bounds__(256) void k_zline_apply_wave(Grid g, const T *__restrict__ za, const T *__restrict__ zi,
-                                                          const T *__restrict__ zc, const T *__restrict__ zq,
-                                                          const double *__restrict__ cag,
-                                                          const double *__restrict__ cden, const T *__restrict__ res,
-                                                          T *__restrict__ z, double scale)
+// ---- multigrid levels with z fastest ----------------------------------------------
+// The multigrid keeps its level fields as [y][x][z]: a group of W lanes owns a
+// column, P consecutive planes a lane (W P >= nz), so that the stencil around a
+// column, the column's z-line system and its solve are contiguous loads and
+// shuffles.  A smoothing sweep is then one launch, x' = x + omega zline^-1 (b -
+// A x), the residual never stored: 6.0 us on 96 x 80 x 50 and 5 on its coarse
+// levels (FP32), where with x fastest it took a residual pass (4 to 6 us) and a
+// solve (16.6 us walking 96 x 80 columns, 4.6 us on fewer).  A preconditioner
+// application there went from 65 launches to 43.  Whole solves: 96 x 80 x 50
+// mixed 26.1 -> 14.6 ms, 64 x 48 x 40 FP64 21.7 -> 12.8, 160 x 144 x 100 mixed
+// 8.9 -> 5.7, 256^3 mixed 22.7 -> 17.9.  What is left is latency: one launch
+// after another on grids that a chip of 256 CUs does in a microsecond or two.
+// (All sweeps of the coarsest level in one workgroup, in LDS and registers,
+// took 27 to 52 us against 8 launches of 4 to 5: the scans' instructions
+// bound a single CU.)
+
+// Bases of a column and of its neighbours along x, y and diagonally
+struct ColNb { int64_t c, xp, xm, yp, ym, pp, pm, mp, mm; };
+
+__device__ __forceinline__ ColNb col_nb(const Grid &g, int col)
 {
-  const int64_t plane = (int64_t)g.nx * g.ny;
-  const int64_t col = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int L = (int)(threadIdx.x & 63), m = g.nz;
-  if (col >= plane) return;  // the wave's column: the whole wave leaves together
-  double r[P], a[P], iv[P], c[P], y[P];
-#pragma unroll
-  for (int u = 0; u < P; u++) {
-    const int k = L * P + u;
-    r[u] = a[u] = iv[u] = c[u] = 0.0;
-    if (k < m) {
-      const int64_t e = col + plane * k;
-      r[u] = (double)res[e]; a[u] = (double)za[e]; iv[u] = (double)zi[e]; c[u] = (double)zc[e];
-    }
+  int i, j, k_;
+  split_cell(g, col, i, j, k_);
+  const int ip = i + 1 == g.nx ? 0 : i + 1, im = i == 0 ? g.nx - 1 : i - 1;
+  const int jp = j + 1 == g.ny ? 0 : j + 1, jm = j == 0 ? g.ny - 1 : j - 1;
+  auto at = [&](int a, int b) { return ((int64_t)a + (int64_t)g.nx * b) * g.nz; };
+  return {at(i, j), at(ip, j), at(im, j), at(i, jp), at(i, jm), at(ip, jp), at(ip, jm), at(im, jp), at(im, jm)};
+}
+
+// Row of A x at plane k of column q
+template <typename T, typename C, bool DIFF, int OP>
+__device__ __forceinline__ C zf_row(const Grid &g, const SCoef &s, const LapRow &lap, const T *__restrict__ n,
+                                    const T *__restrict__ x, const ColNb &q, int k)
+{
+  const int kp = k + 1 == g.nz ? 0 : k + 1, km = k == 0 ? g.nz - 1 : k - 1;
+  C nf[4] = {(C)0, (C)0, (C)0, (C)0}, n0 = (C)0, nzp = (C)0, nzm = (C)0;
+  if (OP != kOpConst) {
+    n0 = (C)n[q.c + k]; nzp = (C)n[q.c + kp]; nzm = (C)n[q.c + km];
+    nf[0] = (C)n[q.xp + k]; nf[1] = (C)n[q.xm + k]; nf[2] = (C)n[q.yp + k]; nf[3] = (C)n[q.ym + k];
   }
-  // forward: y_k = (r_k - a_k y_(k-1)) i_k, y_(-1) = 0; the lane's map y -> A y + B
+  const C xf[4] = {(C)x[q.xp + k], (C)x[q.xm + k], (C)x[q.yp + k], (C)x[q.ym + k]};
+  const C xe[4] = {(C)x[q.pp + k], (C)x[q.pm + k], (C)x[q.mp + k], (C)x[q.mm + k]};
+  C xfp[4], xfm[4];
+  if (OP != kOpKz) {
+    xfp[0] = (C)x[q.xp + kp]; xfp[1] = (C)x[q.xm + kp]; xfp[2] = (C)x[q.yp + kp]; xfp[3] = (C)x[q.ym + kp];
+    xfm[0] = (C)x[q.xp + km]; xfm[1] = (C)x[q.xm + km]; xfm[2] = (C)x[q.yp + km]; xfm[3] = (C)x[q.ym + km];
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; e++) xfp[e] = xfm[e] = (C)0;
+  }
+  return row_apply<C, DIFF, OP>(s, lap, n0, nf, nzp, nzm, (C)x[q.c + k], xf, xe, (C)x[q.c + kp], (C)x[q.c + km], xfp, xfm);
+}
+
+// Orders a wave's own LDS accesses (which the hardware keeps in order)
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The cyclic z-line solve of the column held by W lanes (lane L: planes L P ..
+// L P + P - 1), r in and the solution in r.  The forward and back
+// substitutions are first-order linear recurrences, y_k = alpha_k y_(k-1) +
+// beta_k: each lane composes the affine maps of its planes, a scan over the W
+// lanes gives the value entering them, and the lane then runs its planes with
+// the sequential formulas.
+template <typename T, int W, int P>
+__device__ __forceinline__ void zline_lanes(int L, int m, double (&r)[P], const double (&a)[P], const double (&iv)[P],
+                                            const double (&c)[P], const double (&q)[P], double cag, double cden)
+{
   double A = 1.0, B = 0.0;
 #pragma unroll
   for (int u = 0; u < P; u++) {
@@ -1950,56 +2000,232 @@ __global__ __launch_bounds__(256) void k_zline_apply_wave(Grid g, const T *__res
     }
   }
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {  // inclusive scan: lower lanes' maps first
-    const double A2 = __shfl_up(A, off, 64), B2 = __shfl_up(B, off, 64);
+  for (int off = 1; off < W; off <<= 1) {  // inclusive scan: lower lanes' maps first
+    const double A2 = __shfl_up(A, off, W), B2 = __shfl_up(B, off, W);
     if (L >= off) { B = A * B2 + B; A = A * A2; }
   }
-  double yin = __shfl_up(B, 1, 64);  // the exclusive prefix applied to y_(-1) = 0
-  if (L == 0) yin = 0.0;
-  double yv = yin;
+  double yv = __shfl_up(B, 1, W);  // the exclusive prefix applied to y_(-1) = 0
+  if (L == 0) yv = 0.0;
 #pragma unroll
   for (int u = 0; u < P; u++) {
     if (L * P + u < m) {
       yv = (r[u] - a[u] * yv) * iv[u];
-      y[u] = (double)(T)yv;  // as the sequential kernel stores it
-    } else {
-      y[u] = 0.0;
+      r[u] = yv;
     }
   }
-  const double ylast = __shfl(yv, (m - 1) / P, 64);  // y_(m-1), unrounded
+  const double ylast = __shfl(yv, (m - 1) / P, W);
   // backward: x_(m-1) = y_(m-1), x_k = y_k - c_k x_(k+1); higher planes first
   A = 1.0; B = 0.0;
 #pragma unroll
   for (int u = P - 1; u >= 0; u--) {
     const int k = L * P + u;
     if (k == m - 1) { A = 0.0; B = ylast; }
-    else if (k < m - 1) { B = -c[u] * B + y[u]; A = -c[u] * A; }
+    else if (k < m - 1) { B = -c[u] * B + r[u]; A = -c[u] * A; }
   }
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {  // higher lanes' maps first
-    const double A2 = __shfl_down(A, off, 64), B2 = __shfl_down(B, off, 64);
-    if (L + off < 64) { B = A * B2 + B; A = A * A2; }
+  for (int off = 1; off < W; off <<= 1) {  // higher lanes' maps first
+    const double A2 = __shfl_down(A, off, W), B2 = __shfl_down(B, off, W);
+    if (L + off < W) { B = A * B2 + B; A = A * A2; }
   }
-  double xin = __shfl_down(B, 1, 64);
-  if (L == 63) xin = 0.0;
-  double xv = xin;
+  double xv = __shfl_down(B, 1, W);
+  if (L == W - 1) xv = 0.0;
 #pragma unroll
   for (int u = P - 1; u >= 0; u--) {
     const int k = L * P + u;
-    if (k == m - 1) xv = ylast;  // y[u] keeps y_(m-1) as stored
-    else if (k < m - 1) { xv = y[u] - c[u] * xv; y[u] = (double)(T)xv; }
+    if (k == m - 1) xv = ylast;
+    else if (k < m - 1) { xv = r[u] - c[u] * xv; r[u] = xv; }
   }
-  const double x0 = __shfl(xv, 0, 64);  // x_0, unrounded (lane 0's last step is plane 0)
-  const double f = (x0 + cag[col] * ylast) / cden[col];
+  const double f = (__shfl(xv, 0, W) + cag * ylast) / cden;
+#pragma unroll
+  for (int u = 0; u < P; u++) r[u] -= f * q[u];
+}
+
+// r changes from consecutive lanes on consecutive planes to the lanes' own P
+// planes (to_lanes), or back, through the LDS row t of W P values.
+template <int W, int P>
+__device__ __forceinline__ void turn_planes(bool to_lanes, int L, double (&r)[P], double *t)
+{
+  if (P == 1) return;
+  wave_sync();  // (earlier reads of the row)
+#pragma unroll
+  for (int u = 0; u < P; u++) t[to_lanes ? u * W + L : L * P + u] = r[u];
+  wave_sync();
+#pragma unroll
+  for (int u = 0; u < P; u++) r[u] = t[to_lanes ? L * P + u : u * W + L];
+}
+
+// One column's sweep: xo = x + omega zline^-1 (b - A x), or with FIRST (x = 0)
+// xo = omega zline^-1 b.  zf: the factors za, zi, zc, zq (nc each).  With
+// several planes a lane, the fields are read and written with consecutive
+// lanes on consecutive planes, and the residual and the solution change to and
+// from the lanes' own planes through the wave's LDS row t (W P values); the
+// factors of a lane's planes are consecutive in memory.
+template <typename T, int W, int P, int OP, bool FIRST>
+__device__ __forceinline__ void mg_sweep_col(const Grid &g, const SCoef &s, const LapRow &lap, int col, int L,
+                                             const T *__restrict__ n, const T *__restrict__ zf,
+                                             const double *__restrict__ zcol, const T *__restrict__ b, const T *x,
+                                             T *xo, double omega, double *t)
+{
+  using C = typename std::conditional<sizeof(T) == 4, float, double>::type;
+  const int m = g.nz;
+  const ColNb nb = col_nb(g, col);
+  double r[P], a[P], iv[P], c[P], q[P], xk[P];
 #pragma unroll
   for (int u = 0; u < P; u++) {
     const int k = L * P + u;
+    a[u] = iv[u] = c[u] = q[u] = 0.0;
     if (k < m) {
-      const int64_t e = col + plane * k;
-      z[e] = (T)((double)z[e] + scale * (y[u] - f * (double)zq[e]));
+      const int64_t e = nb.c + k;
+      a[u] = (double)zf[e]; iv[u] = (double)zf[g.nc + e]; c[u] = (double)zf[2 * g.nc + e]; q[u] = (double)zf[3 * g.nc + e];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    const int k = u * W + L;
+    r[u] = xk[u] = 0.0;
+    if (k < m) {
+      const int64_t e = nb.c + k;
+      r[u] = (double)b[e];
+      if (!FIRST) {
+        xk[u] = (double)x[e];
+        r[u] -= (double)zf_row<T, C, sizeof(T) == 4, OP>(g, s, lap, n, x, nb, k);
+      }
+    }
+  }
+  const int64_t plane = (int64_t)g.nx * g.ny;
+  turn_planes<W, P>(true, L, r, t);
+  zline_lanes<T, W, P>(L, m, r, a, iv, c, q, zcol[col], zcol[plane + col]);
+  turn_planes<W, P>(false, L, r, t);
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    const int k = u * W + L;
+    if (k < m) xo[nb.c + k] = (T)(xk[u] + omega * r[u]);
+  }
+}
+
+template <typename T, int W, int P, int OP, bool FIRST>
+__global__ __launch_bounds__(256) void k_mg_sweep(Grid g, SCoef s, LapRow lap, const T *__restrict__ n,
+                                                  const T *__restrict__ zf, const double *__restrict__ zcol,
+                                                  const T *__restrict__ b, const T *__restrict__ x, T *__restrict__ xo,
+                                                  double omega)
+{
+  __shared__ double t[P == 1 ? 1 : 4][W * P];
+  const int col = (int)(blockIdx.x * (256 / W) + threadIdx.x / W);
+  if (col >= g.nx * g.ny) return;  // the column's W lanes leave together
+  mg_sweep_col<T, W, P, OP, FIRST>(g, s, lap, col, (int)(threadIdx.x % W), n, zf, zcol, b, x, xo, omega,
+                                   t[P == 1 ? 0 : threadIdx.x / W]);
+}
+
+// r = b - A x, one thread per node
+template <typename T, int OP>
+__global__ __launch_bounds__(256) void k_mg_residual(Grid g, SCoef s, LapRow lap, const T *__restrict__ n,
+                                                     const T *__restrict__ b, const T *__restrict__ x,
+                                                     T *__restrict__ r)
+{
+  using C = typename std::conditional<sizeof(T) == 4, float, double>::type;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= g.nc) return;
+  const int col = (int)((uint32_t)e / (uint32_t)g.nz), k = (int)((uint32_t)e - (uint32_t)col * (uint32_t)g.nz);
+  const ColNb nb = col_nb(g, col);
+  r[e] = (T)((double)b[e] - (double)zf_row<T, C, sizeof(T) == 4, OP>(g, s, lap, n, x, nb, k));
+}
+
+// dst[c][k] = src[k][c] of up to five fields (TO_Z), or the reverse
+template <typename T>
+struct Fields5 { const T *src[5]; T *dst[5]; };
+template <typename T, bool TO_Z>
+__global__ __launch_bounds__(256) void k_mg_transpose(int cols, int nz, Fields5<T> f)
+{
+  __shared__ T t[32][33];
+  const T *__restrict__ src = f.src[blockIdx.z];
+  T *__restrict__ dst = f.dst[blockIdx.z];
+  const int c0 = (int)blockIdx.x * 32, k0 = (int)blockIdx.y * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+#pragma unroll
+  for (int u = 0; u < 32; u += 8) {
+    const int c = TO_Z ? c0 + tx : c0 + ty + u, k = TO_Z ? k0 + ty + u : k0 + tx;
+    if (c < cols && k < nz) t[ty + u][tx] = TO_Z ? src[(int64_t)k * cols + c] : src[(int64_t)c * nz + k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 32; u += 8) {
+    const int c = TO_Z ? c0 + ty + u : c0 + tx, k = TO_Z ? k0 + tx : k0 + ty + u;
+    if (c < cols && k < nz) {
+      if (TO_Z) dst[(int64_t)c * nz + k] = t[tx][ty + u];
+      else dst[(int64_t)k * cols + c] = t[tx][ty + u];
     }
   }
 }
+
+template <typename T>
+void launch_mg_transpose(chy_ctx *ctx, const Grid &g, bool to_z, int nf, const T *const *src, T *const *dst)
+{
+  Fields5<T> f = {};
+  for (int q = 0; q < nf; q++) { f.src[q] = src[q]; f.dst[q] = dst[q]; }
+  const int cols = g.nx * g.ny;
+  const dim3 grid((unsigned)((cols + 31) / 32), (unsigned)((g.nz + 31) / 32), (unsigned)nf);
+  if (to_z) hipLaunchKernelGGL((k_mg_transpose<T, true>), grid, 256, 0, ctx->stream, cols, g.nz, f);
+  else hipLaunchKernelGGL((k_mg_transpose<T, false>), grid, 256, 0, ctx->stream, cols, g.nz, f);
+}
+
+// The operator kind and row constants of a level
+static int mg_op(chy_ctx *ctx, const double d[3], SCoef &s, LapRow &L)
+{
+  const int lt = ctx->prm.lhs_type;
+  s = full_scoef(d, ctx->prm.kappa_e);
+  uniform_row(lt == CHY_LHS_FULL ? CHY_LHS_IDENTITY : lt, d, ctx->prm.kappa_e, 0.0, L.v);
+  return kz_operator(lt, s) ? kOpKz : lt == CHY_LHS_FULL ? kOpFull : kOpConst;
+}
+
+// Lanes per column and planes per lane for nz planes (at most kMgMaxPlanes)
+#define MG_WP(nz, call)                                                    \
+  do {                                                                     \
+    if (nz <= 16) { constexpr int W = 16, P = 1; call; }                   \
+    else if (nz <= 32) { constexpr int W = 32, P = 1; call; }              \
+    else if (nz <= 64) { constexpr int W = 64, P = 1; call; }              \
+    else if (nz <= 128) { constexpr int W = 64, P = 2; call; }             \
+    else if (nz <= 256) { constexpr int W = 64, P = 4; call; }             \
+    else { constexpr int W = 64, P = 8; call; }                            \
+  } while (0)
+#define MG_OP(op, call)                                                    \
+  do {                                                                     \
+    if (op == kOpKz) { constexpr int OP = kOpKz; call; }                   \
+    else if (op == kOpFull) { constexpr int OP = kOpFull; call; }          \
+    else { constexpr int OP = kOpConst; call; }                            \
+  } while (0)
+
+template <typename T>
+void launch_mg_sweep(chy_ctx *ctx, const Grid &g, const double d[3], const T *n, const T *zf, const double *zcol,
+                     const T *b, const T *x, T *xo, double omega)
+{
+  SCoef s;
+  LapRow L;
+  const int op = mg_op(ctx, d, s, L), cols = g.nx * g.ny;
+  MG_WP(g.nz, MG_OP(op, {
+    const unsigned nb = (unsigned)((cols + 256 / W - 1) / (256 / W));
+    if (x)
+      hipLaunchKernelGGL((k_mg_sweep<T, W, P, OP, false>), nb, 256, 0, ctx->stream, g, s, L, n, zf, zcol, b, x, xo, omega);
+    else
+      hipLaunchKernelGGL((k_mg_sweep<T, W, P, OP, true>), nb, 256, 0, ctx->stream, g, s, L, n, zf, zcol, b, x, xo, omega);
+  }));
+}
+
+template <typename T>
+void launch_mg_residual(chy_ctx *ctx, const Grid &g, const double d[3], const T *n, const T *b, const T *x, T *r)
+{
+  SCoef s;
+  LapRow L;
+  const int op = mg_op(ctx, d, s, L);
+  MG_OP(op, hipLaunchKernelGGL((k_mg_residual<T, OP>), nblocks(g.nc), 256, 0, ctx->stream, g, s, L, n, b, x, r));
+}
+
+#define MG_INST(T)                                                                                                  \
+  template void launch_mg_transpose<T>(chy_ctx *, const Grid &, bool, int, const T *const *, T *const *);           \
+  template void launch_mg_sweep<T>(chy_ctx *, const Grid &, const double[3], const T *, const T *, const double *,  \
+                                   const T *, const T *, T *, double);                                              \
+  template void launch_mg_residual<T>(chy_ctx *, const Grid &, const double[3], const T *, const T *, const T *, T *);
+MG_INST(double)
+MG_INST(float)
+#undef MG_INST
 
 // Both once-per-solve column walks of the two-level preconditioners for the
 // full operator (COEF: k_zcoef's z-means, FACT: k_zline_factor's factors,
@@ -2152,33 +2378,6 @@ bool zline_e2_applies(chy_ctx *ctx)
   return kz_operator(ctx->prm.lhs_type, full_scoef(ctx->prm.d, ctx->prm.kappa_e));
 }
 
-// The wave-per-column form for grids of at most kZlineWaveCols columns and 3 to
-// 512 planes (the multigrid's coarse levels); otherwise the thread-per-column
-// one.  A wave's loads along its column touch one cache line per value, so
-// above a few thousand columns the thread-per-column form, whose loads are
-// coalesced across columns, is faster despite its serial walk.
-constexpr int64_t kZlineWaveCols = 4096;
-template <typename T>
-void launch_zline_apply_coarse(chy_ctx *ctx, const Grid &g, const T *zbuf, const double *colbuf, T *res, T *z,
-                               double scale)
-{
-  const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
-  const int m = g.nz;
-  if (plane > kZlineWaveCols || m < 3 || m > 512) {
-    launch_zline_apply_g<T>(ctx, g, zbuf, colbuf, res, z, scale);
-    return;
-  }
-  const unsigned nb = (unsigned)((plane + 3) / 4);
-#define ZW(P)                                                                                                      \
-  hipLaunchKernelGGL((k_zline_apply_wave<T, P>), nb, 256, 0, ctx->stream, g, zbuf, zbuf + nc, zbuf + 2 * nc,       \
-                     zbuf + 3 * nc, colbuf, colbuf + plane, (const T *)res, z, scale)
-  if (m <= 64) ZW(1);
-  else if (m <= 128) ZW(2);
-  else if (m <= 256) ZW(4);
-  else ZW(8);
-#undef ZW
-}
-
 template <typename T>
 void launch_zline_factor_g(chy_ctx *ctx, const Grid &g, const double d[3], int lhs_type, const T *n, T *zbuf,
                            double *colbuf)
@@ -2229,10 +2428,6 @@ template void launch_zline_apply_g<double>(chy_ctx *, const Grid &, const double
                                            double *, double);
 template void launch_zline_apply_g<float>(chy_ctx *, const Grid &, const float *, const double *, float *, float *,
                                           double);
-template void launch_zline_apply_coarse<double>(chy_ctx *, const Grid &, const double *, const double *, double *,
-                                                double *, double);
-template void launch_zline_apply_coarse<float>(chy_ctx *, const Grid &, const float *, const double *, float *,
-                                               float *, double);
 template void launch_zline_factor_g<double>(chy_ctx *, const Grid &, const double *, int, const double *, double *,
                                             double *);
 template void launch_zline_factor_g<float>(chy_ctx *, const Grid &, const double *, int, const float *, float *,

@@ -420,13 +420,20 @@ void launch_zline_factor_g(chy_ctx *ctx, const Grid &g, const double d[3], int l
 template <typename T>
 void launch_zline_apply_g(chy_ctx *ctx, const Grid &g, const T *zbuf, const double *colbuf, T *res, T *z,
                           double scale);
-// the same, one wave per column on grids of few columns (res is only read)
-template <typename T>
-void launch_zline_apply_coarse(chy_ctx *ctx, const Grid &g, const T *zbuf, const double *colbuf, T *res, T *z,
-                               double scale);
 template <typename T>
 void launch_residual_g(chy_ctx *ctx, const Grid &g, const double d[3], int lhs_type, const T *n, const T *b,
                        const T *x, T *res);
+// multigrid levels, fields as [y][x][z] (z fastest), at most kMgMaxPlanes planes:
+// transposes of nf <= 5 fields to or from [z][y][x]; one sweep xo = x + omega
+// zline^-1 (b - A x) (x null: from zero; xo is not x); r = b - A x.  zf: the factors za, zi, zc, zq (nc each).
+constexpr int kMgMaxPlanes = 512;
+template <typename T>
+void launch_mg_transpose(chy_ctx *ctx, const Grid &g, bool to_z, int nf, const T *const *src, T *const *dst);
+template <typename T>
+void launch_mg_sweep(chy_ctx *ctx, const Grid &g, const double d[3], const T *n, const T *zf, const double *zcol,
+                     const T *b, const T *x, T *xo, double omega);
+template <typename T>
+void launch_mg_residual(chy_ctx *ctx, const Grid &g, const double d[3], const T *n, const T *b, const T *x, T *r);
 // The two-level preconditioner z = fft2(r).  With zline set it goes on to
 // fft2z's z-line stage, z += zline(r - A(n) z), in the fused form where that
 // applies, and says so in *zline_done (else the caller runs the stage); w3 is

@@ -14,6 +14,8 @@
 // cycle from a zero guess per application, 8 sweeps on the coarsest level.
 // Unlike the FFT preconditioners it needs no power-of-two axes, and its
 // iteration counts do not grow with the grid or with the density contrast.
+#include <utility>
+
 #include "chy_internal.h"
 
 namespace chy {
@@ -29,21 +31,46 @@ struct MgLevel {
   Grid g;
   double d[3];
   void *n = nullptr, *x = nullptr, *b = nullptr, *r = nullptr, *zf = nullptr;  // T arrays
+  void *nz = nullptr, *x2 = nullptr;  // the density with z fastest, the sweeps' other x
   double *zcol = nullptr;  // per-column z-line scalars (2 per column)
 };
 
 struct Mg {
   int nlev = 0;
   MgLevel lv[kMgMax];
+  bool zfast = false;   // level fields as [y][x][z] (at most kMgMaxPlanes planes)
+  void *tmp = nullptr;  // z-line factors of a level before their transposition
 };
 
 // c = x-y full weighting of f (weights 1/4, 1/2, 1/4 along x and y, periodic).
-template <typename T>
+// ZF: fields as [y][x][z].
+template <bool ZF>
+__device__ __forceinline__ int64_t mg_at(const Grid &g, int i, int j, int k)
+{
+  return ZF ? (int64_t)k + (int64_t)g.nz * ((int64_t)i + (int64_t)g.nx * j)
+            : (int64_t)i + (int64_t)g.nx * ((int64_t)j + (int64_t)g.ny * k);
+}
+
+template <bool ZF>
+__device__ __forceinline__ void mg_split(const Grid &g, int64_t q, int &i, int &j, int &k)
+{
+  if (ZF) {
+    const uint32_t col = (uint32_t)q / (uint32_t)g.nz;  // nc < 2^31
+    k = (int)((uint32_t)q - col * (uint32_t)g.nz);
+    int z;
+    split_cell(g, (int)col, i, j, z);
+  } else {
+    split_cell(g, (int)q, i, j, k);
+  }
+}
+
+template <typename T, bool ZF>
 __global__ __launch_bounds__(256) void k_mg_restrict(Grid gf, Grid gc, const T *__restrict__ f, T *__restrict__ c)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= gc.nc) return;
-  const int I = (int)(q % gc.nx), J = (int)((q / gc.nx) % gc.ny), k = (int)(q / ((int64_t)gc.nx * gc.ny));
+  int I, J, k;
+  mg_split<ZF>(gc, q, I, J, k);
   const double w[3] = {0.25, 0.5, 0.25};
   double s = 0.0;
 #pragma unroll
@@ -52,24 +79,25 @@ __global__ __launch_bounds__(256) void k_mg_restrict(Grid gf, Grid gc, const T *
 #pragma unroll
     for (int a = 0; a < 3; a++) {
       const int i = wrapi(2 * I + a - 1, gf.nx);
-      s += (w[bq] * w[a]) * (double)f[(int64_t)i + (int64_t)gf.nx * ((int64_t)j + (int64_t)gf.ny * k)];
+      s += (w[bq] * w[a]) * (double)f[mg_at<ZF>(gf, i, j, k)];
     }
   }
   c[q] = (T)s;
 }
 
 // f += bilinear x-y interpolation of c.
-template <typename T>
+template <typename T, bool ZF>
 __global__ __launch_bounds__(256) void k_mg_prolong(Grid gf, Grid gc, const T *__restrict__ c, T *__restrict__ f)
 {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= gf.nc) return;
-  const int i = (int)(q % gf.nx), j = (int)((q / gf.nx) % gf.ny), k = (int)(q / ((int64_t)gf.nx * gf.ny));
+  int i, j, k;
+  mg_split<ZF>(gf, q, i, j, k);
   const int I0 = i >> 1, J0 = j >> 1;
   const int I1 = (i & 1) ? (I0 + 1 == gc.nx ? 0 : I0 + 1) : I0, J1 = (j & 1) ? (J0 + 1 == gc.ny ? 0 : J0 + 1) : J0;
-  const T *ck = c + (int64_t)gc.nx * gc.ny * k;
-  const double v = 0.25 * (((double)ck[I0 + (int64_t)gc.nx * J0] + (double)ck[I1 + (int64_t)gc.nx * J0]) +
-                           ((double)ck[I0 + (int64_t)gc.nx * J1] + (double)ck[I1 + (int64_t)gc.nx * J1]));
+  const double v =
+      0.25 * (((double)c[mg_at<ZF>(gc, I0, J0, k)] + (double)c[mg_at<ZF>(gc, I1, J0, k)]) +
+              ((double)c[mg_at<ZF>(gc, I0, J1, k)] + (double)c[mg_at<ZF>(gc, I1, J1, k)]));
   f[q] = (T)((double)f[q] + v);
 }
 
@@ -88,6 +116,33 @@ int level_sizes(int64_t nx, int64_t ny, int64_t out[kMgMax][2])
   return L;
 }
 
+// The V-cycle on levels with z fastest: A x = b from zero; the result is in
+// the returned buffer, L.x or L.x2.
+template <typename T>
+T *vcycle_z(chy_ctx *ctx, Mg &M, int l)
+{
+  MgLevel &L = M.lv[l];
+  const Grid &g = L.g;
+  const T *n = (const T *)L.nz, *zf = (const T *)L.zf, *b = (const T *)L.b;
+  T *x = (T *)L.x, *y = (T *)L.x2;
+  const bool coarsest = l == M.nlev - 1;
+  launch_mg_sweep<T>(ctx, g, L.d, n, zf, L.zcol, b, (const T *)nullptr, x, kMgOmega);
+  auto sweep = [&]() {
+    launch_mg_sweep<T>(ctx, g, L.d, n, zf, L.zcol, b, (const T *)x, y, kMgOmega);
+    std::swap(x, y);
+  };
+  for (int s = 1; s < (coarsest ? kMgCoarseSweeps : kMgSweeps); s++) sweep();
+  if (coarsest) return x;
+  MgLevel &C = M.lv[l + 1];
+  launch_mg_residual<T>(ctx, g, L.d, n, b, (const T *)x, (T *)L.r);
+  hipLaunchKernelGGL((k_mg_restrict<T, true>), nb_of(C.g.nc), kBlock, 0, ctx->stream, g, C.g, (const T *)L.r, (T *)C.b);
+  const T *xc = vcycle_z<T>(ctx, M, l + 1);
+  hipLaunchKernelGGL((k_mg_prolong<T, true>), nb_of(g.nc), kBlock, 0, ctx->stream, g, C.g, xc, x);
+  for (int s = 0; s < kMgSweeps; s++) sweep();
+  return x;
+}
+
+// The same with x fastest, for columns longer than kMgMaxPlanes.
 template <typename T>
 void vcycle(chy_ctx *ctx, Mg &M, int l, const T *b, T *x)
 {
@@ -100,19 +155,19 @@ void vcycle(chy_ctx *ctx, Mg &M, int l, const T *b, T *x)
   // overwrites its input, so it gets a copy)
   launch_fill<T>(ctx, g.nc, x, (T)0);
   (void)hipMemcpyAsync(r, b, sizeof(T) * g.nc, hipMemcpyDeviceToDevice, ctx->stream);
-  launch_zline_apply_coarse<T>(ctx, g, zf, L.zcol, r, x, kMgOmega);
+  launch_zline_apply_g<T>(ctx, g, zf, L.zcol, r, x, kMgOmega);
   auto sweep = [&]() {
     launch_residual_g<T>(ctx, g, L.d, lt, n, b, x, r);
-    launch_zline_apply_coarse<T>(ctx, g, zf, L.zcol, r, x, kMgOmega);
+    launch_zline_apply_g<T>(ctx, g, zf, L.zcol, r, x, kMgOmega);
   };
   const bool coarsest = l == M.nlev - 1;
   for (int s = 1; s < (coarsest ? kMgCoarseSweeps : kMgSweeps); s++) sweep();
   if (coarsest) return;
   MgLevel &C = M.lv[l + 1];
   launch_residual_g<T>(ctx, g, L.d, lt, n, b, x, r);
-  hipLaunchKernelGGL((k_mg_restrict<T>), nb_of(C.g.nc), kBlock, 0, ctx->stream, g, C.g, (const T *)r, (T *)C.b);
+  hipLaunchKernelGGL((k_mg_restrict<T, false>), nb_of(C.g.nc), kBlock, 0, ctx->stream, g, C.g, (const T *)r, (T *)C.b);
   vcycle<T>(ctx, M, l + 1, (const T *)C.b, (T *)C.x);
-  hipLaunchKernelGGL((k_mg_prolong<T>), nb_of(g.nc), kBlock, 0, ctx->stream, g, C.g, (const T *)C.x, x);
+  hipLaunchKernelGGL((k_mg_prolong<T, false>), nb_of(g.nc), kBlock, 0, ctx->stream, g, C.g, (const T *)C.x, x);
   for (int s = 0; s < kMgSweeps; s++) sweep();
 }
 
@@ -125,7 +180,12 @@ int mg_setup(chy_ctx *ctx)
   ctx->mg = M;
   int64_t sz[kMgMax][2];
   M->nlev = level_sizes(p.N[0], p.N[1], sz);
+  M->zfast = p.N[2] <= kMgMaxPlanes;
   const size_t ts = ctx->mixed ? 4 : 8;
+  if (M->zfast) {
+    unsigned char *q = nullptr;
+    TRY(dalloc(ctx, &q, (int64_t)ts * 4 * ctx->g.nc)); M->tmp = q;
+  }
   for (int l = 0; l < M->nlev; l++) {
     MgLevel &L = M->lv[l];
     Grid &g = L.g;
@@ -144,10 +204,14 @@ int mg_setup(chy_ctx *ctx)
     TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.r = q;
     TRY(dalloc(ctx, &q, (int64_t)ts * 4 * nc)); L.zf = q;
     TRY(dalloc(ctx, &L.zcol, 2 * plane));
-    if (l > 0) {
-      TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.n = q;
+    if (l > 0) { TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.n = q; }
+    if (l > 0 || M->zfast) {
       TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.x = q;
       TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.b = q;
+    }
+    if (M->zfast) {
+      TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.nz = q;
+      TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.x2 = q;
     }
   }
   return CHY_OK;
@@ -159,9 +223,10 @@ void mg_release(chy_ctx *ctx)
   if (!M) return;
   for (int l = 0; l < M->nlev; l++) {
     MgLevel &L = M->lv[l];
-    void *ps[] = {L.r, L.zf, L.zcol, l > 0 ? L.n : nullptr, L.x, L.b};
+    void *ps[] = {L.r, L.zf, L.zcol, l > 0 ? L.n : nullptr, L.x, L.b, L.nz, L.x2};
     for (void *p : ps) if (p) (void)hipFree(p);
   }
+  if (M->tmp) (void)hipFree(M->tmp);
   delete M;
   ctx->mg = nullptr;
 }
@@ -179,9 +244,16 @@ int mg_prepare(chy_ctx *ctx, const T *n)
   for (int l = 0; l < M->nlev; l++) {
     MgLevel &L = M->lv[l];
     if (l > 0)
-      hipLaunchKernelGGL((k_mg_restrict<T>), nb_of(L.g.nc), kBlock, 0, ctx->stream, M->lv[l - 1].g, L.g,
+      hipLaunchKernelGGL((k_mg_restrict<T, false>), nb_of(L.g.nc), kBlock, 0, ctx->stream, M->lv[l - 1].g, L.g,
                          (const T *)M->lv[l - 1].n, (T *)L.n);
-    launch_zline_factor_g<T>(ctx, L.g, L.d, ctx->prm.lhs_type, (const T *)L.n, (T *)L.zf, L.zcol);
+    T *zf = M->zfast ? (T *)M->tmp : (T *)L.zf;
+    launch_zline_factor_g<T>(ctx, L.g, L.d, ctx->prm.lhs_type, (const T *)L.n, zf, L.zcol);
+    if (M->zfast) {
+      const int64_t nc = L.g.nc;
+      const T *src[5] = {(const T *)L.n, zf, zf + nc, zf + 2 * nc, zf + 3 * nc};
+      T *lz = (T *)L.zf, *dst[5] = {(T *)L.nz, lz, lz + nc, lz + 2 * nc, lz + 3 * nc};
+      launch_mg_transpose<T>(ctx, L.g, true, 5, src, dst);
+    }
   }
   CHY_HIP(hipGetLastError());
   return CHY_OK;
@@ -193,7 +265,15 @@ int mg_apply(chy_ctx *ctx, const T *r, T *z)
 {
   Mg *M = (Mg *)ctx->mg;
   if (!M || !M->lv[0].n) return set_err(ctx, CHY_ERR_LIB, "multigrid used before its set-up");
-  vcycle<T>(ctx, *M, 0, r, z);
+  if (M->zfast) {
+    const Grid &g = M->lv[0].g;
+    T *b = (T *)M->lv[0].b;
+    launch_mg_transpose<T>(ctx, g, true, 1, &r, &b);
+    const T *x = vcycle_z<T>(ctx, *M, 0);
+    launch_mg_transpose<T>(ctx, g, false, 1, &x, &z);
+  } else {
+    vcycle<T>(ctx, *M, 0, r, z);
+  }
   CHY_HIP(hipGetLastError());
   return CHY_OK;
 }
