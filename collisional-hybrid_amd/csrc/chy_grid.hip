@@ -1920,6 +1920,154 @@ __global__ __launch_bounds__(256) void k_zline_apply_e2(Grid g, const T *__restr
   }
 }
 
+// ---- z-line stage with the columns cut into segments -------------------------------
+// k_zline_apply and k_zline_apply_e2 in one pass over memory: NC consecutive
+// columns a block, each cut into SG segments of P planes, a thread a segment,
+// whose values stay in registers from the load to the store.  The forward and
+// back substitutions are first-order linear recurrences: every thread composes
+// the affine map of its planes, runs through the maps before (after) it for the
+// value that enters them, and then its planes with the sequential formulas.
+//
+// One thread a column leaves most of the chip idle (4 blocks at 32^2, 64 at
+// 128^2) and reads the intermediate values back twice.  Measured with the 2-D
+// correction folded in, column walk -> segments: 32^3 FP64 19.3 -> 4.7 us, 64^3
+// FP32 23.1 -> 5.8, 128^3 FP32 45.6 -> 16.2 and FP64 72.7 -> 28.0, 128x128x256
+// FP64 172 -> 66, 256^3 FP32 145 -> 137.  On the largest FP64 grids the walk's
+// block reads longer runs of each plane: 256x256x128 137 -> 129, but 256^3 271
+// -> 297, so those keep the walk, as columns beyond 256 planes do, whose values
+// do not fit the registers.  Blocks of 16 columns were the faster ones but for
+// FP32 columns of more than 64 planes (64-byte runs of a plane against 128);
+// 8 to 64 segments were tried with 1 to 16 planes each.
+template <typename T, int NC, int SG, int P, bool E2>
+__global__ __launch_bounds__(NC * SG) void k_zline_seg(Grid g, const T *__restrict__ za, const T *__restrict__ zi,
+                                                       const T *__restrict__ zc, const T *__restrict__ zq,
+                                                       const double *__restrict__ cag,
+                                                       const double *__restrict__ cden, const T *__restrict__ res,
+                                                       T *__restrict__ z, const T *__restrict__ n, SCoef s,
+                                                       const T *__restrict__ Z2, const double *__restrict__ y2,
+                                                       double scale)
+{
+  __shared__ double mA[SG][NC], mB[SG][NC], ends[2][NC];
+  uint32_t bx, by, bz;
+  (void)xcd_tile(bx, by, bz);
+  const int plane = g.nx * g.ny, m = g.nz, cx = threadIdx.x % NC, sg = threadIdx.x / NC;
+  const int col = (int)bx * NC + cx;
+  const bool live = col < plane;
+  // (loads past the last plane or column read a valid value that is not used)
+  int64_t e[P];
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    const int k = sg * P + u;
+    e[u] = (live ? col : 0) + (int64_t)plane * (k < m ? k : m - 1);
+  }
+  double r[P];
+  T cc[P];
+  double ec = 0.0;
+  {
+    T rr[P], aa[P], ii[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      rr[u] = res[e[u]];
+      aa[u] = za[e[u]];
+      ii[u] = zi[e[u]];
+      cc[u] = zc[e[u]];
+    }
+    if constexpr (E2) {
+      // (A e2)(k) from the column's five constants, as k_zline_apply_e2
+      int i, j, k_;
+      split_cell(g, live ? col : 0, i, j, k_);
+      const int ip = i + 1 == g.nx ? 0 : i + 1, im = i == 0 ? g.nx - 1 : i - 1;
+      const int jp = j + 1 == g.ny ? 0 : j + 1, jm = j == 0 ? g.ny - 1 : j - 1;
+      const int64_t oxp = ip - i, oxm = im - i, oyp = (int64_t)g.nx * (jp - j), oym = (int64_t)g.nx * (jm - j);
+      T nc[P], nxp[P], nxm[P], nyp[P], nym[P];
+#pragma unroll
+      for (int u = 0; u < P; u++) {
+        nc[u] = n[e[u]];
+        nxp[u] = n[e[u] + oxp]; nxm[u] = n[e[u] + oxm];
+        nyp[u] = n[e[u] + oyp]; nym[u] = n[e[u] + oym];
+      }
+      const double y0 = y2[0], y1 = y2[1];
+      auto e2 = [&](int ii, int jj) {
+        const int q = ii + g.nx * jj;
+        return y0 * (double)Z2[q] + y1 * (double)Z2[(int64_t)plane + q];
+      };
+      ec = e2(i, j);
+      const double de0 = e2(ip, j) - ec, de1 = e2(im, j) - ec, de2 = e2(i, jp) - ec, de3 = e2(i, jm) - ec;
+      const double de6 = e2(ip, jp) - ec, de7 = e2(ip, jm) - ec, de8 = e2(im, jp) - ec, de9 = e2(im, jm) - ec;
+      const double kc = s.sxx * (de0 + de1) + s.syy * (de2 + de3) + (s.sxy + s.syx) * ((de6 - de7) + (de9 - de8));
+      const double kxp = s.sxx * de0 + s.sxy * (de2 - de3) + s.sxy * (de6 - de7);
+      const double kxm = s.sxx * de1 - s.sxy * (de2 - de3) + s.sxy * (de9 - de8);
+      const double kyp = s.syx * (de0 - de1) + s.syy * de2 + s.syx * (de6 - de8);
+      const double kym = -s.syx * (de0 - de1) + s.syy * de3 + s.syx * (de9 - de7);
+#pragma unroll
+      for (int u = 0; u < P; u++)
+        r[u] = (double)rr[u] - (kc * (double)nc[u] + kxp * (double)nxp[u] + kxm * (double)nxm[u] + kyp * (double)nyp[u] +
+                                kym * (double)nym[u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < P; u++) r[u] = (double)rr[u];
+    }
+    double A = 1.0, B = 0.0;
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      if (sg * P + u < m) {
+        const double iv = (double)ii[u], al = -(double)aa[u] * iv;
+        A = al * A;
+        B = al * B + r[u] * iv;
+      }
+    }
+    mA[sg][cx] = A;
+    mB[sg][cx] = B;
+    __syncthreads();
+    double y = 0.0;
+    for (int t = 0; t < sg; t++) y = mA[t][cx] * y + mB[t][cx];
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      if (sg * P + u < m) {
+        y = (r[u] - (double)aa[u] * y) * (double)ii[u];
+        r[u] = y;
+      }
+    }
+    if (sg == (m - 1) / P) ends[0][cx] = y;
+  }
+  __syncthreads();  // (the maps are read; the last y is known)
+  const double ylast = ends[0][cx];
+  double A = 1.0, B = 0.0;
+#pragma unroll
+  for (int u = P - 1; u >= 0; u--) {
+    const int k = sg * P + u;
+    if (k == m - 1) { A = 0.0; B = ylast; }
+    else if (k < m - 1) { B = r[u] - (double)cc[u] * B; A = -(double)cc[u] * A; }
+  }
+  mA[sg][cx] = A;
+  mB[sg][cx] = B;
+  // the final operands are in flight while the maps are run through
+  T qq[P], zz[P];
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    qq[u] = zq[e[u]];
+    zz[u] = z[e[u]];
+  }
+  const double ag = live ? cag[col] : 0.0, dn = live ? cden[col] : 1.0;
+  __syncthreads();
+  double x = 0.0;
+  for (int t = SG - 1; t > sg; t--) x = mA[t][cx] * x + mB[t][cx];
+#pragma unroll
+  for (int u = P - 1; u >= 0; u--) {
+    const int k = sg * P + u;
+    if (k == m - 1) x = ylast;
+    else if (k < m - 1) { x = r[u] - (double)cc[u] * x; r[u] = x; }
+  }
+  if (sg == 0) ends[1][cx] = x;
+  __syncthreads();
+  const double f = (ends[1][cx] + ag * ylast) / dn;
+#pragma unroll
+  for (int u = 0; u < P; u++) {
+    if (live && sg * P + u < m)
+      z[e[u]] = (T)(((double)zz[u] + ec) + scale * (r[u] - f * (double)qq[u]));
+  }
+}
+
 // ---- multigrid levels with z fastest ----------------------------------------------
 // The multigrid keeps its level fields as [y][x][z]: a group of W lanes owns a
 // column, P consecutive planes a lane (W P >= nz), so that the stencil around a
@@ -2350,11 +2498,36 @@ void launch_zline_apply(chy_ctx *ctx, const T *zbuf, const double *colbuf, T *re
   launch_zline_apply_g<T>(ctx, ctx->g, zbuf, colbuf, res, z, 1.0);
 }
 
+// The segmented z-line stage where it is the faster one; false: it is not.
+template <typename T, bool E2>
+static bool launch_zline_seg(chy_ctx *ctx, const Grid &g, const T *zbuf, const double *colbuf, const T *res, T *z,
+                             const T *n, const SCoef &s, const T *Z2, const double *y2, double scale)
+{
+  const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
+  constexpr bool fp32 = sizeof(T) == 4;
+  if (g.nz > 256 || (!fp32 && g.nz > 128 && nc > (int64_t)1 << 23)) return false;
+#define ZSEG(NC, SG, P)                                                                                             \
+  hipLaunchKernelGGL((k_zline_seg<T, NC, SG, P, E2>), (unsigned)((plane + NC - 1) / NC), NC * SG, 0, ctx->stream, g, \
+                     zbuf, zbuf + nc, zbuf + 2 * nc, zbuf + 3 * nc, colbuf, colbuf + plane, res, z, n, s, Z2, y2, scale)
+  if (g.nz <= 32) ZSEG(16, 8, 4);
+  else if (g.nz <= 64) ZSEG(16, 8, 8);
+  else if constexpr (fp32) {
+    if (g.nz <= 128) ZSEG(32, 16, 8);
+    else ZSEG(32, 16, 16);
+  } else {
+    if (g.nz <= 128) ZSEG(16, 16, 8);
+    else ZSEG(16, 32, 8);
+  }
+#undef ZSEG
+  return true;
+}
+
 template <typename T>
 void launch_zline_apply_g(chy_ctx *ctx, const Grid &g, const T *zbuf, const double *colbuf, T *res, T *z,
                           double scale)
 {
   const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
+  if (launch_zline_seg<T, false>(ctx, g, zbuf, colbuf, res, z, nullptr, SCoef(), nullptr, nullptr, scale)) return;
   hipLaunchKernelGGL((k_zline_apply<T>), nblocks(plane), kBlock, 0, ctx->stream, g, zbuf, zbuf + nc,
                      zbuf + 2 * nc, zbuf + 3 * nc, colbuf, colbuf + plane, res, z, scale);
 }
@@ -2369,6 +2542,7 @@ void launch_zline_apply_e2(chy_ctx *ctx, const T *zbuf, const double *colbuf, T 
   const Grid &g = ctx->g;
   const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
   const SCoef s = full_scoef(ctx->prm.d, ctx->prm.kappa_e);
+  if (launch_zline_seg<T, true>(ctx, g, zbuf, colbuf, res, z, n, s, Z2, y2, 1.0)) return;
   hipLaunchKernelGGL((k_zline_apply_e2<T, kFft2Its>), nblocks(plane), kBlock, 0, ctx->stream, g, zbuf, zbuf + nc,
                      zbuf + 2 * nc, zbuf + 3 * nc, colbuf, colbuf + plane, res, z, n, s, Z2, y2);
 }

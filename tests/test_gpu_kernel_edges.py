@@ -82,3 +82,28 @@ def test_multigrid_columns_of_any_length(N, extra, prec, tol):
     ref = orc.pc_apply(g, K, mom[0], r, orc.PC_MG, lhs_type=lt)
     z, ref = z - z.mean(), ref - ref.mean()
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
+
+
+# the z-line stage in segments: full and ragged columns of each segmentation,
+# planes that are no multiple of a block's 16 or 32 columns (x-y axes of a power
+# of two, as the preconditioner needs), and the column walk beyond 256 planes;
+# B along z (the 2-D correction folded in) and oblique (the plain stage)
+@pytest.mark.parametrize("prec,base", [("fp64", 1e-11), ("mixed", 2e-5)])
+@pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5"])
+@pytest.mark.parametrize("N", [(4, 4, 4), (8, 4, 8), (4, 4, 32), (8, 8, 64), (16, 4, 128), (8, 4, 256), (4, 4, 512)])
+def test_zline_stage_on_columns_of_any_length(N, extra, prec, base):
+    rng = np.random.default_rng(14)
+    with context(opts(N, extra=f"-pc_type fft2z -precision {prec} {extra}")) as ctx:
+        g = grid_of(ctx.prm)
+        mom = [m.astype(np.float32).astype(np.float64) for m in _moments(g, rng, amp=0.1)]
+        ctx.set_moments(vlasov_from(mom))
+        r = rng.standard_normal(g.nc)
+        r -= r.mean()
+        z = ctx.pc_apply(r)
+        K = list(ctx.prm.kappa_e)
+    # the FFT stage's symbol, as in the test of the 2-D correction, and the z-line
+    # systems' condition, 2 (1 + K_z^2) / (1 - cos(2 pi / nz)) ulps at most
+    tol = base + 16 * 2.0 ** -52 * (3 + K[2] ** 2) / (1 - np.cos(2 * np.pi / max(N)))
+    ref = orc.pc_apply(g, K, mom[0], r, orc.PC_FFT2Z)
+    z, ref = z - z.mean(), ref - ref.mean()
+    assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
