@@ -224,8 +224,8 @@ class Context:
     # particles --------------------------------------------------------------
     def set_particles(self, x, y, z, vx, vy, vz, w=None, pid=None):
         n = len(x)
-        pos = np.zeros((n, 4))
-        vel = np.zeros((n, 4))
+        pos = np.empty((n, 4))  # (the fourth value is ignored)
+        vel = np.empty((n, 4))
         pos[:, 0], pos[:, 1], pos[:, 2] = x, y, z
         vel[:, 0], vel[:, 1], vel[:, 2] = vx, vy, vz
         w = None if w is None else _f64(w)
@@ -234,10 +234,10 @@ class Context:
 
     def get_particles(self):
         n = int(lib().chy_num_particles(self._p))
-        pos = np.zeros((n, 4))
-        vel = np.zeros((n, 4))
-        w = np.zeros(n)
-        pid = np.zeros(n, np.uint32)
+        pos = np.empty((n, 4))
+        vel = np.empty((n, 4))
+        w = np.empty(n)
+        pid = np.empty(n, np.uint32)
         self._chk(lib().chy_get_particles(self._p, _ptr(pos), _ptr(vel), _ptr(w), _ptr(pid)))
         return dict(x=pos[:, 0].copy(), y=pos[:, 1].copy(), z=pos[:, 2].copy(),
                     vx=vel[:, 0].copy(), vy=vel[:, 1].copy(), vz=vel[:, 2].copy(), w=w, pid=pid)
@@ -267,7 +267,7 @@ class Context:
         if not download:
             self._chk(lib().chy_collect_moments(self._p, None))
             return None
-        v = np.zeros((self.nc, 4))
+        v = np.empty((self.nc, 4))
         self._chk(lib().chy_collect_moments(self._p, _ptr(v)))
         return v
 
@@ -276,7 +276,7 @@ class Context:
         self._chk(lib().chy_set_moments(self._p, _ptr(v)))
 
     def get_moments(self):
-        v = np.zeros((self.nc, 4))
+        v = np.empty((self.nc, 4))
         self._chk(lib().chy_get_moments(self._p, _ptr(v)))
         return v
 
@@ -299,19 +299,19 @@ class Context:
         return rc
 
     def compute_rhs(self):
-        b = np.zeros(self.nc)
+        b = np.empty(self.nc)
         self._chk(lib().chy_compute_rhs(self._p, _ptr(b)))
         return b
 
     def lhs_apply(self, x, transpose=False):
         x = _f64(x)
-        y = np.zeros(self.nc)
+        y = np.empty(self.nc)
         f = lib().chy_lhs_apply_transpose if transpose else lib().chy_lhs_apply
         self._chk(f(self._p, _ptr(x), _ptr(y)))
         return y
 
     def solve_potential(self):
-        phi = np.zeros(self.nc)
+        phi = np.empty(self.nc)
         st = SolveStats()
         self._chk(lib().chy_solve_potential(self._p, _ptr(phi), C.byref(st)))
         return phi, st
@@ -325,12 +325,12 @@ class Context:
 
     def pc_apply(self, r):
         r = _f64(r)
-        z = np.zeros(self.nc)
+        z = np.empty(self.nc)
         self._chk(lib().chy_pc_apply(self._p, _ptr(r), _ptr(z)))
         return z
 
     def get_potential(self):
-        phi = np.zeros(self.nc)
+        phi = np.empty(self.nc)
         self._chk(lib().chy_get_potential(self._p, _ptr(phi)))
         return phi
 
@@ -339,7 +339,7 @@ class Context:
         self._chk(lib().chy_set_potential(self._p, _ptr(phi)))
 
     def get_rhs(self):
-        b = np.zeros(self.nc)
+        b = np.empty(self.nc)
         self._chk(lib().chy_get_rhs(self._p, _ptr(b)))
         return b
 

@@ -607,6 +607,7 @@ int chy_create(const chy_params *prm_in, int64_t np_capacity, chy_ctx **out)
   {
     unsigned char *q = nullptr;
     A(dalloc(ctx, &q, (int64_t)ts * nc * nvec_V(ctx))); ctx->V = q;
+    ctx->V_bytes = ts * (size_t)(nc * nvec_V(ctx));
     A(dalloc(ctx, &q, (int64_t)ts * nc * ctx->restart)); ctx->Z = q;
     A(dalloc(ctx, &q, (int64_t)ts * nc)); ctx->wv = q;
     A(dalloc(ctx, &q, (int64_t)ts * 2 * (nc + 32 * (int64_t)ctx->g.nz))); ctx->fft_buf = q;  // half spectrum, padded planes
@@ -668,6 +669,7 @@ int chy_destroy(chy_ctx *ctx)
   if (ctx->out_stream) (void)hipStreamDestroy(ctx->out_stream);
   adjoint_release(ctx);
   mg_release(ctx);
+  transfer_release(ctx);
   for (int s = 0; s < 2; s++) { free_state(ctx->pd[s]); free_state(ctx->pf[s]); }
   void *ps[] = {ctx->perm, ctx->slotkey, ctx->counts, ctx->offsets, ctx->cursor, ctx->scan_tmp, ctx->maxcount,
                 ctx->trans, ctx->info, ctx->dir, ctx->nbase, ctx->offs_alt, ctx->sortflag,
@@ -782,18 +784,7 @@ int chy_collect_moments(chy_ctx *ctx, double *vlasov)
 int chy_set_moments(chy_ctx *ctx, const double *vlasov)
 {
   if (!ctx || !vlasov) return CHY_ERR_ARG_WRONG;
-  const int64_t nc = ctx->g.nc;
-  for (int a = 0; a < 4; a++) {
-    if (ctx->mixed) {
-      std::vector<float> f(nc);
-      for (int64_t c = 0; c < nc; c++) f[c] = (float)vlasov[4 * c + a];
-      CHY_HIP(hipMemcpy(ctx->mom[a], f.data(), sizeof(float) * nc, hipMemcpyHostToDevice));
-    } else {
-      std::vector<double> f(nc);
-      for (int64_t c = 0; c < nc; c++) f[c] = vlasov[4 * c + a];
-      CHY_HIP(hipMemcpy(ctx->mom[a], f.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
-    }
-  }
+  TRY(moments_upload(ctx, vlasov));
   ctx->moments_valid = true;
   return CHY_OK;
 }
@@ -803,18 +794,7 @@ int chy_get_moments(chy_ctx *ctx, double *vlasov)
   if (!ctx || !vlasov) return CHY_ERR_ARG_WRONG;
   const int64_t nc = ctx->g.nc;
   if (!ctx->moments_valid) { for (int64_t c = 0; c < 4 * nc; c++) vlasov[c] = 0.0; return CHY_OK; }
-  for (int a = 0; a < 4; a++) {
-    std::vector<double> m(nc);
-    if (ctx->mixed) {
-      std::vector<float> f(nc);
-      CHY_HIP(hipMemcpy(f.data(), ctx->mom[a], sizeof(float) * nc, hipMemcpyDeviceToHost));
-      for (int64_t c = 0; c < nc; c++) m[c] = f[c];
-    } else {
-      CHY_HIP(hipMemcpy(m.data(), ctx->mom[a], sizeof(double) * nc, hipMemcpyDeviceToHost));
-    }
-    for (int64_t c = 0; c < nc; c++) vlasov[4 * c + a] = m[c];
-  }
-  return CHY_OK;
+  return moments_download(ctx, vlasov);
 }
 
 int chy_compute_rhs(chy_ctx *ctx, double *b)
@@ -822,7 +802,7 @@ int chy_compute_rhs(chy_ctx *ctx, double *b)
   if (!ctx) return CHY_ERR_ARG_WRONG;
   int rc = do_rhs(ctx);
   if (rc) return rc;
-  if (b) CHY_HIP(hipMemcpy(b, ctx->b, sizeof(double) * ctx->g.nc, hipMemcpyDeviceToHost));
+  if (b) return copy_to_host(ctx, b, ctx->b, sizeof(double) * ctx->g.nc);
   return sync(ctx);
 }
 
@@ -840,8 +820,7 @@ static int lhs_apply_host(chy_ctx *ctx, const double *x, double *y, bool transpo
     launch_lhs_apply<double, double, double>(ctx, ctx->prm.lhs_type, transpose, mom<double>(ctx, 0), ctx->r64,
                                              ctx->t64);
   timer_stop(ctx, "lhs_apply");
-  CHY_HIP(hipMemcpyAsync(y, ctx->t64, sizeof(double) * nc, hipMemcpyDeviceToHost, ctx->stream));
-  return sync(ctx);
+  return copy_to_host(ctx, y, ctx->t64, sizeof(double) * nc);
 }
 
 int chy_lhs_apply(chy_ctx *ctx, const double *x, double *y) { return lhs_apply_host(ctx, x, y, false); }
@@ -856,7 +835,7 @@ int chy_solve_potential(chy_ctx *ctx, double *phi, chy_solve_stats *st)
   rc = do_solve(ctx, st);
   if (st) st->ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (rc) return rc;
-  if (phi) CHY_HIP(hipMemcpy(phi, ctx->phi, sizeof(double) * ctx->g.nc, hipMemcpyDeviceToHost));
+  if (phi) return copy_to_host(ctx, phi, ctx->phi, sizeof(double) * ctx->g.nc);
   return CHY_OK;
 }
 
@@ -879,8 +858,7 @@ int chy_solve(chy_ctx *ctx, const double *b, double *phi, chy_solve_stats *st)
   ctx->phi_valid = true;
   int rc = do_solve(ctx, st);
   if (rc) return rc;
-  CHY_HIP(hipMemcpy(phi, ctx->phi, sizeof(double) * nc, hipMemcpyDeviceToHost));
-  return CHY_OK;
+  return copy_to_host(ctx, phi, ctx->phi, sizeof(double) * nc);
 }
 
 int chy_pc_apply(chy_ctx *ctx, const double *r, double *z)
@@ -901,16 +879,14 @@ int chy_pc_apply(chy_ctx *ctx, const double *r, double *z)
     TRY(pc_symbol<double>(ctx, v19));
     TRY(pc_apply<double>(ctx, v19, ctx->r64, ctx->t64));
   }
-  CHY_HIP(hipMemcpyAsync(z, ctx->t64, sizeof(double) * nc, hipMemcpyDeviceToHost, ctx->stream));
-  return sync(ctx);
+  return copy_to_host(ctx, z, ctx->t64, sizeof(double) * nc);
 }
 
 int chy_get_potential(chy_ctx *ctx, double *phi)
 {
   if (!ctx || !phi) return CHY_ERR_ARG_WRONG;
   if (!ctx->phi_valid) { for (int64_t c = 0; c < ctx->g.nc; c++) phi[c] = 0.0; return CHY_OK; }
-  CHY_HIP(hipMemcpy(phi, ctx->phi, sizeof(double) * ctx->g.nc, hipMemcpyDeviceToHost));
-  return CHY_OK;
+  return copy_to_host(ctx, phi, ctx->phi, sizeof(double) * ctx->g.nc);
 }
 
 int chy_set_potential(chy_ctx *ctx, const double *phi)
@@ -1002,8 +978,7 @@ int chy_output_wait(chy_ctx *ctx)
 int chy_get_rhs(chy_ctx *ctx, double *b)
 {
   if (!ctx || !b) return CHY_ERR_ARG_WRONG;
-  CHY_HIP(hipMemcpy(b, ctx->b, sizeof(double) * ctx->g.nc, hipMemcpyDeviceToHost));
-  return CHY_OK;
+  return copy_to_host(ctx, b, ctx->b, sizeof(double) * ctx->g.nc);
 }
 
 int chy_step(chy_ctx *ctx, chy_step_stats *st)

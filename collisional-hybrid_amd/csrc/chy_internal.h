@@ -66,6 +66,12 @@ struct Timer {
 
 }  // namespace chy
 
+namespace chy {
+constexpr size_t kStageBytes = (size_t)64 << 20;  // largest staging buffer
+constexpr int kPinThreads = 4;
+constexpr size_t kPinChunk = (size_t)2 << 20;
+}  // namespace chy
+
 struct chy_ctx {
   chy_params prm;
   chy::Grid g;
@@ -123,6 +129,7 @@ struct chy_ctx {
   // Krylov workspace (T = double in FP64 mode, float in mixed mode)
   int64_t restart = 30;
   void *V = nullptr, *Z = nullptr, *wv = nullptr;
+  size_t V_bytes = 0;           // scratch between solves
   double *red = nullptr;        // reduction partials [nblk][restart+2]
   double *red_out = nullptr;    // reduced values [red_out_n]
   int64_t red_out_n = 0;
@@ -163,6 +170,12 @@ struct chy_ctx {
   hipEvent_t out_snap = nullptr, out_copied = nullptr;
   std::thread out_thread;
   int out_rc = 0;
+  // host arrays in and out (chy_transfer.hip): the staging buffer of layout changes
+  // that V does not take, and the pinned chunks of large copies, made at first use
+  void *stage = nullptr;
+  size_t stage_bytes = 0;
+  void *pin = nullptr;
+  hipEvent_t pin_ev[chy::kPinThreads] = {};
   double *tw[3] = {nullptr, nullptr, nullptr};   // twiddles per axis (complex)
   double *trig[3] = {nullptr, nullptr, nullptr}; // cos/sin of 2 pi k / N per axis
   bool fft_ok = false;
@@ -358,6 +371,17 @@ int particles_normaliser(chy_ctx *ctx);
 // deposit of an arbitrary cell-sorted FP64 state (segments `offs`) into
 // out[4] = {sum w W, sum w W vx, sum w W vy, sum w W vz}
 void deposit_state(chy_ctx *ctx, const PState<double> &st, const uint32_t *offs, bool weighted, double *const out[4]);
+
+// ---- host arrays in and out (chy_transfer.hip) ----
+// device bytes to pageable host memory, after the work on the context's stream;
+// complete on return
+int copy_to_host(chy_ctx *ctx, void *dst, const void *src, size_t bytes);
+int moments_upload(chy_ctx *ctx, const double *v);   // [nc][4] f64
+int moments_download(chy_ctx *ctx, double *v);
+// the current generation's ions from or to the ABI's arrays (w: weighted contexts)
+int ions_upload(chy_ctx *ctx, int64_t np, const double *pos, const double *vel, const double *w, const uint32_t *pid);
+int ions_download(chy_ctx *ctx, int64_t np, double *pos, double *vel, double *w, uint32_t *pid);
+void transfer_release(chy_ctx *ctx);
 
 // ---- diagnostics (chy_diag.hip) ----
 int diagnostics(chy_ctx *ctx, chy_diag_stats *d);

@@ -1548,18 +1548,6 @@ static int settle(chy_ctx *ctx)
   return particles_normaliser(ctx);
 }
 
-// The device wrap rule on the host (upload of positions from the caller).
-static double host_wrap(double x, double p0, double p1, double L)
-{
-  if (!(x >= p0 - L && x < p1 + L)) {
-    if (!std::isfinite(x)) return x;
-    x = x - std::floor((x - p0) / L) * L;
-  }
-  if (x < p0) { x += L; if (x >= p1) x = p0; }
-  else if (x >= p1) { x -= L; if (x < p0) x = p0; }
-  return x;
-}
-
 int particles_upload(chy_ctx *ctx, int64_t np, const double *pos, const double *vel, const double *w,
                      const uint32_t *pid)
 {
@@ -1567,60 +1555,8 @@ int particles_upload(chy_ctx *ctx, int64_t np, const double *pos, const double *
   if (w && !ctx->weighted) return set_err(ctx, CHY_ERR_ARG_INCOMP, "weights given but the context has no weight buffers");
   ctx->np = np;
   if (np == 0) return settle(ctx);
-  const chy::Grid &g = ctx->g;
-  std::vector<uint32_t> hp(np);
-  for (int64_t i = 0; i < np; i++) hp[i] = pid ? pid[i] : (uint32_t)i;
-  if (!ctx->mixed) {
-    std::vector<double> a(np);
-    PState<double> &s = ctx->pd[ctx->cur];
-    double *dst[6] = {s.x, s.y, s.z, s.vx, s.vy, s.vz};
-    for (int f = 0; f < 6; f++) {
-      const double *src = f < 3 ? pos : vel;
-      for (int64_t i = 0; i < np; i++) a[i] = src[4 * i + (f % 3)];
-      if (f < 3) {
-        // wrap into [p0, p1) as the move does
-        for (int64_t i = 0; i < np; i++) {
-          a[i] = host_wrap(a[i], g.p0[f], g.p1[f], g.L[f]);
-        }
-      }
-      CHY_HIP(hipMemcpyAsync(dst[f], a.data(), sizeof(double) * np, hipMemcpyHostToDevice, ctx->stream));
-      CHY_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    if (w) CHY_HIP(hipMemcpyAsync(s.w, w, sizeof(double) * np, hipMemcpyHostToDevice, ctx->stream));
-    else if (ctx->weighted) launch_fill<double>(ctx, np, s.w, 1.0);
-    CHY_HIP(hipMemcpyAsync(s.pid, hp.data(), sizeof(uint32_t) * np, hipMemcpyHostToDevice, ctx->stream));
-    CHY_HIP(hipStreamSynchronize(ctx->stream));
-  } else {
-    PState<float> &s = ctx->pf[ctx->cur];
-    std::vector<Vec4<float>> hp4(np), hv4(np);
-    std::vector<int32_t> cell(np);
-    const int nn[3] = {g.nx, g.ny, g.nz};
-    for (int64_t i = 0; i < np; i++) {
-      int ci[3];
-      float o[3];
-      for (int a = 0; a < 3; a++) {
-        const double p0 = g.p0[a];
-        const double x = host_wrap(pos[4 * i + a], p0, g.p1[a], g.L[a]);
-        const double xi = (x - p0) / g.d[a];
-        int ii = (int)xi;
-        if (ii > nn[a] - 1) ii = nn[a] - 1;
-        float f = (float)(xi - (double)ii);
-        if (f >= 1.0f) { f = 0.0f; ii = (ii + 1) % nn[a]; }
-        ci[a] = ii;
-        o[a] = f;
-      }
-      uint32_t id = hp[i];
-      float idf;
-      memcpy(&idf, &id, sizeof idf);
-      hp4[i] = Vec4<float>{o[0], o[1], o[2], w ? (float)w[i] : 1.0f};
-      hv4[i] = Vec4<float>{(float)vel[4 * i], (float)vel[4 * i + 1], (float)vel[4 * i + 2], idf};
-      cell[i] = ci[0] + g.nx * (ci[1] + g.ny * ci[2]);
-    }
-    CHY_HIP(hipMemcpyAsync(s.pos, hp4.data(), sizeof(Vec4<float>) * np, hipMemcpyHostToDevice, ctx->stream));
-    CHY_HIP(hipMemcpyAsync(s.vel, hv4.data(), sizeof(Vec4<float>) * np, hipMemcpyHostToDevice, ctx->stream));
-    CHY_HIP(hipMemcpyAsync(s.cell, cell.data(), sizeof(int32_t) * np, hipMemcpyHostToDevice, ctx->stream));
-    CHY_HIP(hipStreamSynchronize(ctx->stream));
-  }
+  if (!ctx->mixed && !w && ctx->weighted) launch_fill<double>(ctx, np, ctx->pd[ctx->cur].w, 1.0);
+  TRY(ions_upload(ctx, np, pos, vel, w, pid));
   return settle(ctx);
 }
 
@@ -1628,58 +1564,7 @@ int particles_download(chy_ctx *ctx, double *pos, double *vel, double *w, uint32
 {
   const int64_t np = ctx->np;
   if (np == 0) return CHY_OK;
-  const chy::Grid &g = ctx->g;
-  if (!ctx->mixed) {
-    const PState<double> &s = ctx->pd[ctx->cur];
-    std::vector<double> a[6];
-    const double *src[6] = {s.x, s.y, s.z, s.vx, s.vy, s.vz};
-    for (int f = 0; f < 6; f++) {
-      a[f].resize(np);
-      CHY_HIP(hipMemcpyAsync(a[f].data(), src[f], sizeof(double) * np, hipMemcpyDeviceToHost, ctx->stream));
-    }
-    CHY_HIP(hipStreamSynchronize(ctx->stream));
-    for (int64_t i = 0; i < np; i++) {
-      if (pos) {
-        for (int q = 0; q < 3; q++) pos[4 * i + q] = a[q][i];
-        pos[4 * i + 3] = sqrt(a[0][i] * a[0][i] + a[1][i] * a[1][i] + a[2][i] * a[2][i]);
-      }
-      if (vel) {
-        for (int q = 0; q < 3; q++) vel[4 * i + q] = a[3 + q][i];
-        vel[4 * i + 3] = sqrt(a[3][i] * a[3][i] + a[4][i] * a[4][i] + a[5][i] * a[5][i]);
-      }
-    }
-    if (w) {
-      if (ctx->weighted) CHY_HIP(hipMemcpy(w, s.w, sizeof(double) * np, hipMemcpyDeviceToHost));
-      else for (int64_t i = 0; i < np; i++) w[i] = 1.0;
-    }
-    if (pid) CHY_HIP(hipMemcpy(pid, s.pid, sizeof(uint32_t) * np, hipMemcpyDeviceToHost));
-  } else {
-    const PState<float> &s = ctx->pf[ctx->cur];
-    std::vector<Vec4<float>> hp4(np), hv4(np);
-    std::vector<int32_t> cell(np);
-    CHY_HIP(hipMemcpyAsync(hp4.data(), s.pos, sizeof(Vec4<float>) * np, hipMemcpyDeviceToHost, ctx->stream));
-    CHY_HIP(hipMemcpyAsync(hv4.data(), s.vel, sizeof(Vec4<float>) * np, hipMemcpyDeviceToHost, ctx->stream));
-    CHY_HIP(hipMemcpyAsync(cell.data(), s.cell, sizeof(int32_t) * np, hipMemcpyDeviceToHost, ctx->stream));
-    CHY_HIP(hipStreamSynchronize(ctx->stream));
-    for (int64_t i = 0; i < np; i++) {
-      const int c = cell[i];
-      const int ci[3] = {c % g.nx, (c / g.nx) % g.ny, c / (g.nx * g.ny)};
-      const float o[3] = {hp4[i].x, hp4[i].y, hp4[i].z}, v[3] = {hv4[i].x, hv4[i].y, hv4[i].z};
-      double r2 = 0.0, v2 = 0.0;
-      for (int q = 0; q < 3; q++) {
-        const double x = g.p0[q] + ((double)ci[q] + (double)o[q]) * g.d[q];
-        if (pos) pos[4 * i + q] = x;
-        if (vel) vel[4 * i + q] = (double)v[q];
-        r2 += x * x;
-        v2 += (double)v[q] * (double)v[q];
-      }
-      if (pos) pos[4 * i + 3] = sqrt(r2);
-      if (vel) vel[4 * i + 3] = sqrt(v2);
-      if (w) w[i] = ctx->weighted ? (double)hp4[i].w : 1.0;
-      if (pid) memcpy(&pid[i], &hv4[i].w, sizeof(uint32_t));
-    }
-  }
-  return CHY_OK;
+  return ions_download(ctx, np, pos, vel, w, pid);
 }
 
 // The reference's placements (InitializePositions, particles.c:26-45).

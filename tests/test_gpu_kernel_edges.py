@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import orc
-from gpu_cases import context, grid_of, opts, vlasov_from
+from gpu_cases import context, grid_of, opts, random_particles, upload, vlasov_from
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,44 @@ def test_zline_stage_on_columns_of_any_length(N, extra, prec, base):
     ref = orc.pc_apply(g, K, mom[0], r, orc.PC_FFT2Z)
     z, ref = z - z.mean(), ref - ref.mean()
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
+
+
+# host arrays: one block and its neighbours, many ions on a grid whose Krylov
+# basis is too small a scratch for them (one staging piece, and several: 1.2 M
+# ions are 91 MB), and a field of 32 MiB and a bit, which comes back in pinned
+# chunks.  The values only change layout (and type, in mixed mode)
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("N,n", [((3, 3, 3), 1), ((4, 5, 6), 257), ((4, 4, 4), 70000), ((12, 10, 11), 1200000)])
+def test_ions_survive_the_host_round_trip(N, n, prec):
+    rng = np.random.default_rng(15)
+    with context(opts(N, extra=f"-precision {prec}"), capacity=n, weighted=True) as ctx:
+        p = random_particles(grid_of(ctx.prm), n, rng, weights=True)
+        p.pid = rng.permutation(n).astype(np.uint32)
+        upload(ctx, p)
+        d = ctx.get_particles()
+        L = np.array([ctx.prm.L[a] for a in range(3)])
+    back = np.argsort(d["pid"])
+    want = np.argsort(p.pid)
+    assert np.array_equal(d["pid"][back], p.pid[want])
+    # mixed: the offset within a cell rounds to FP32 (half an ulp below one, of
+    # a cell), velocities and weights to FP32
+    tol = 0.0 if prec == "fp64" else 2.0 ** -25 * 1.01
+    for a, name in enumerate("xyz"):
+        assert np.abs(d[name][back] - getattr(p, name)[want]).max() <= tol * L[a] / N[a] + 4 * 2.0 ** -53 * (tol > 0) * L[a]
+    for name in ("vx", "vy", "vz", "w"):
+        v = getattr(p, name)[want]
+        ref = v if prec == "fp64" else v.astype(np.float32).astype(np.float64)
+        assert np.array_equal(d[name][back], ref)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("N", [(3, 3, 3), (7, 5, 9), (128, 128, 129)])
+def test_grid_arrays_survive_the_host_round_trip(N, prec):
+    rng = np.random.default_rng(16)
+    with context(opts(N, extra=f"-ksp_gmres_restart 2 -precision {prec}")) as ctx:
+        v = rng.standard_normal((ctx.nc, 4))
+        ctx.set_moments(v)
+        phi = rng.standard_normal(ctx.nc)
+        ctx.set_potential(phi)
+        assert np.array_equal(ctx.get_moments(), v if prec == "fp64" else v.astype(np.float32).astype(np.float64))
+        assert np.array_equal(ctx.get_potential(), phi)
