@@ -67,8 +67,9 @@ __device__ void scatter_vjp(const PushConst &pc, uint32_t pid, double vx, double
   const U4 b = philox4x32_10(U4{pid, pc.step, STREAM_COLLIDE_B, 0u}, pc.k0, pc.k1);
   const double uz = 2.0 * u24<double>(b.x) - 1.0;
   const double uperp = sqrt(1.0 - uz * uz);
-  const double uphi = 2.0 * M_PI * u24<double>(b.y);
-  const double ux = uperp * cos(uphi), uy = uperp * sin(uphi);
+  double sphi, cphi;
+  sincos2pi(u24<double>(b.y), sphi, cphi);
+  const double ux = uperp * cphi, uy = uperp * sphi;
   const D3 Vx{vx, {1.0, 0.0, 0.0}}, Vy{vy, {0.0, 1.0, 0.0}}, Vz{vz, {0.0, 0.0, 1.0}};
   const double mi = pc.mi, mn = pc.mn, M = mn + mi;
   const D3 vrx = Vx - dconst(vnx), vry = Vy - dconst(vny), vrz = Vz - dconst(vnz);
@@ -100,9 +101,9 @@ __device__ __forceinline__ void weights_and_slopes(const Grid &g, double x, doub
                                                    double W[8], double Wx[8], double Wy[8], double Wz[8])
 {
   double fx, fy, fz;
-  cell_coord(x, g.p0[0], g.d[0], g.nx, i, fx);
-  cell_coord(y, g.p0[1], g.d[1], g.ny, j, fy);
-  cell_coord(z, g.p0[2], g.d[2], g.nz, k, fz);
+  cell_coord(x, g.p0[0], g.d[0], g.rd[0], g.nx, i, fx);
+  cell_coord(y, g.p0[1], g.d[1], g.rd[1], g.ny, j, fy);
+  cell_coord(z, g.p0[2], g.d[2], g.rd[2], g.nz, k, fz);
   const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy}, wz[2] = {1.0 - fz, fz};
   const double sx[2] = {-1.0 / g.d[0], 1.0 / g.d[0]}, sy[2] = {-1.0 / g.d[1], 1.0 / g.d[1]};
   const double sz[2] = {-1.0 / g.d[2], 1.0 / g.d[2]};

@@ -559,7 +559,7 @@ int chy_create(const chy_params *prm_in, int64_t np_capacity, chy_ctx **out)
   g.mx = fastdiv_magic((uint32_t)g.nx);
   g.my = fastdiv_magic((uint32_t)g.ny);
   g.nc = p.N[0] * p.N[1] * p.N[2];
-  for (int a = 0; a < 3; a++) { g.p0[a] = p.p0[a]; g.p1[a] = p.p1[a]; g.d[a] = p.d[a]; g.L[a] = p.L[a]; }
+  for (int a = 0; a < 3; a++) { g.p0[a] = p.p0[a]; g.p1[a] = p.p1[a]; g.d[a] = p.d[a]; g.rd[a] = 1.0 / p.d[a]; g.L[a] = p.L[a]; }
   // node counts index 32-bit; row launches put ny and nz on the y and z grid axes
   if (g.nc >= (int64_t)1 << 31 || g.ny > 65535 || g.nz > 65535) { delete ctx; return CHY_ERR_ARG_RANGE; }
   ctx->cap = np_capacity > 0 ? np_capacity : std::max<int64_t>(p.Np, 1);

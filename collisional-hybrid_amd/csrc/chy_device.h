@@ -14,6 +14,7 @@ struct Grid {
   int nx, ny, nz;
   int64_t nc;
   double p0[3], p1[3], d[3], L[3];
+  double rd[3];  // 1 / d, rounded to nearest (div_rn)
   // ceil(2^64 / nx) and ceil(2^64 / ny): q = mulhi64(m, c) is c / n exactly for
   // every 32-bit c and n >= 2 (Lemire, Kaser and Kurz, "Faster remainder by
   // direct computation", 2019)
@@ -83,11 +84,124 @@ __device__ __forceinline__ T u24(uint32_t w) { return ((T)(w >> 8) + (T)0.5) * (
 // RNG streams: counter = {id, step, stream, block}, key = seed.
 enum : uint32_t { STREAM_INIT = 0, STREAM_COLLIDE_A = 1, STREAM_COLLIDE_B = 2, STREAM_WEIGHT = 3 };
 
+// ---- FP64 arithmetic of the ions ------------------------------------------------
+// The FP64 ion kernels are bound by instruction issue: the push of an ion
+// issued 2154 vector instructions, most of them in the library's division,
+// square root, logarithm, sine and cosine, which take any argument.  These take
+// the arguments that occur.
+
+// a / d rounded to nearest, rd = 1 / d rounded to nearest: a quotient within an
+// ulp corrected by its exact remainder (Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990); 5 instructions
+// against 12.  Finite operands, no over- or underflow.
+__host__ __device__ __forceinline__ double div_rn(double a, double d, double rd)
+{
+  double q = a * rd;
+  q = __builtin_fma(__builtin_fma(-q, d, a), rd, q);
+  return __builtin_fma(__builtin_fma(-q, d, a), rd, q);
+}
+
+// a / b for normal b whose quotient neither over- nor underflows: the hardware's
+// reciprocal refined twice, then one exact remainder (the last bit may differ
+// from a / b's where that is a near tie)
+__device__ __forceinline__ double div_normal(double a, double b)
+{
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-q, b, a), y, q);
+}
+
+// sin and cos of 2 pi u for 0 <= u <= 1: 4 u = k + f, |f| <= 1/2, exactly, and
+// the Taylor series of sin and cos(pi f / 2) (remainders below 1e-16 of the
+// values); one call of about 35 instructions for both, against 80 for each of
+// the library's.  Unlike cos(2 pi u) it does not round 2 pi u first.
+__host__ __device__ __forceinline__ void sincos2pi(double u, double &s, double &c)
+{
+  const double t = 4.0 * u, k = __builtin_rint(t), f = t - k, z = f * f;
+  double a = -6.688035109811468e-10;
+  a = __builtin_fma(a, z, 5.692172921967927e-08);
+  a = __builtin_fma(a, z, -3.598843235212085e-06);
+  a = __builtin_fma(a, z, 0.00016044118478735983);
+  a = __builtin_fma(a, z, -0.004681754135318688);
+  a = __builtin_fma(a, z, 0.07969262624616705);
+  a = __builtin_fma(a, z, -0.6459640975062463);
+  a = __builtin_fma(a * z, f, 1.5707963267948966 * f);
+  double b = 6.565963114979473e-11;
+  b = __builtin_fma(b, z, -6.386603083791852e-09);
+  b = __builtin_fma(b, z, 4.710874778818172e-07);
+  b = __builtin_fma(b, z, -2.5202042373060607e-05);
+  b = __builtin_fma(b, z, 0.0009192602748394266);
+  b = __builtin_fma(b, z, -0.02086348076335296);
+  b = __builtin_fma(b, z, 0.25366950790104803);
+  b = __builtin_fma(b, z, -1.2337005501361697);
+  b = __builtin_fma(b, z, 1.0);
+  const int q = (int)k;
+  const double sn = (q & 1) ? b : a, cn = (q & 1) ? a : b;
+  s = (q & 2) ? -sn : sn;
+  c = ((q + 1) & 2) ? -cn : cn;
+}
+
+// log(u) for normal u in (0, 1): u = 2^e m, m in [1/sqrt 2, sqrt 2), f = m - 1,
+// s = f / (2 + f), log m = f - (f^2/2 - s (f^2/2 + R)), R the atanh series
+// 2/3 s^2 + 2/5 s^4 + ... (to s^18: below 3e-17 of the logarithm), log 2 in two
+// parts of which the first has few enough bits for e.
+__host__ __device__ __forceinline__ double log_unit(double u)
+{
+  int e;
+#if defined(__HIP_DEVICE_COMPILE__)
+  double m = __builtin_amdgcn_frexp_mant(u);
+  e = __builtin_amdgcn_frexp_exp(u);
+#else
+  double m = __builtin_frexp(u, &e);
+#endif
+  if (m < 0.70710678118654752440) { m *= 2.0; e -= 1; }
+  const double f = m - 1.0, d = 2.0 + f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(d);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+#else
+  const double y = 1.0 / d;
+#endif
+  double s = f * y;
+  s = __builtin_fma(__builtin_fma(-d, s, f), y, s);
+  const double z = s * s;
+  double R = 2.0 / 19.0;
+  R = __builtin_fma(R, z, 2.0 / 17.0);
+  R = __builtin_fma(R, z, 2.0 / 15.0);
+  R = __builtin_fma(R, z, 2.0 / 13.0);
+  R = __builtin_fma(R, z, 2.0 / 11.0);
+  R = __builtin_fma(R, z, 2.0 / 9.0);
+  R = __builtin_fma(R, z, 2.0 / 7.0);
+  R = __builtin_fma(R, z, 2.0 / 5.0);
+  R = __builtin_fma(R, z, 2.0 / 3.0);
+  R = R * z;
+  const double h = 0.5 * f * f, ed = (double)e;
+  return __builtin_fma(ed, 0.6931467056274414, -((h - __builtin_fma(s, h + R, ed * 4.7493250390316726e-07)) - f));
+}
+
+// sqrt(x) for normal positive x (zero for x = 0): the hardware's reciprocal
+// square root refined as the library does (two residuals from the exact x -
+// g^2), without its scaling for the ends of the exponent range.
+__device__ __forceinline__ double sqrt_normal(double x)
+{
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return x > 0.0 ? g : 0.0;
+}
+
 // ---- periodic cells ----------------------------------------------------------
 // Cell of an absolute coordinate, clamped to [0, n-1]; f = fraction in cell.
-__device__ __forceinline__ void cell_coord(double x, double p0, double d, int n, int &i, double &f)
+__device__ __forceinline__ void cell_coord(double x, double p0, double d, double rd, int n, int &i, double &f)
 {
-  const double xi = (x - p0) / d;
+  const double xi = div_rn(x - p0, d, rd);
   int ii = (int)xi;
   if (ii > n - 1) ii = n - 1;
   if (ii < 0) ii = 0;

@@ -198,7 +198,7 @@ int mg_setup(chy_ctx *ctx)
     L.d[0] = p.d[0] * (double)(p.N[0] / g.nx);
     L.d[1] = p.d[1] * (double)(p.N[1] / g.ny);
     L.d[2] = p.d[2];
-    for (int a = 0; a < 3; a++) g.d[a] = L.d[a];
+    for (int a = 0; a < 3; a++) { g.d[a] = L.d[a]; g.rd[a] = 1.0 / L.d[a]; }
     const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
     unsigned char *q = nullptr;
     TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.r = q;

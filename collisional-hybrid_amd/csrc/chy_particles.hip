@@ -168,41 +168,92 @@ __device__ __forceinline__ void flush_scatter_counts(unsigned long long *cs, uin
 // collide, the scattering, which runs in place: every ion's new state is
 // written by the same store instructions as its neighbours' (no scattered
 // write-back of the colliders).
-// At least 3 waves per SIMD: 168 registers (a few spills) against 178 at 2.
+// The FP64 push was bound by the latency of one ion after another: a later
+// load's arrival waits for the stores before it, so each ion paid for its
+// stores, its loads and its corners in turn, and 61 % of the waves' time went
+// into waiting at a few hundred GB/s.  With the next ion's loads issued before
+// this one's stores, its arguments reloaded instead of spilled and arithmetic
+// for the arguments that occur (chy_device.h: 2154 -> 1164 vector instructions
+// in all) it went from 11.43 to 8.63 ms on 268 M ions and from 3.20 to 2.24 on
+// 67 M, of which the instructions make up about two thirds.  (The arithmetic
+// alone gained 4 %; four waves per SIMD instead of three cost spills.)
+// The kernel's (only) argument in its constant segment, by a pointer of which
+// the compiler cannot tell that its target's values were already loaded.
+template <typename T>
+__device__ __forceinline__ const T *reload_args()
+{
+  auto p = __builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return (const T *)p;
+}
+
+struct PushArgs {
+  Grid g;
+  PushConst pc;
+  int64_t np;
+  PState<double> st;
+  const Vec4<double> *E4;
+  const double *Sdev;
+  uint32_t *counts;
+  unsigned long long *cstats;
+  double *bpart;
+  uint8_t *dir;
+};
+
 template <bool COLLIDE, bool MOVE>
-__global__ __launch_bounds__(256, 3) void k_push_fp64(Grid g, PushConst pc, int64_t np, PState<double> st,
-                                                   const Vec4<double> *__restrict__ E4, const double *__restrict__ Sdev,
-                                                   uint32_t *__restrict__ counts, unsigned long long *__restrict__ cstats,
-                                                   double *__restrict__ bpart, uint8_t *__restrict__ dir)
+__global__ __launch_bounds__(256, 3) void k_push_fp64(PushArgs args)
 {
   __shared__ unsigned int sacc[2];
   __shared__ double smom[8];
   double pm = 0.0, pv = 0.0;  // sums of the collision probabilities p and of p (1 - p)
   if (threadIdx.x < 2) sacc[threadIdx.x] = 0u;
   __syncthreads();
-  const double S = COLLIDE ? Sdev[0] : 0.0;
+  const int64_t np = args.np;
+  unsigned long long *const cstats = args.cstats;
+  const double S = COLLIDE ? args.Sdev[0] : 0.0;
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   // every lane iterates the same number of times so wave-level collectives stay convergent
   const int64_t iters = (np + stride - 1) / stride;
   uint32_t nacc = 0, nref = 0;
+  struct Ion { double x, y, z, vx, vy, vz; uint32_t pid; };
+  auto load = [&](const PState<double> &st, int64_t q) {
+    q = q < np ? q : np > 0 ? np - 1 : 0;  // (past the end: any ion, not used)
+    Ion a{st.x[q], st.y[q], st.z[q], st.vx[q], st.vy[q], st.vz[q], 0u};
+    if (COLLIDE) a.pid = st.pid[q];
+    return a;
+  };
+  const int64_t p0 = xcd_block() * blockDim.x + threadIdx.x;
+  Ion next = load(args.st, p0);
   for (int64_t it = 0; it < iters; it++) {
-    const int64_t p = it * stride + xcd_block() * blockDim.x + threadIdx.x;
+    // the arguments read anew for each ion (the scalar cache holds them): kept
+    // across the loop they do not fit the scalar registers and are spilled to
+    // and from vector lanes, 270 instructions an ion
+    const PushArgs &A = *reload_args<PushArgs>();
+    const Grid &g = A.g;
+    const PushConst &pc = A.pc;
+    const PState<double> &st = A.st;
+    uint8_t *const dir = A.dir;
+    const int64_t p = it * stride + p0;
+    const Ion ion = next;
     const bool live = p < np;
     int key = -1, capped = 0;
     bool bad = false;
+    double x = ion.x, y = ion.y, z = ion.z, vx = ion.vx, vy = ion.vy, vz = ion.vz;
+    int i, j, k;
+    double fx, fy, fz, e0, e1, e2;
+    cell_coord(x, g.p0[0], g.d[0], g.rd[0], g.nx, i, fx);
+    cell_coord(y, g.p0[1], g.d[1], g.rd[1], g.ny, j, fy);
+    cell_coord(z, g.p0[2], g.d[2], g.rd[2], g.nz, k, fz);
+    gather_c<double>(g, A.E4, (int64_t)i + (int64_t)g.nx * ((int64_t)j + (int64_t)g.ny * k), i, j, k, fx, fy, fz, e0,
+                     e1, e2);
+    // the thread's next ion is on its way while this one is pushed, and ahead of
+    // this one's stores, which a later load's arrival would wait for
+    next = load(st, p + stride);
+    __builtin_amdgcn_sched_barrier(0);
     if (live) {
-      double x = st.x[p], y = st.y[p], z = st.z[p];
-      double vx = st.vx[p], vy = st.vy[p], vz = st.vz[p];
-      int i, j, k;
-      double fx, fy, fz, e0, e1, e2;
-      cell_coord(x, g.p0[0], g.d[0], g.nx, i, fx);
-      cell_coord(y, g.p0[1], g.d[1], g.ny, j, fy);
-      cell_coord(z, g.p0[2], g.d[2], g.nz, k, fz);
-      gather_c<double>(g, E4, (int64_t)i + (int64_t)g.nx * ((int64_t)j + (int64_t)g.ny * k), i, j, k, fx, fy, fz, e0,
-                       e1, e2);
       boris<double>(pc, e0, e1, e2, vx, vy, vz);
       if (COLLIDE) {
-        const uint32_t pid = st.pid[p];
+        const uint32_t pid = ion.pid;
         double vnx, vny, vnz, ud;
         neutral_draw<double>(pc, pid, vnx, vny, vnz, ud);
         const double pr = collide_prob_n<double>(pc, S, vnx, vny, vnz, vx, vy, vz, capped);
@@ -228,7 +279,7 @@ __global__ __launch_bounds__(256, 3) void k_push_fp64(Grid g, PushConst pc, int6
       }
       bad = !isfinite(vx) || !isfinite(vy) || !isfinite(vz) || !isfinite(x) || !isfinite(y) || !isfinite(z);
     }
-    if (MOVE && counts) count_key(counts, key);
+    if (MOVE && A.counts) count_key(A.counts, key);
     if (COLLIDE) count_flags(cstats, 2, capped != 0);
     count_flags(cstats, 3, bad);
   }
@@ -386,9 +437,9 @@ __global__ __launch_bounds__(256) void k_keys_fp64(Grid g, int64_t np, PState<do
     if (p < np) {
       int i, j, k;
       double f;
-      cell_coord(st.x[p], g.p0[0], g.d[0], g.nx, i, f);
-      cell_coord(st.y[p], g.p0[1], g.d[1], g.ny, j, f);
-      cell_coord(st.z[p], g.p0[2], g.d[2], g.nz, k, f);
+      cell_coord(st.x[p], g.p0[0], g.d[0], g.rd[0], g.nx, i, f);
+      cell_coord(st.y[p], g.p0[1], g.d[1], g.rd[1], g.ny, j, f);
+      cell_coord(st.z[p], g.p0[2], g.d[2], g.rd[2], g.nz, k, f);
       key = (int)(i + (int64_t)g.nx * (j + (int64_t)g.ny * k));
       st.cell[p] = key;
     }
@@ -935,9 +986,9 @@ __global__ __launch_bounds__(256) void k_cell_partials(Grid g, const uint32_t *_
             if (ABS) {
               int i;
               double f;
-              cell_coord((double)x[u], g.p0[0], g.d[0], g.nx, i, f); r.fx = (T)f;
-              cell_coord((double)y[u], g.p0[1], g.d[1], g.ny, i, f); r.fy = (T)f;
-              cell_coord((double)z[u], g.p0[2], g.d[2], g.nz, i, f); r.fz = (T)f;
+              cell_coord((double)x[u], g.p0[0], g.d[0], g.rd[0], g.nx, i, f); r.fx = (T)f;
+              cell_coord((double)y[u], g.p0[1], g.d[1], g.rd[1], g.ny, i, f); r.fy = (T)f;
+              cell_coord((double)z[u], g.p0[2], g.d[2], g.rd[2], g.nz, i, f); r.fz = (T)f;
             } else {
               r.fx = x[u]; r.fy = y[u]; r.fz = z[u];
             }
@@ -1187,9 +1238,9 @@ __global__ __launch_bounds__(256) void k_init_density(Grid g, int kind, int64_t 
   // cell of the position (the clamped truncation of cell_coord)
   int ci[3];
   double fr[3];
-  cell_coord(q[0], g.p0[0], g.d[0], g.nx, ci[0], fr[0]);
-  cell_coord(q[1], g.p0[1], g.d[1], g.ny, ci[1], fr[1]);
-  cell_coord(q[2], g.p0[2], g.d[2], g.nz, ci[2], fr[2]);
+  cell_coord(q[0], g.p0[0], g.d[0], g.rd[0], g.nx, ci[0], fr[0]);
+  cell_coord(q[1], g.p0[1], g.d[1], g.rd[1], g.ny, ci[1], fr[1]);
+  cell_coord(q[2], g.p0[2], g.d[2], g.rd[2], g.nz, ci[2], fr[2]);
   const int64_t c = ci[0] + (int64_t)g.nx * (ci[1] + (int64_t)g.ny * ci[2]);
   double wgt = 1.0;
   if (pert == CHY_PERT_SINUSOIDAL_X) {
@@ -1701,13 +1752,14 @@ int particles_push(chy_ctx *ctx, bool move, bool collide, chy_collision_stats *s
     else LAUNCH(k_push_mixed, float, false, false, dir);
     if (move) ctx->dir_valid = dir != nullptr;
   } else {
-    const PushConst &pcT = pc;
     PState<double> st = ctx->pd[ctx->cur];
     uint8_t *dir = move && ctx->order_valid && !ctx->keys_moved ? ctx->dir : nullptr;
-    if (collide && move) LAUNCH(k_push_fp64, double, true, true, dir);
-    else if (collide) LAUNCH(k_push_fp64, double, true, false, dir);
-    else if (move) LAUNCH(k_push_fp64, double, false, true, dir);
-    else LAUNCH(k_push_fp64, double, false, false, dir);
+    const PushArgs args{ctx->g, pc, ctx->np, st, (const Vec4<double> *)ctx->efield[0], ctx->S_dev,
+                        count ? ctx->counts : nullptr, ctx->cstats, ctx->push_part, dir};
+    if (collide && move) hipLaunchKernelGGL((k_push_fp64<true, true>), nb, kBlock, 0, ctx->stream, args);
+    else if (collide) hipLaunchKernelGGL((k_push_fp64<true, false>), nb, kBlock, 0, ctx->stream, args);
+    else if (move) hipLaunchKernelGGL((k_push_fp64<false, true>), nb, kBlock, 0, ctx->stream, args);
+    else hipLaunchKernelGGL((k_push_fp64<false, false>), nb, kBlock, 0, ctx->stream, args);
     if (move) ctx->dir_valid = dir != nullptr;
   }
 #undef LAUNCH

@@ -75,19 +75,23 @@ inline int64_t collision_count(const chy_params &p, int64_t Np)
 }
 
 // Arithmetic of the collision kinematics.  FP64 (the reference's
-// arithmetic): IEEE square root, division, sine and cosine.  FP32 (the mixed
+// arithmetic): square root, division, sine and cosine to double rounding.  FP32 (the mixed
 // path): the hardware square root, reciprocal and sine/cosine, each within a
 // few ulp -- the neutral draw and the scattering are Monte Carlo samples whose
 // FP32 rounding is far below their sampling noise -- with the square root
 // clamped at zero against rounding that pushes 1 - cos^2 below it.
-template <typename T> __device__ __forceinline__ T kin_sqrt(T x) { return sqrt(x); }
+template <typename T> __device__ __forceinline__ T kin_sqrt(T x) { return sqrt_normal(x); }
 template <> __device__ __forceinline__ float kin_sqrt<float>(float x) { return __builtin_amdgcn_sqrtf(fmaxf(x, 0.0f)); }
-template <typename T> __device__ __forceinline__ T kin_div(T a, T b) { return a / b; }
+template <typename T> __device__ __forceinline__ T kin_div(T a, T b) { return div_normal(a, b); }
 template <> __device__ __forceinline__ float kin_div<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-template <typename T> __device__ __forceinline__ T kin_cos(T a) { return cos(a); }
-template <> __device__ __forceinline__ float kin_cos<float>(float a) { return __cosf(a); }
-template <typename T> __device__ __forceinline__ T kin_sin(T a) { return sin(a); }
-template <> __device__ __forceinline__ float kin_sin<float>(float a) { return __sinf(a); }
+// sine and cosine of 2 pi u, 0 <= u <= 1
+__device__ __forceinline__ void kin_sincos2pi(double u, double &s, double &c) { sincos2pi(u, s, c); }
+__device__ __forceinline__ void kin_sincos2pi(float u, float &s, float &c)
+{
+  const float a = (float)(2.0 * M_PI) * u;
+  s = __sinf(a);
+  c = __cosf(a);
+}
 
 // ---- ion-neutral collisions (reference particles.c:529-611) ---------------------
 // Neutral draw and Bernoulli decision from one Philox block: Box-Muller on the
@@ -107,10 +111,13 @@ __device__ __forceinline__ void neutral_draw(const PC &pc, uint32_t pid, T &vnx,
     const float a1 = 6.28318530717958647692f * (float)u1, a2 = 6.28318530717958647692f * (float)u3;
     c1 = __cosf(a1); s1 = __sinf(a1); c2 = __cosf(a2);
   } else {
-    r1 = sqrt(-2.0 * log((double)u0));
-    r2 = sqrt(-2.0 * log((double)u2));
-    const double a1 = 2.0 * M_PI * (double)u1, a2 = 2.0 * M_PI * (double)u3;
-    c1 = cos(a1); s1 = sin(a1); c2 = cos(a2);
+    r1 = sqrt_normal(-2.0 * log_unit((double)u0));
+    r2 = sqrt_normal(-2.0 * log_unit((double)u2));
+    double s2, cc, ss;
+    sincos2pi((double)u1, ss, cc);
+    c1 = cc; s1 = ss;
+    sincos2pi((double)u3, s2, cc);
+    c2 = cc;
   }
   const T vnT = (T)pc.vnT;
   vnx = (T)pc.vn0[0] + vnT * (r1 * c1);
@@ -171,7 +178,6 @@ __device__ __forceinline__ int scatter_n(const PC &pc, uint32_t pid, T vnx, T vn
   const T vrx = vx - vnx, vry = vy - vny, vrz = vz - vnz;
   const T vrr = kin_sqrt<T>(vrx * vrx + vry * vry + vrz * vrz);
   const U4 b = philox4x32_10(U4{pid, pc.step, STREAM_COLLIDE_B, 0u}, pc.k0, pc.k1);
-  const T twopi = (T)(2.0 * M_PI);
   const T mi = (T)pc.mi, mn = (T)pc.mn, M = mn + mi;
   const T vcx = kin_div<T>(vx * mi + vnx * mn, M);
   const T vcy = kin_div<T>(vy * mi + vny * mn, M);
@@ -180,8 +186,9 @@ __device__ __forceinline__ int scatter_n(const PC &pc, uint32_t pid, T vnx, T vn
   const T vcr = kin_sqrt<T>(ex * ex + ey * ey + ez * ez);
   const T uz = (T)2.0 * u24<T>(b.x) - (T)1.0;
   const T uperp = kin_sqrt<T>((T)1.0 - uz * uz);
-  const T uphi = twopi * u24<T>(b.y);
-  const T ux = uperp * kin_cos<T>(uphi), uy = uperp * kin_sin<T>(uphi);
+  T sphi, cphi;
+  kin_sincos2pi(u24<T>(b.y), sphi, cphi);
+  const T ux = uperp * cphi, uy = uperp * sphi;
   const T costht = kin_div<T>(vrz, vrr);
   const T sintht = kin_sqrt<T>((T)1.0 - costht * costht);
   T cosphi = (T)1, sinphi = (T)0;
@@ -306,9 +313,9 @@ __device__ __forceinline__ int move_fp64(const Grid &g, double dt, double &x, do
   z = wrap_pos(z + vz * dt, g.p0[2], g.p1[2], g.L[2]);
   int i, j, k;
   double f;
-  cell_coord(x, g.p0[0], g.d[0], g.nx, i, f);
-  cell_coord(y, g.p0[1], g.d[1], g.ny, j, f);
-  cell_coord(z, g.p0[2], g.d[2], g.nz, k, f);
+  cell_coord(x, g.p0[0], g.d[0], g.rd[0], g.nx, i, f);
+  cell_coord(y, g.p0[1], g.d[1], g.rd[1], g.ny, j, f);
+  cell_coord(z, g.p0[2], g.d[2], g.rd[2], g.nz, k, f);
   return (int)(i + (int64_t)g.nx * (j + (int64_t)g.ny * k));
 }
 

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(256) void k_ions_in_mixed(Grid g, int64_t n, int64_
 #pragma unroll
   for (int a = 0; a < 3; a++) {
     double f;
-    cell_coord(wrap_pos(x[a], g.p0[a], g.p1[a], g.L[a]), g.p0[a], g.d[a], nn[a], ci[a], f);
+    cell_coord(wrap_pos(x[a], g.p0[a], g.p1[a], g.L[a]), g.p0[a], g.d[a], g.rd[a], nn[a], ci[a], f);
     o[a] = (float)f;
     if (o[a] >= 1.0f) { o[a] = 0.0f; ci[a] = ci[a] + 1 == nn[a] ? 0 : ci[a] + 1; }
   }

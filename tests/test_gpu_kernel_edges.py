@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import orc
-from gpu_cases import context, grid_of, opts, random_particles, upload, vlasov_from
+from gpu_cases import (as_particles, context, grid_of, opts, push_params_of, random_particles, relmax, upload,
+                       vlasov_from)
 
 pytestmark = pytest.mark.gpu
 
@@ -148,3 +149,29 @@ def test_grid_arrays_survive_the_host_round_trip(N, prec):
         ctx.set_potential(phi)
         assert np.array_equal(ctx.get_moments(), v if prec == "fp64" else v.astype(np.float32).astype(np.float64))
         assert np.array_equal(ctx.get_potential(), phi)
+
+
+# the FP64 push carries its next ion along: no ion, one, a wave and its
+# neighbours, a block, and more ions than one trip of the largest grid; every
+# wave with and without colliders (nu_in 1e3 and 1e5 s^-1)
+@pytest.mark.parametrize("nui", [1e3, 1e5])
+@pytest.mark.parametrize("N,n", [((3, 3, 3), 1), ((5, 4, 3), 63), ((5, 4, 3), 65), ((4, 4, 4), 256), ((7, 5, 6), 1023),
+                                 ((20, 20, 20), 40000)])
+def test_fp64_push_of_any_number_of_ions(N, n, nui):
+    rng = np.random.default_rng(17)
+    with context(opts(N, extra=f"-nui {nui} -seed 5 --collision-refusal-limit 0 -Np {n}"), capacity=n) as ctx:
+        g = grid_of(ctx.prm)
+        upload(ctx, random_particles(g, n, rng))
+        phi = 0.01 * rng.standard_normal(g.nc)
+        ctx.set_potential(phi)
+        before = as_particles(ctx.get_particles())
+        S = orc.normaliser(before, list(ctx.prm.vn0), ctx.prm.vnT)
+        _, P = push_params_of(ctx.prm, step=0)
+        st = ctx.update_velocities()
+        ctx.update_positions()
+        after = as_particles(ctx.get_particles())
+    nxt, key, _, _, stats = orc.step(g, P, before, phi, S, list(ctx.prm.E0))
+    assert np.array_equal(after.pid, nxt.pid)
+    assert (st.accepted, st.refused) == (stats[0], stats[1])
+    for a in ("x", "y", "z", "vx", "vy", "vz"):
+        assert relmax(getattr(after, a), getattr(nxt, a)) <= 1e-12
