@@ -11,7 +11,8 @@
 // division and the inverse FFT.  The x pass is real-to-complex (half
 // spectrum, nx/2 complex values per line), so every pass moves as many bytes
 // as the real field: x-fwd, y-fwd, z-fwd/scale/z-inv, y-inv, x-inv.  Grid
-// sizes: powers of two.
+// sizes: powers of two.  Axes of 16 to 512 points (256 in FP64) take
+// register-resident four-step transforms instead.
 #include <algorithm>
 #include <cmath>
 
@@ -418,11 +419,11 @@ __device__ __forceinline__ void fft_col0_body(int p, int logn, int64_t estride, 
   __syncthreads();
   dif_fwd<T>(s, nl, logn, tws);
   // every new value needs its partner's old one: compute into registers, then write
-  constexpr int kPerThread = 2 * kFftMaxN / 256;
+  constexpr int kPerThread = 2 * kFftMaxN / 256;  // (shorter lines in blocks of 128 threads too)
   cpx<T> nv[kPerThread];
 #pragma unroll
   for (int q = 0; q < kPerThread; q++) {
-    const int e = threadIdx.x + 256 * q;
+    const int e = threadIdx.x + blockDim.x * q;
     if (e >= nl * n) break;
     const int b = e >> logn, t = e & (n - 1);
     const int kyb = b == 0 ? ky : (ny - ky) & (ny - 1);
@@ -440,7 +441,7 @@ __device__ __forceinline__ void fft_col0_body(int p, int logn, int64_t estride, 
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < kPerThread; q++) {
-    const int e = threadIdx.x + 256 * q;
+    const int e = threadIdx.x + blockDim.x * q;
     if (e >= nl * n) break;
     s[(e >> logn) * (n + 1) + (e & (n - 1))] = nv[q];
   }
@@ -466,22 +467,34 @@ __global__ __launch_bounds__(256) void k_fft_col0(int logn, int64_t estride, int
   fft_col0_body<T>((int)blockIdx.x, logn, estride, hx, buf, tws, s, sym, trx, try_, trz);
 }
 
-// ---- 256- and 512-point lines: register-resident four-step transforms -----------------
-// A line of N = 16 R points (R = 16: 256, R = 32: 512) is held by 16 threads,
-// thread j owning the elements j + 16 m (m < R) in registers.  Each thread
-// transforms its R values (a length-R DFT in registers over m), multiplies by
-// the twiddles W_N^(j k1), and one transpose through LDS hands thread j the
-// 16 values of rows k1 = j + 16 c (c < R/16), whose 16-point DFTs over j
-// give X[k1 + R k2].  That is element j + 16 (c + (R/16) k2): input and output
-// use the same register pattern in natural order, so forward and inverse
-// compose without permutations, and LDS carries each value twice per
-// transform.  The LDS strides (values split into real and imaginary arrays)
-// make the 64 lanes of a wave touch 64 distinct banks in both layouts.
-constexpr int kQSk = 17;  // LDS stride between the k1 rows of a line
-// line strides: strided passes (lanes: 16 lines x 4 threads), x pass (lanes:
-// 16 threads x 4 line pairs); 4 and 16 modulo 64 respectively
-template <int R> constexpr int q_sbs() { return R == 16 ? 324 : 580; }
-template <int R> constexpr int q_sbx() { return R == 16 ? 272 : 592; }
+// ---- lines of 16 to 512 points: register-resident four-step transforms --------------
+// A line of N = TH R points (TH <= R: 4x4, 4x8, 8x8, 8x16, 16x16 and 16x32) is
+// held by TH threads, thread j owning the elements j + TH m (m < R) in
+// registers.  Each thread transforms its R values (a length-R DFT in registers
+// over m), multiplies by the twiddles W_N^(j k1), and one transpose through LDS
+// hands thread j the TH values of rows k1 = j + TH c (c < R/TH), whose TH-point
+// DFTs over j give X[k1 + R k2].  That is element j + TH (c + (R/TH) k2): input
+// and output use the same register pattern in natural order, so forward and
+// inverse compose without permutations, and LDS carries each value twice per
+// transform, where the radix-4 passes carry it once a stage with a barrier
+// each.  Short lines are bound by that chain of LDS round trips, long ones by
+// the bytes.  Measured against the radix-4 passes, us for x + y + z + y + x of
+// one application with the packed column: FP64 32^3 44.2 -> 20.9, 64^3 71.5 ->
+// 23.6, 128^3 122.6 -> 55.8; FP32 32^3 40.8 -> 19.4, 64^3 60.4 -> 19.8, 128^3
+// 84.8 -> 39.9.
+//
+// LDS strides between the rows of a line (TH + 1) and between the lines of a
+// block, for values split into real and imaginary arrays: with 16 threads a
+// line the 64 lanes of a wave touch 64 distinct banks in both layouts (strided
+// passes: lanes are 16 lines x 4 threads, x pass: 16 threads x 4 line pairs);
+// shorter lines take an odd stride (strided) or an odd multiple of TH (x pass).
+template <int TH, int R> constexpr int q_sbs() { return TH == 16 ? (R == 16 ? 324 : 580) : (R * (TH + 1)) | 1; }
+template <int TH, int R> constexpr int q_sbx()
+{
+  return TH * ((R * (TH + 1) + TH - 1) / TH | 1);
+}
+// threads of a block: 128 where 256 threads' lines would fill half of a CU's LDS
+template <typename T, int TH, int R> constexpr int q_block() { return sizeof(T) == 8 && TH * R == 128 ? 128 : 256; }
 
 template <typename T, bool INV>
 __device__ __forceinline__ void dft4(cpx<T> &a0, cpx<T> &a1, cpx<T> &a2, cpx<T> &a3)
@@ -530,15 +543,39 @@ __device__ __forceinline__ void dft16(cpx<T> (&v)[16])
   for (int q = 0; q < 16; q++) v[q] = o[q];
 }
 
-// In-place R-point DFT (R = 16 or 32), natural order in and out; 32 points
-// as two 16-point DFTs of the even and odd elements and one radix-2 stage.
+// In-place 8-point DFT, natural order in and out: the 4-point DFTs of the even
+// and odd elements and one radix-2 stage.
+template <typename T, bool INV>
+__device__ __forceinline__ void dft8(cpx<T> (&v)[8])
+{
+  constexpr T h = (T)0.70710678118654752;
+  cpx<T> e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1], o1 = v[3], o2 = v[5], o3 = v[7];
+  dft4<T, INV>(e0, e1, e2, e3);
+  dft4<T, INV>(o0, o1, o2, o3);
+  const T sg = INV ? (T)1 : (T)-1;  // W_8^k = cos(2 pi k / 8) -+ i sin(2 pi k / 8)
+  o1 = cmul<T>(o1, {h, sg * h});
+  o2 = {-sg * o2.y, sg * o2.x};
+  o3 = cmul<T>(o3, {-h, sg * h});
+  v[0] = {e0.x + o0.x, e0.y + o0.y}; v[4] = {e0.x - o0.x, e0.y - o0.y};
+  v[1] = {e1.x + o1.x, e1.y + o1.y}; v[5] = {e1.x - o1.x, e1.y - o1.y};
+  v[2] = {e2.x + o2.x, e2.y + o2.y}; v[6] = {e2.x - o2.x, e2.y - o2.y};
+  v[3] = {e3.x + o3.x, e3.y + o3.y}; v[7] = {e3.x - o3.x, e3.y - o3.y};
+}
+
+// In-place R-point DFT (R = 4, 8, 16 or 32), natural order in and out; 32
+// points as two 16-point DFTs of the even and odd elements and one radix-2
+// stage.
 template <typename T, bool INV, int R>
 __device__ __forceinline__ void dftR(cpx<T> (&v)[R])
 {
-  if constexpr (R == 16) {
+  if constexpr (R == 4) {
+    dft4<T, INV>(v[0], v[1], v[2], v[3]);
+  } else if constexpr (R == 8) {
+    dft8<T, INV>(v);
+  } else if constexpr (R == 16) {
     dft16<T, INV>(v);
   } else {
-    static_assert(R == 32, "16- or 32-point register DFTs");
+    static_assert(R == 32, "4- to 32-point register DFTs");
     cpx<T> e[16], o[16];
 #pragma unroll
     for (int q = 0; q < 16; q++) { e[q] = v[2 * q]; o[q] = v[2 * q + 1]; }
@@ -558,12 +595,12 @@ __device__ __forceinline__ void dftR(cpx<T> (&v)[R])
 }
 
 // The four-step transform of the line held by this thread's group (thread j
-// of 16; its LDS rows start at gbase).  tws: W_N^m, m < N/2 (forward).  Every
+// of TH; its LDS rows start at gbase).  tws: W_N^m, m < N/2 (forward).  Every
 // thread of the block calls it (two barriers).
-template <typename T, bool INV, int R>
+template <typename T, bool INV, int TH, int R>
 __device__ __forceinline__ void fft_line(cpx<T> (&v)[R], int j, T *lre, T *lim, int gbase, const cpx<T> *tws)
 {
-  constexpr int N = 16 * R, H = N / 2;
+  constexpr int N = TH * R, H = N / 2, SK = TH + 1;
   dftR<T, INV, R>(v);
 #pragma unroll
   for (int k1 = 1; k1 < R; k1++) {
@@ -575,65 +612,66 @@ __device__ __forceinline__ void fft_line(cpx<T> (&v)[R], int j, T *lre, T *lim, 
   }
 #pragma unroll
   for (int k1 = 0; k1 < R; k1++) {
-    lre[gbase + k1 * kQSk + j] = v[k1].x;
-    lim[gbase + k1 * kQSk + j] = v[k1].y;
+    lre[gbase + k1 * SK + j] = v[k1].x;
+    lim[gbase + k1 * SK + j] = v[k1].y;
   }
   __syncthreads();
 #pragma unroll
-  for (int c = 0; c < R / 16; c++) {
-    cpx<T> u[16];
-    const int row = gbase + (j + 16 * c) * kQSk;
+  for (int c = 0; c < R / TH; c++) {
+    cpx<T> u[TH];
+    const int row = gbase + (j + TH * c) * SK;
 #pragma unroll
-    for (int n2 = 0; n2 < 16; n2++) u[n2] = {lre[row + n2], lim[row + n2]};
-    dft16<T, INV>(u);
+    for (int n2 = 0; n2 < TH; n2++) u[n2] = {lre[row + n2], lim[row + n2]};
+    dftR<T, INV, TH>(u);
 #pragma unroll
-    for (int k2 = 0; k2 < 16; k2++) v[c + (R / 16) * k2] = u[k2];
+    for (int k2 = 0; k2 < TH; k2++) v[c + (R / TH) * k2] = u[k2];
   }
   __syncthreads();
 }
 
-// Strided N-point pass: lines a = a0 .. a0+15 (16 per block) of the set c,
-// line (a, c) at a + c*cstride, element t at + t*estride; thread (b, j) =
-// (threadIdx & 15, threadIdx >> 4).  MODE 0 forward, 1 inverse, 2 forward +
-// symbol division + inverse (z axis, lines a = kx + (nx/2)*py; the packed
-// kx = 0 slot is left to k_fft_col0).
-template <typename T, int MODE, int R>
-__global__ __launch_bounds__(256) void k_fftq_s(int64_t A, int64_t estride, int64_t cstride,
+// Strided N-point pass over `lines` lines: line l = a + A c (A = 2^lA) at a + c
+// cstride, element t at + t estride; a block takes NL consecutive lines, thread
+// (b, j) = (threadIdx % NL, threadIdx / NL).  MODE 0 forward, 1 inverse, 2
+// forward + symbol division + inverse (z axis, lines a = kx + (nx/2)*py; the
+// packed kx = 0 slot is left to fft_col0_body).
+template <typename T, int MODE, int TH, int R>
+__global__ __launch_bounds__((q_block<T, TH, R>())) void k_fftq_s(int64_t lines, int lA, int64_t estride, int64_t cstride,
                                                 cpx<T> *__restrict__ buf, const double *__restrict__ tw, Symbol sym,
                                                 const double *__restrict__ trx, const double *__restrict__ try_,
                                                 const double *__restrict__ trz)
 {
-  constexpr int N = 16 * R, SB = q_sbs<R>();
-  __shared__ T lre[16 * SB], lim[16 * SB];
+  constexpr int N = TH * R, SB = q_sbs<TH, R>(), NL = q_block<T, TH, R>() / TH;
+  // (the packed column's scratch: 2 (N + 1) complex values)
+  constexpr int kLds = 2 * NL * SB > 4 * (N + 1) ? 2 * NL * SB : 4 * (N + 1);
+  __shared__ T lds[kLds];
+  T *lre = lds, *lim = lds + NL * SB;
   __shared__ cpx<T> tws[N / 2];
   load_twiddles<T>(tws, tw, N);
   __syncthreads();
   if constexpr (MODE == 2) {
-    // blocks past the lines take the packed kx = 0 column (k_fft_col0's work,
-    // the z lines the others leave), so it needs no launch of its own; lre is
-    // their scratch
-    static_assert(2 * (N + 1) * 2 <= 16 * SB, "column-0 scratch");
-    const int64_t nmain = A / 16;
+    // blocks past the lines take the packed kx = 0 column (the z lines the
+    // others leave), so it needs no launch of its own
+    const int64_t nmain = (lines + NL - 1) / NL;
     if ((int64_t)blockIdx.x >= nmain) {
-      fft_col0_body<T>((int)(blockIdx.x - nmain), R == 16 ? 8 : 9, estride, sym.nx >> 1, buf, tws,
-                       reinterpret_cast<cpx<T> *>(lre), sym, trx, try_, trz);
+      constexpr int kLog = N == 512 ? 9 : N == 256 ? 8 : N == 128 ? 7 : N == 64 ? 6 : N == 32 ? 5 : 4;
+      fft_col0_body<T>((int)(blockIdx.x - nmain), kLog, estride, sym.nx >> 1, buf, tws, reinterpret_cast<cpx<T> *>(lds),
+                       sym, trx, try_, trz);
       return;
     }
   }
-  const int b = threadIdx.x & 15, j = threadIdx.x >> 4;
-  const int64_t blocks_per_c = A / 16;
-  const int64_t c = blockIdx.x / blocks_per_c, a = (blockIdx.x % blocks_per_c) * 16 + b;
-  const int64_t base = a + c * cstride;
+  const int b = threadIdx.x % NL, j = threadIdx.x / NL;
+  const int64_t l = (int64_t)blockIdx.x * NL + b, a = l & (((int64_t)1 << lA) - 1);
+  const int64_t base = a + (l >> lA) * cstride;
   const int hx = sym.nx >> 1;
-  const bool live = MODE != 2 || (a & (hx - 1)) != 0;
+  const bool live = l < lines && (MODE != 2 || (a & (hx - 1)) != 0);
   cpx<T> v[R];
 #pragma unroll
-  for (int m = 0; m < R; m++) v[m] = live ? buf[base + (int64_t)(j + 16 * m) * estride] : cpx<T>{(T)0, (T)0};
-  fft_line<T, MODE == 1, R>(v, j, lre, lim, b * SB, tws);
+  for (int m = 0; m < R; m++) v[m] = live ? buf[base + (int64_t)(j + TH * m) * estride] : cpx<T>{(T)0, (T)0};
+  fft_line<T, MODE == 1, TH, R>(v, j, lre, lim, b * SB, tws);
   if (MODE == 2) {
-    // symbol along the line: la + lb cos(kz) - lc sin(kz), kz = j + 16 m
+    // symbol along the line: la + lb cos(kz) - lc sin(kz), kz = j + TH m
     const int kx = (int)(a & (hx - 1));
-    const int py = (int)(a >> (sym.lx - 1));
+    const int py = live ? (int)(a >> (sym.lx - 1)) : 0;
     const int ky = sym.ynat ? py : bitrev(py, sym.ly);
     const double cx = trx[2 * kx], sx = trx[2 * kx + 1], cy = try_[2 * ky], sy = try_[2 * ky + 1];
     const double la = sym.A0 + sym.F[0] * cx + sym.F[1] * cy + (sym.P[0] * cx * cy - sym.M[0] * sx * sy);
@@ -641,7 +679,7 @@ __global__ __launch_bounds__(256) void k_fftq_s(int64_t A, int64_t estride, int6
     const double lc = sym.M[1] * sx + sym.M[2] * sy;
 #pragma unroll
     for (int m = 0; m < R; m++) {
-      const int kz = j + 16 * m;
+      const int kz = j + TH * m;
       // lambda in FP64 (it cancels near k = 0); the FP32 pass then takes its
       // reciprocal in FP32, the FP64 pass divides exactly
       const double lam = la + lb * trz[2 * kz] - lc * trz[2 * kz + 1];
@@ -653,32 +691,34 @@ __global__ __launch_bounds__(256) void k_fftq_s(int64_t A, int64_t estride, int6
         v[m] = {(T)((double)v[m].x * f), (T)((double)v[m].y * f)};
       }
     }
-    fft_line<T, true, R>(v, j, lre, lim, b * SB, tws);
+    fft_line<T, true, TH, R>(v, j, lre, lim, b * SB, tws);
   }
   if (live) {
 #pragma unroll
-    for (int m = 0; m < R; m++) buf[base + (int64_t)(j + 16 * m) * estride] = v[m];
+    for (int m = 0; m < R; m++) buf[base + (int64_t)(j + TH * m) * estride] = v[m];
   }
 }
 
-// x pass for nx = N, two real lines per 16-thread group (32 lines per
+// x pass for nx = N, two real lines per group of TH threads (2 NL lines per
 // block): z = x_a + i x_b is transformed once, and X_a = (Z_k + conj Z_-k)/2,
 // X_b = (Z_k - conj Z_-k)/(2i) are written for k < N/2 (slot 0 packs X_0 and
 // X_(N/2) as X_0 + i X_(N/2)), to the same layout as k_rfft_x.  MODE 1 is the
 // exact reverse: Z_k = X_a + i X_b over the Hermitian extension, inverse
-// transform, x_a = Re, x_b = Im (N times the input), times scale.
-template <typename T, int MODE, int R>
-__global__ __launch_bounds__(256) void k_rfftq_x(int64_t nlines, const T *__restrict__ rin,
+// transform, x_a = Re, x_b = Im (N times the input), times scale.  nlines is
+// even (axes have a power of two of nodes, at least 4).
+template <typename T, int MODE, int TH, int R>
+__global__ __launch_bounds__((q_block<T, TH, R>())) void k_rfftq_x(int64_t nlines, const T *__restrict__ rin,
                                                  cpx<T> *__restrict__ buf, T *__restrict__ rout,
                                                  const double *__restrict__ tw, double scale, int ly, int64_t plane)
 {
-  constexpr int N = 16 * R, H = N / 2, SB = q_sbx<R>();
-  __shared__ T lre[16 * SB], lim[16 * SB];
+  constexpr int N = TH * R, H = N / 2, SB = q_sbx<TH, R>(), NL = q_block<T, TH, R>() / TH;
+  static_assert(SB >= R * (TH + 1) && SB >= N, "a line's rows, and its N values in natural order");
+  __shared__ T lre[NL * SB], lim[NL * SB];
   __shared__ cpx<T> tws[H];
   load_twiddles<T>(tws, tw, N);
   __syncthreads();
-  const int j = threadIdx.x & 15, g = threadIdx.x >> 4;
-  const int64_t la = (int64_t)blockIdx.x * 32 + 2 * g, lb = la + 1;
+  const int j = threadIdx.x % TH, g = threadIdx.x / TH;
+  const int64_t la = (int64_t)blockIdx.x * (2 * NL) + 2 * g, lb = la + 1;
   const bool ok = lb < nlines;
   auto at = [&](int64_t l) { return (l & ((1 << ly) - 1)) * (int64_t)H + (l >> ly) * plane; };
   const int gb = g * SB;
@@ -686,20 +726,20 @@ __global__ __launch_bounds__(256) void k_rfftq_x(int64_t nlines, const T *__rest
   if (MODE == 0) {
 #pragma unroll
     for (int m = 0; m < R; m++)
-      v[m] = ok ? cpx<T>{rin[la * N + j + 16 * m], rin[lb * N + j + 16 * m]} : cpx<T>{(T)0, (T)0};
-    fft_line<T, false, R>(v, j, lre, lim, gb, tws);
+      v[m] = ok ? cpx<T>{rin[la * N + j + TH * m], rin[lb * N + j + TH * m]} : cpx<T>{(T)0, (T)0};
+    fft_line<T, false, TH, R>(v, j, lre, lim, gb, tws);
     // Z in natural order in LDS, for the partner values Z_-k
 #pragma unroll
     for (int m = 0; m < R; m++) {
-      lre[gb + j + 16 * m] = v[m].x;
-      lim[gb + j + 16 * m] = v[m].y;
+      lre[gb + j + TH * m] = v[m].x;
+      lim[gb + j + TH * m] = v[m].y;
     }
     __syncthreads();
     if (ok) {
       const int64_t oa = at(la), ob = at(lb);
 #pragma unroll
       for (int m = 0; m < R / 2; m++) {
-        const int k = j + 16 * m;
+        const int k = j + TH * m;
         const T zx = lre[gb + k], zy = lim[gb + k];
         cpx<T> xa, xb;
         if (k == 0) {
@@ -722,14 +762,14 @@ __global__ __launch_bounds__(256) void k_rfftq_x(int64_t nlines, const T *__rest
     T *are = lre + gb, *aim = lim + gb, *bre = are + H, *bim = aim + H;
 #pragma unroll
     for (int m = 0; m < R / 2; m++) {
-      const int t = j + 16 * m;
+      const int t = j + TH * m;
       const cpx<T> A = ok ? buf[oa + t] : cpx<T>{(T)0, (T)0}, B = ok ? buf[ob + t] : cpx<T>{(T)0, (T)0};
       are[t] = A.x; aim[t] = A.y; bre[t] = B.x; bim[t] = B.y;
     }
     __syncthreads();
 #pragma unroll
     for (int m = 0; m < R; m++) {
-      const int t = j + 16 * m;
+      const int t = j + TH * m;
       cpx<T> z;
       if (t == 0) z = {are[0], bre[0]};
       else if (t == H) z = {aim[0], bim[0]};
@@ -738,12 +778,12 @@ __global__ __launch_bounds__(256) void k_rfftq_x(int64_t nlines, const T *__rest
       v[m] = z;
     }
     __syncthreads();
-    fft_line<T, true, R>(v, j, lre, lim, gb, tws);
+    fft_line<T, true, TH, R>(v, j, lre, lim, gb, tws);
     if (ok) {
 #pragma unroll
       for (int m = 0; m < R; m++) {
-        rout[la * N + j + 16 * m] = (T)((double)v[m].x * scale);
-        rout[lb * N + j + 16 * m] = (T)((double)v[m].y * scale);
+        rout[la * N + j + TH * m] = (T)((double)v[m].x * scale);
+        rout[lb * N + j + TH * m] = (T)((double)v[m].y * scale);
       }
     }
   }
@@ -751,10 +791,21 @@ __global__ __launch_bounds__(256) void k_rfftq_x(int64_t nlines, const T *__rest
 
 static bool pow2(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
 
-// Register radix R of the four-step kernels for an axis of n points: 16 for
-// 256, 32 for 512 in FP32 (the FP64 512-point tiles would not fit LDS twice
-// per CU); 0: the radix-4 LDS passes.
-template <typename T> static int q_radix(int n) { return n == 256 ? 16 : (n == 512 && sizeof(T) == 4 ? 32 : 0); }
+// Axis lengths of the four-step kernels: 16 to 512 points (512 in FP32 only:
+// the FP64 tiles would not fit LDS twice per CU); the others take the radix-4
+// LDS passes.
+template <typename T> static bool q_axis(int n) { return pow2(n) && n >= 16 && n <= (sizeof(T) == 4 ? 512 : 256); }
+
+// call with the axis' TH and R, and NL = the lines (x pass: line pairs) of a block
+#define Q_AXIS(T, n, call)                                                                              \
+  do {                                                                                                  \
+    if (n == 16) { constexpr int TH = 4, R = 4, NL = q_block<T, TH, R>() / TH; call; }                  \
+    else if (n == 32) { constexpr int TH = 4, R = 8, NL = q_block<T, TH, R>() / TH; call; }             \
+    else if (n == 64) { constexpr int TH = 8, R = 8, NL = q_block<T, TH, R>() / TH; call; }             \
+    else if (n == 128) { constexpr int TH = 8, R = 16, NL = q_block<T, TH, R>() / TH; call; }           \
+    else if (n == 256) { constexpr int TH = 16, R = 16, NL = q_block<T, TH, R>() / TH; call; }          \
+    else if constexpr (sizeof(T) == 4) { constexpr int TH = 16, R = 32, NL = q_block<T, TH, R>() / TH; call; } \
+  } while (0)
 
 // Complex elements between z planes of the half spectrum: (nx/2) ny plus
 // 256 bytes
@@ -813,32 +864,18 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
   // z planes of the half spectrum are spaced P = (nx/2) ny + padding apart, so
   // that the rows of a z line do not all fall at one power-of-two stride
   const int64_t P = spec_plane<T>(nx, ny);
-  // 256-point axes (and 512-point ones in FP32) use the four-step kernels
-  // (16 lines per block); their y pass leaves the y frequencies in natural
-  // order.  xq, yq, zq: the register radix R of each axis (0: radix-4 passes)
-  const int xq = q_radix<T>(nx), yq = hx % 16 == 0 ? q_radix<T>(ny) : 0,
-            zq = ((int64_t)hx * ny) % 16 == 0 ? q_radix<T>(nz) : 0;
+  // the four-step kernels' y pass leaves the y frequencies in natural order
+  const bool xq = q_axis<T>(nx), yq = q_axis<T>(ny), zq = q_axis<T>(nz);
   sym.ynat = yq ? 1 : 0;
   const int nlines = ny * nz;
-  const unsigned nxb = (unsigned)((nlines + 31) / 32), nyb = (unsigned)((hx / 16) * nz);
+  const int lhx = ilog2(hx);
+  auto blocks = [](int64_t n, int per) { return (unsigned)((n + per - 1) / per); };
 #define RFFTQ(MODE, RIN, ROUT)                                                                                        \
-  do {                                                                                                             \
-    if (xq == 16)                                                                                                  \
-      hipLaunchKernelGGL((k_rfftq_x<T, MODE, 16>), nxb, 256, 0, ctx->stream, (int64_t)nlines, RIN, buf, ROUT,       \
-                         ctx->tw[0], 1.0, ilog2(ny), P);                                                           \
-    else if constexpr (sizeof(T) == 4)                                                                             \
-      hipLaunchKernelGGL((k_rfftq_x<T, MODE, 32>), nxb, 256, 0, ctx->stream, (int64_t)nlines, RIN, buf, ROUT,       \
-                         ctx->tw[0], 1.0, ilog2(ny), P);                                                           \
-  } while (0)
-#define FFTQ(MODE, RQ, NB, A_, ES, CS, TW)                                                                           \
-  do {                                                                                                             \
-    if (RQ == 16)                                                                                                  \
-      hipLaunchKernelGGL((k_fftq_s<T, MODE, 16>), NB, 256, 0, ctx->stream, A_, ES, CS, buf, TW, sym, ctx->trig[0], \
-                         ctx->trig[1], ctx->trig[2]);                                                              \
-    else if constexpr (sizeof(T) == 4)                                                                             \
-      hipLaunchKernelGGL((k_fftq_s<T, MODE, 32>), NB, 256, 0, ctx->stream, A_, ES, CS, buf, TW, sym, ctx->trig[0], \
-                         ctx->trig[1], ctx->trig[2]);                                                              \
-  } while (0)
+  Q_AXIS(T, nx, hipLaunchKernelGGL((k_rfftq_x<T, MODE, TH, R>), blocks(nlines, 2 * NL), NL * TH, 0, ctx->stream,       \
+                                   (int64_t)nlines, RIN, buf, ROUT, ctx->tw[0], 1.0, ilog2(ny), P))
+#define FFTQ(MODE, n, LINES, LA, EXTRA, ES, CS, TW)                                                                    \
+  Q_AXIS(T, n, hipLaunchKernelGGL((k_fftq_s<T, MODE, TH, R>), blocks(LINES, NL) + EXTRA, NL * TH, 0, ctx->stream,      \
+                                  (int64_t)(LINES), LA, ES, CS, buf, TW, sym, ctx->trig[0], ctx->trig[1], ctx->trig[2]))
   if (xq) {  // x forward: real lines -> half spectra (kx < nx/2, slot 0 packs kx = 0, nx/2)
     RFFTQ(0, r, (T *)nullptr);
   } else {
@@ -848,7 +885,7 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
   }
   // y forward: lines (kx, iz); A = nx/2 contiguous, c = iz with stride P
   if (yq) {
-    FFTQ(0, yq, nyb, (int64_t)hx, (int64_t)hx, P, ctx->tw[1]);
+    FFTQ(0, ny, (int64_t)hx * nz, lhx, 0u, (int64_t)hx, P, ctx->tw[1]);
   } else {
     const int n = ny, B = fft_batch<T>(n, hx);
     hipLaunchKernelGGL((k_fft_s<T, 0>), (unsigned)((hx / B) * nz), kBlock, fft_lds<T>(n, B), ctx->stream, ilog2(n),
@@ -859,7 +896,7 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
     const int n = nz;
     const int64_t A = (int64_t)hx * ny;
     if (zq) {  // (ny more blocks take the kx = 0 column)
-      FFTQ(2, zq, (unsigned)(A / 16 + ny), A, P, (int64_t)0, ctx->tw[2]);
+      FFTQ(2, nz, A, ilog2(A), (unsigned)ny, P, (int64_t)0, ctx->tw[2]);
     } else {
       const int B = fft_batch_z<T>(n, A);
       hipLaunchKernelGGL((k_fft_s<T, 2>), (unsigned)(A / B), kBlock, fft_lds_z<T>(n, B), ctx->stream, ilog2(n), A, P,
@@ -870,7 +907,7 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
     }
   }
   if (yq) {  // y inverse
-    FFTQ(1, yq, nyb, (int64_t)hx, (int64_t)hx, P, ctx->tw[1]);
+    FFTQ(1, ny, (int64_t)hx * nz, lhx, 0u, (int64_t)hx, P, ctx->tw[1]);
   } else {
     const int n = ny, B = fft_batch<T>(n, hx);
     hipLaunchKernelGGL((k_fft_s<T, 1>), (unsigned)((hx / B) * nz), kBlock, fft_lds<T>(n, B), ctx->stream, ilog2(n),

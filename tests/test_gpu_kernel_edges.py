@@ -61,6 +61,36 @@ def test_two_level_correction_on_any_plane(N, prec, base):
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
 
 
+# each length of the register four-step passes on each axis (FP64: 16 to 256,
+# FP32: to 512), beside lengths of the LDS passes (4, 8); line counts below and
+# above a block's 16 to 64 lines.  A mode's symbol is a sum of weights v_o that
+# cancels to lambda(k): its roundings, 16 on the two sides, move the mode by
+# eps sum|v_o| / |lambda(k)|.  An FP32 transform moves each mode of white noise
+# by some eps32 log2(nodes).
+@pytest.mark.parametrize("prec,base", [("fp64", 1e-13), ("mixed", 2e-5)])
+@pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5"])
+@pytest.mark.parametrize("N", [(16, 4, 4), (4, 16, 4), (4, 4, 16), (16, 16, 32), (32, 32, 16), (64, 16, 8), (8, 64, 16),
+                               (32, 8, 64), (128, 32, 4), (16, 128, 8), (4, 8, 128), (64, 64, 64), (256, 16, 4),
+                               (8, 256, 16), (4, 4, 256), (512, 4, 16), (4, 512, 4), (8, 4, 512)])
+def test_fft_passes_on_axes_of_any_length(N, extra, prec, base):
+    rng = np.random.default_rng(17)
+    with context(opts(N, extra=f"-pc_type fft -precision {prec} {extra}")) as ctx:
+        g = grid_of(ctx.prm)
+        ctx.set_moments(vlasov_from([np.ones(g.nc)] + _moments(g, rng)[1:]))
+        r = rng.standard_normal(g.nc)
+        r -= r.mean()
+        z = ctx.pc_apply(r)
+        K = list(ctx.prm.kappa_e)
+    delta = np.zeros(g.nc)
+    delta[0] = 1
+    row = orc.lhs_apply(g, K, np.ones(g.nc), delta)
+    lam = np.abs(np.fft.fftn(row.reshape(N[::-1]))).ravel()
+    tol = base + 16 * 2.0 ** -52 * np.abs(row).sum() / lam[1:].min()
+    ref = orc.pc_apply(g, K, np.ones(g.nc), r, orc.PC_FFT)
+    z, ref = z - z.mean(), ref - ref.mean()
+    assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
+
+
 # columns of 16, 32 and 64 lanes of 1, 2, 4 and 8 planes each, full and ragged,
 # and one beyond (513 planes, the levels with x fastest); level widths that are
 # and are not multiples of a block's columns.  The level solves are exact but
