@@ -166,6 +166,18 @@ int fetch(chy_ctx *ctx, const double *dev, int nv, double *host)
   return CHY_OK;
 }
 
+// Largest grid whose next direction is launched before the dot products of the
+// present one are read, and the margin by which another iteration has to be
+// expected.  A read leaves the GPU idle for the round trip and the launches
+// after it: 6 to 9 us of an iteration of 75 to 110 us.  us of a solve with the
+// direction after and before the read: 16^3 FP64 1065 -> 980, 32^3 FP64 1002 ->
+// 946, 64^3 FP64 1195 -> 1153, 64 x 48 x 40 FP64 with multigrid 14.8 -> 14.3
+// ms, 128^3 FP64 2.33 -> 2.30 ms.  Beyond 128^3 nothing is left to gain, and a
+// direction launched in vain costs (256^3 mixed, 5.9 ms: 0.5 ms with a margin
+// of 2, which expects one too many there; none with 5).
+constexpr int64_t kAheadMax = (int64_t)1 << 21;
+constexpr double kAheadMargin = 5.0;
+
 // ---- inner GMRES on A e = rhs (e starts at zero), precision T -------------------
 // rhs == V (basis slot 0): the caller wrote the right-hand side there, and
 // beta_hint > 0 is its norm; the first cycle then starts without a copy or a
@@ -190,6 +202,7 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
   double *sc2 = ctx->h_scale;  // sc[q]^2, passed by value to the combines
   launch_fill<T>(ctx, nc, e, (T)0);
   double beta0 = -1.0, beta_prev = -1.0;
+  double rate = 0.1;  // the last iteration's reduction of the residual norm
   *its = 0;
   *relres = 1.0;
   const bool in_place = rhs == V;
@@ -235,13 +248,27 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
     std::fill(g.begin(), g.end(), 0.0);
     g[0] = beta;
     int64_t j = 0;
-    bool done = false;
-    for (; j < m && *its < max_it; j++) {
-      T *Vj = V + j * nc, *Zj = Z + j * nc, *Vn = V + (j + 1) * nc;
-      TRY(pc_apply<T>(ctx, v19, Vj, Zj));
+    bool done = false, ahead = false;
+    // Z_j = M^-1 U_j and A Z_j, built in place in slot j + 1
+    auto direction = [&](int64_t q) -> int {
+      TRY(pc_apply<T>(ctx, v19, V + q * nc, Z + q * nc));
       timer_start(ctx, "lhs_apply");
-      launch_lhs_apply<T, T, T>(ctx, lt, ctx->solve_transpose, n, Zj, Vn);  // w built in place in slot j+1
+      launch_lhs_apply<T, T, T>(ctx, lt, ctx->solve_transpose, n, Z + q * nc, V + (q + 1) * nc);
       timer_stop(ctx, "lhs_apply");
+      return CHY_OK;
+    };
+    // The next direction needs nothing that the host is about to read, so it is
+    // launched before the read when another iteration is expected.
+    auto run_ahead = [&](int64_t q) -> int {
+      const bool last = q + 1 >= m || *its + 1 >= max_it || fabs(g[q]) * rate <= kAheadMargin * rtol * beta0;
+      if (last || nc > kAheadMax) return CHY_OK;
+      ahead = true;
+      return direction(q + 1);
+    };
+    for (; j < m && *its < max_it; j++) {
+      T *Vn = V + (j + 1) * nc;
+      if (!ahead) TRY(direction(j));
+      ahead = false;
       timer_start(ctx, "krylov");
       // classical Gram-Schmidt; the norm of the result is fused into the last
       // update and everything is read back at once.  REFINE_ALWAYS makes a
@@ -256,11 +283,17 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
       if (refine == CHY_CGS_REFINE_ALWAYS) {
         launch_gs_update_dots<T>(ctx, (int)(j + 1), V, nc, hdev, Vn, nc, h2dev, sc2);
         launch_gs_update_norm<T>(ctx, (int)(j + 1), V, nc, h2dev, Vn, nc, ndev);
+        timer_stop(ctx, "krylov");
+        TRY(run_ahead(j));
         TRY(fetch(ctx, ctx->red_out, (int)(2 * (m + 2) + 1), ctx->h_red));
         for (int64_t q = 0; q <= j; q++) h[q] = sc[q] > 0.0 ? (ctx->h_red[q] + ctx->h_red[(m + 2) + q]) * sj / sc[q] : 0.0;
         wn = sqrt(ctx->h_red[2 * (m + 2)]);
       } else {
         launch_gs_update_norm<T>(ctx, (int)(j + 1), V, nc, hdev, Vn, nc, ndev);
+        if (refine == CHY_CGS_REFINE_NEVER) {
+          timer_stop(ctx, "krylov");
+          TRY(run_ahead(j));
+        }
         TRY(fetch(ctx, ctx->red_out, (int)(2 * (m + 2) + 1), ctx->h_red));
         double proj = 0.0;
         for (int64_t q = 0; q <= j; q++) {
@@ -275,8 +308,8 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
           for (int64_t q = 0; q <= j; q++) h[q] += sc[q] > 0.0 ? ctx->h_red[(m + 2) + q] * sj / sc[q] : 0.0;
           wn = sqrt(ctx->h_red[2 * (m + 2)]);
         }
+        if (refine == CHY_CGS_REFINE_IFNEEDED) timer_stop(ctx, "krylov");
       }
-      timer_stop(ctx, "krylov");
       h[j + 1] = wn * sj;
       if (!std::isfinite(h[j + 1])) return set_err(ctx, CHY_ERR_FP, "non-finite Arnoldi vector");
       sc[j + 1] = wn > 0.0 ? 1.0 / wn : 0.0;
@@ -291,6 +324,7 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
       sn[j] = rr > 0.0 ? h[j + 1] / rr : 0.0;
       h[j] = rr;
       g[j + 1] = -sn[j] * g[j];
+      rate = fabs(g[j + 1] / g[j]);
       g[j] = cs[j] * g[j];
       for (int64_t q = 0; q <= j; q++) H[q * m + j] = h[q];
       (*its)++;

@@ -91,6 +91,27 @@ def test_fft_passes_on_axes_of_any_length(N, extra, prec, base):
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
 
 
+# the next direction is launched before the present one's dot products are read,
+# except where the cycle, the iteration limit or the expected convergence ends
+# it: each end of a cycle against the oracle's iterate after as many steps (in
+# exact arithmetic the same; the least-squares step amplifies the rounding of
+# the basis by the conditioning of the preconditioned operator, below 100)
+@pytest.mark.parametrize("restart", [1, 2, 3, 30])
+@pytest.mark.parametrize("max_it", [1, 2, 3, 4, 6])
+def test_gmres_cycles_cut_at_any_iteration(restart, max_it):
+    N = (16, 16, 8)
+    with context(opts(N, extra=f"-pc_type fft -ksp_rtol 1e-14 -ksp_max_it {max_it} -ksp_gmres_restart {restart}")) as ctx:
+        g = grid_of(ctx.prm)
+        mom = _moments(g, np.random.default_rng(18))
+        ctx.set_moments(vlasov_from(mom))
+        phi, st = ctx.solve_potential()
+        b = ctx.get_rhs()
+        K = list(ctx.prm.kappa_e)
+    ref, its, conv, _ = orc.solve(g, K, mom[0], b, rtol=1e-14, max_it=max_it, restart=restart)
+    assert (st.iterations, st.converged) == (its, 0) and not conv
+    assert np.abs(phi - ref).max() <= 1e-11 * np.abs(ref).max()
+
+
 # columns of 16, 32 and 64 lanes of 1, 2, 4 and 8 planes each, full and ragged,
 # and one beyond (513 planes, the levels with x fastest); level widths that are
 # and are not multiples of a block's columns.  The level solves are exact but
