@@ -929,30 +929,46 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
 }
 
 // ---- two-level preconditioner: kz = 0 correction -------------------------------------
-// The 2-D inner GMRES runs on up to kNB2 blocks of 256 threads.  Every global
-// sum is left as one partial per block; the kernel that needs it adds the
-// partials itself (every block in the same fixed order, so all blocks agree
-// bit for bit), which keeps one launch per Gram-Schmidt pass.
+// The 2-D inner GMRES keeps its basis unnormalised (U_q), so that no pass
+// waits for a norm: a step is three launches, each leaving one partial per
+// block of the sums that the next one needs (every block adds them in the same
+// fixed order, so all blocks agree bit for bit).  The launches are 4 to 6 us
+// each, bound by latency: seven with the final solve, where a launch per pass
+// and a second Gram-Schmidt pass made fourteen.  us of a solve of 8
+// iterations, fourteen -> seven launches: 64 x 128 x 64 mixed 1270 -> 1060,
+// 128^3 FP64 2290 -> 2090, 128^3 mixed 1770 -> 1575, 256^3 FP64 11300 -> 11180.
 constexpr int kHm = kFft2Its;
-constexpr int kNB2 = 256;
 constexpr int kExtZ = 16;  // planes per block when the correction is added
 
-static int nb2_of(int64_t nxy) { return (int)std::min<int64_t>(kNB2, (nxy + 255) / 256); }
+// Rows of a block of the x passes: 64 blocks or more where there are rows
+// enough, and with the two rows around them within 64 KB of LDS.
+template <typename T>
+static int rows2_of(int nx, int ny)
+{
+  int R = std::max(1, ny / 64);
+  while (R > 1 && fft_lds<T>(nx, R + 2) > 65536) R >>= 1;
+  return R;
+}
 
-// x-y fields in pc2_buf (T): C (9), V (kFft2Its + 1), Z (kFft2Its), w, and a
+static int nb2_of(const chy_ctx *ctx, bool fp32)
+{
+  const int nx = ctx->g.nx, ny = ctx->g.ny;
+  return ny / (fp32 ? rows2_of<float>(nx, ny) : rows2_of<double>(nx, ny));
+}
+
+// x-y fields in pc2_buf (T): C (9), U (kFft2Its), Z (kFft2Its), w, and a
 // complex work plane (2).
 int64_t fft2_buf_elems(const chy_ctx *ctx)
 {
-  return (int64_t)(9 + (kFft2Its + 1) + kFft2Its + 1 + 2) * ctx->g.nx * ctx->g.ny;
+  return (int64_t)(9 + kFft2Its + kFft2Its + 1 + 2) * ctx->g.nx * ctx->g.ny;
 }
 
 // Double workspace in pc2_h: the z-chunk column sums part[zc][nxy], the
 // stencil-block sums pl[nlb], then per-block partials of the inner GMRES:
-// pn[j][nb] (|V_j|^2 before normalisation, j <= m), p1[j][q][nb] and
-// p2[j][q][nb] (V_q . w in the two Gram-Schmidt passes of step j), and the
-// least-squares coefficients y[m].
+// pn[j][nb] (|U_j|^2), pd[j][q][nb] (U_q . w in step j, q <= j, and |w|^2 of
+// the last step at q = m), and the coefficients y[m] of the Z_q.
 struct H2 {
-  double *part, *pl, *pn, *p1, *p2, *y;
+  double *part, *pl, *pn, *pd, *y;
   int64_t nlb;
   int nb;
 };
@@ -961,24 +977,23 @@ static H2 h2_layout(const chy_ctx *ctx, bool fp32)
 {
   const int64_t nxy = (int64_t)ctx->g.nx * ctx->g.ny;
   H2 h;
-  h.nb = nb2_of(nxy);
+  h.nb = nb2_of(ctx, fp32);
   h.nlb = lhs_zsum_blocks(ctx->g, fp32);
   h.part = ctx->pc2_h;
   h.pl = h.part + (int64_t)lhs_zchunks(ctx->g, fp32) * nxy;
   h.pn = h.pl + h.nlb;
-  h.p1 = h.pn + (int64_t)(kHm + 1) * h.nb;
-  h.p2 = h.p1 + (int64_t)kHm * kHm * h.nb;
-  h.y = h.p2 + (int64_t)kHm * kHm * h.nb;
+  h.pd = h.pn + (int64_t)kHm * h.nb;
+  h.y = h.pd + (int64_t)kHm * (kHm + 1) * h.nb;
   return h;
 }
 
 int64_t fft2_h_elems(const chy_ctx *ctx)
 {
   const int64_t nxy = (int64_t)ctx->g.nx * ctx->g.ny;
-  const int nb = nb2_of(nxy);
   const bool fp32 = ctx->mixed;
-  return (int64_t)lhs_zchunks(ctx->g, fp32) * nxy + lhs_zsum_blocks(ctx->g, fp32) + (int64_t)(kHm + 1) * nb +
-         2 * (int64_t)kHm * kHm * nb + kHm;
+  const int nb = nb2_of(ctx, fp32);
+  return (int64_t)lhs_zchunks(ctx->g, fp32) * nxy + lhs_zsum_blocks(ctx->g, fp32) +
+         (int64_t)kHm * (kHm + 2) * nb + kHm;
 }
 
 // Block-wide sums of nv values per thread: out[q] (LDS) for q < nv.
@@ -1005,153 +1020,144 @@ __device__ __forceinline__ void block_sums(double (&v)[NV], int nv, double *out)
   __syncthreads();
 }
 
-// out[q] = sum over b < nb of p[q * nb + b], q < nv (LDS; same value in every block)
-template <int NV>
-__device__ __forceinline__ void sum_partials(const double *__restrict__ p, int nb, int nv, double *out)
-{
-  double a[NV];
-#pragma unroll
-  for (int q = 0; q < NV; q++) a[q] = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-#pragma unroll
-    for (int q = 0; q < NV; q++)
-      if (q < nv) a[q] += p[(int64_t)q * nb + b];
-  }
-  block_sums<NV>(a, nv, out);
-}
-
-// V0 = r2 - mean(r2), with r2[col] = (1/nz) sum_k (r - A z) from the z-chunk
-// column sums; pn[0][blk] = the block's part of |V0|^2
-template <typename T>
-__global__ __launch_bounds__(256) void k2_r2(int64_t nxy, int nz, int nzc, const double *__restrict__ part,
-                                             const double *__restrict__ pl, int64_t nlb, T *__restrict__ V0,
-                                             double *__restrict__ pn)
-{
-  __shared__ double m[1], q2[1];
-  double a[1] = {0.0};
-  for (int64_t b = threadIdx.x; b < nlb; b += blockDim.x) a[0] += pl[b];
-  block_sums<1>(a, 1, m);
-  const double inz = 1.0 / (double)nz, mean = m[0] * inz / (double)nxy;
-  a[0] = 0.0;
-  for (int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; col < nxy; col += (int64_t)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int zc = 0; zc < nzc; zc++) s += part[(int64_t)zc * nxy + col];
-    const T x = (T)(s * inz - mean);
-    V0[col] = x;
-    a[0] += (double)x * (double)x;
-  }
-  block_sums<1>(a, 1, q2);
-  if (threadIdx.x == 0) pn[blockIdx.x] = q2[0];
-}
-
-// 2-D complex pass along x.  MODE 0: V_j (before normalisation, |V_j|^2 in
-// the partials pn) is scaled to unit norm (zero when the norm is zero),
-// written back, and transformed forward.  MODE 1: inverse transform, real
-// part to io.
-template <typename T, int MODE>
-__global__ __launch_bounds__(256) void k_fft2_x(int logn, int nlines, int B, T *__restrict__ io,
-                                                cpx<T> *__restrict__ buf, const double *__restrict__ tw,
-                                                const double *__restrict__ pn, int nb)
+// Direction j, forward along x.  j = 0: U_0 = r2 - mean(r2), with r2[col] =
+// (1/nz) sum_k (r - A z) from the z-chunk column sums; else U_j = w less its
+// parts along U_0 .. U_(j-1) (one classical Gram-Schmidt pass: with two
+// directions a second one changes the last bits only).  Stores U_j, |U_j|^2
+// in the partials, and the rows' transforms (bit-reversed along x) in cb.
+template <typename T, bool FIRST>
+__global__ __launch_bounds__(256) void k2_dir(int lx, int R, int64_t nxy, int j, int nz, int nzc,
+                                              const double *__restrict__ part, const double *__restrict__ pl,
+                                              int64_t nlb, T *__restrict__ U, const T *__restrict__ w,
+                                              cpx<T> *__restrict__ cb, const double *__restrict__ tw,
+                                              double *__restrict__ pn, const double *__restrict__ pd)
 {
   extern __shared__ unsigned char smem_raw[];
-  const int n = 1 << logn;
+  const int nx = 1 << lx, nb = (int)gridDim.x;
+  cpx<T> *tws = reinterpret_cast<cpx<T> *>(smem_raw);
+  cpx<T> *s = tws + (nx >> 1);
+  __shared__ double h[2 * kHm];
+  load_twiddles<T>(tws, tw, nx);
+  const int64_t c0 = (int64_t)blockIdx.x * R << lx;
+  double mean = 0.0, a[1] = {0.0};
+  if (FIRST) {
+    for (int64_t b = threadIdx.x; b < nlb; b += blockDim.x) a[0] += pl[b];
+    block_sums<1>(a, 1, h);
+    mean = h[0] / ((double)nz * (double)nxy);
+  } else {
+    // the coefficients of the U_q: (U_q . w) / |U_q|^2
+    double t[2 * kHm];
+#pragma unroll
+    for (int q = 0; q < 2 * kHm; q++) t[q] = 0.0;
+    for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+#pragma unroll
+      for (int q = 0; q < kHm; q++)
+        if (q < j) {
+          t[q] += pd[(int64_t)((j - 1) * (kHm + 1) + q) * nb + b];
+          t[kHm + q] += pn[(int64_t)q * nb + b];
+        }
+    }
+    block_sums<2 * kHm>(t, 2 * kHm, h);
+  }
+  a[0] = 0.0;
+  for (int e = threadIdx.x; e < R << lx; e += blockDim.x) {
+    const int64_t col = c0 + e;
+    double x;
+    if (FIRST) {
+      double t = 0.0;
+#pragma unroll 8
+      for (int zc = 0; zc < nzc; zc++) t += part[(int64_t)zc * nxy + col];
+      x = t / (double)nz - mean;
+    } else {
+      x = (double)w[col];
+#pragma unroll
+      for (int q = 0; q < kHm; q++)
+        if (q < j && h[kHm + q] > 0.0) x -= h[q] / h[kHm + q] * (double)U[(int64_t)q * nxy + col];
+    }
+    const T xt = (T)x;
+    U[(int64_t)j * nxy + col] = xt;
+    s[(e >> lx) * (nx + 1) + (e & (nx - 1))] = {xt, (T)0};
+    a[0] += (double)xt * (double)xt;
+  }
+  __syncthreads();
+  dif_fwd<T>(s, R, lx, tws);
+  for (int e = threadIdx.x; e < R << lx; e += blockDim.x) cb[c0 + e] = s[(e >> lx) * (nx + 1) + (e & (nx - 1))];
+  block_sums<1>(a, 1, h);
+  if (threadIdx.x == 0) pn[(int64_t)j * nb + blockIdx.x] = h[0];
+}
+
+// Z_j back along x and w = A2 Z_j with the z-averaged 9-point coefficients:
+// a block transforms its R rows and the two around them (INV; else Z_j is
+// there already), stores its rows of Z_j and of w, and leaves its parts of
+// U_q . w (q <= j), in the last step of |w|^2 too.
+template <typename T, bool INV>
+__global__ __launch_bounds__(256) void k2_apply(int lx, int R, int ny, int j, const T *__restrict__ C,
+                                                const cpx<T> *__restrict__ cb, const double *__restrict__ tw,
+                                                T *__restrict__ Zj, const T *__restrict__ U, T *__restrict__ w,
+                                                double *__restrict__ pd)
+{
+  extern __shared__ unsigned char smem_raw[];
+  __shared__ double h[kHm + 1];
+  const int nx = 1 << lx, nb = (int)gridDim.x;
+  const int64_t nxy = (int64_t)ny << lx;
+  cpx<T> *tws = reinterpret_cast<cpx<T> *>(smem_raw);
+  cpx<T> *s = tws + (nx >> 1);  // line l: row r0 - 1 + l
+  const int r0 = (int)blockIdx.x * R;
+  if (INV) {
+    load_twiddles<T>(tws, tw, nx);
+    for (int e = threadIdx.x; e < (R + 2) << lx; e += blockDim.x) {
+      const int l = e >> lx, t = e & (nx - 1);
+      s[l * (nx + 1) + t] = cb[((int64_t)((r0 - 1 + l) & (ny - 1)) << lx) + t];
+    }
+    __syncthreads();
+    dit_inv<T>(s, R + 2, lx, tws);
+  }
+  double a[kHm + 1];
+#pragma unroll
+  for (int q = 0; q <= kHm; q++) a[q] = 0.0;
+  for (int e = threadIdx.x; e < R << lx; e += blockDim.x) {
+    const int l = (e >> lx) + 1, i = e & (nx - 1);
+    const int64_t col = ((int64_t)r0 << lx) + e;
+    const int xs[3] = {(i - 1) & (nx - 1), i, (i + 1) & (nx - 1)};
+    double acc = 0.0;
+#pragma unroll
+    for (int o = 0; o < 9; o++) {
+      const int lo = l + o / 3 - 1;
+      const T zv = INV ? s[lo * (nx + 1) + xs[o % 3]].x
+                       : Zj[((int64_t)((r0 - 1 + lo) & (ny - 1)) << lx) + xs[o % 3]];
+      acc += (double)C[o * nxy + col] * (double)zv;
+    }
+    const T wt = (T)acc;
+    if (INV) Zj[col] = s[l * (nx + 1) + i].x;
+    if (j + 1 < kHm) w[col] = wt;
+#pragma unroll
+    for (int q = 0; q < kHm; q++)
+      if (q <= j) a[q] += (double)U[(int64_t)q * nxy + col] * (double)wt;
+    a[kHm] += (double)wt * (double)wt;
+  }
+  block_sums<kHm + 1>(a, kHm + 1, h);
+  if (threadIdx.x <= kHm) pd[(int64_t)(j * (kHm + 1) + (int)threadIdx.x) * nb + blockIdx.x] = h[threadIdx.x];
+}
+
+// Inverse transform along x, real part to io (lines too long for k2_apply's
+// rows in LDS)
+template <typename T>
+__global__ __launch_bounds__(256) void k2_inv_x(int lx, int nlines, int B, T *__restrict__ io,
+                                                const cpx<T> *__restrict__ cb, const double *__restrict__ tw)
+{
+  extern __shared__ unsigned char smem_raw[];
+  const int n = 1 << lx;
   cpx<T> *tws = reinterpret_cast<cpx<T> *>(smem_raw);
   cpx<T> *s = tws + (n >> 1);
-  __shared__ double hn[1];
-  double inv = 1.0;
-  if (MODE == 0) {
-    sum_partials<1>(pn, nb, 1, hn);
-    const double h = sqrt(hn[0]);
-    inv = h > 0.0 ? 1.0 / h : 0.0;
-  }
   load_twiddles<T>(tws, tw, n);
   const int64_t l0 = (int64_t)blockIdx.x * B;
   const int nbl = (int)((nlines - l0) < B ? (nlines - l0) : B);
-  for (int e = threadIdx.x; e < (nbl << logn); e += blockDim.x) {
-    const int b = e >> logn, t = e & (n - 1);
-    const int64_t a = (l0 + b) * n + t;
-    if (MODE == 0) {
-      const T v = (T)((double)io[a] * inv);
-      io[a] = v;
-      s[b * (n + 1) + t] = {v, (T)0};
-    } else {
-      s[b * (n + 1) + t] = buf[a];
-    }
-  }
+  for (int e = threadIdx.x; e < (nbl << lx); e += blockDim.x)
+    s[(e >> lx) * (n + 1) + (e & (n - 1))] = cb[(l0 << lx) + e];
   __syncthreads();
-  if (MODE == 0) dif_fwd<T>(s, nbl, logn, tws);
-  else dit_inv<T>(s, nbl, logn, tws);
-  for (int e = threadIdx.x; e < (nbl << logn); e += blockDim.x) {
-    const int b = e >> logn, t = e & (n - 1);
-    const int64_t a = (l0 + b) * n + t;
-    if (MODE == 0) buf[a] = s[b * (n + 1) + t];
-    else io[a] = s[b * (n + 1) + t].x;
-  }
-}
-
-// w = A2 Z_j with the z-averaged 9-point coefficients; p1[q][blk] = the
-// block's part of V_q . w, q <= j
-template <typename T>
-__global__ __launch_bounds__(256) void k2_a2dots(int nx, int ny, int j, const T *__restrict__ C,
-                                                 const T *__restrict__ Zj, const T *__restrict__ V,
-                                                 T *__restrict__ w, double *__restrict__ p1, int nb)
-{
-  __shared__ double h[kHm];
-  const int64_t nxy = (int64_t)nx * ny;
-  double a[kHm];
-#pragma unroll
-  for (int q = 0; q < kHm; q++) a[q] = 0.0;
-  for (int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; col < nxy; col += (int64_t)gridDim.x * blockDim.x) {
-    const int i = (int)(col % nx), jy = (int)(col / nx);
-    const int ip = i + 1 == nx ? 0 : i + 1, im = i == 0 ? nx - 1 : i - 1;
-    const int jp = jy + 1 == ny ? 0 : jy + 1, jm = jy == 0 ? ny - 1 : jy - 1;
-    const int xs[3] = {im, i, ip}, ys[3] = {jm, jy, jp};
-    double acc = 0.0;
-#pragma unroll
-    for (int o = 0; o < 9; o++) acc += (double)C[o * nxy + col] * (double)Zj[xs[o % 3] + (int64_t)nx * ys[o / 3]];
-    const T wt = (T)acc;
-    w[col] = wt;
-#pragma unroll
-    for (int q = 0; q < kHm; q++)
-      if (q <= j) a[q] += (double)V[(int64_t)q * nxy + col] * (double)wt;
-  }
-  block_sums<kHm>(a, j + 1, h);
-  if (threadIdx.x <= j) p1[(int64_t)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
-}
-
-// One classical Gram-Schmidt pass of step j: h = the sums of pin,
-// x = w - sum_q h_q V_q.  PASS 1: w = x, pout[q][blk] = parts of V_q . x.
-// PASS 2: V_{j+1} = x (normalised by the next pass along x), pout[blk] = part
-// of |x|^2.
-template <typename T, int PASS>
-__global__ __launch_bounds__(256) void k2_gs_pass(int64_t nxy, int j, T *__restrict__ V, T *__restrict__ w,
-                                                  const double *__restrict__ pin, double *__restrict__ pout, int nb)
-{
-  __shared__ double h[kHm], o[kHm];
-  sum_partials<kHm>(pin, nb, j + 1, h);
-  double a[kHm];
-#pragma unroll
-  for (int q = 0; q < kHm; q++) a[q] = 0.0;
-  T *Vn = V + (int64_t)(j + 1) * nxy;
-  for (int64_t col = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; col < nxy; col += (int64_t)gridDim.x * blockDim.x) {
-    double x = (double)w[col];
-#pragma unroll
-    for (int q = 0; q < kHm; q++)
-      if (q <= j) x -= h[q] * (double)V[(int64_t)q * nxy + col];
-    const T xt = (T)x;
-    if (PASS == 1) {
-      w[col] = xt;
-#pragma unroll
-      for (int q = 0; q < kHm; q++)
-        if (q <= j) a[q] += (double)V[(int64_t)q * nxy + col] * (double)xt;
-    } else {
-      Vn[col] = xt;
-      a[0] += (double)xt * (double)xt;
-    }
-  }
-  const int nv = PASS == 1 ? j + 1 : 1;
-  block_sums<kHm>(a, nv, o);
-  if (threadIdx.x < nv) pout[(int64_t)threadIdx.x * nb + blockIdx.x] = o[threadIdx.x];
+  dit_inv<T>(s, nbl, lx, tws);
+  for (int e = threadIdx.x; e < (nbl << lx); e += blockDim.x)
+    io[(l0 << lx) + e] = s[(e >> lx) * (n + 1) + (e & (n - 1))].x;
 }
 
 // Givens QR of the Hessenberg columns h[q][j] (q <= j) with subdiagonals
@@ -1195,54 +1201,54 @@ __device__ __forceinline__ void h2_lstsq(const double (&sub)[kHm + 1], const dou
 }
 
 // Hessenberg columns from the partials, Givens QR and back substitution
-// (one block): y[q], q < kHm (zero past a breakdown).
-// (Every sum is formed as sum_partials forms it, so the values are those the
-// other kernels used.)
-constexpr int kNSums = (kHm + 1) + kHm * (kHm + 1);
-__global__ __launch_bounds__(256) void k2_solve(const double *__restrict__ pn, const double *__restrict__ p1,
-                                                const double *__restrict__ p2, int nb, double *__restrict__ y)
+// (one block): the coefficients y[q] of the Z_q, q < kHm (zero past a
+// breakdown).  The normalised basis is U_q / n_q, n_q = |U_q|; the last
+// subdiagonal entry, the norm of what is left of w, comes from |w|^2 less the
+// parts taken out.
+constexpr int kNSums = kHm * (kHm + 2);
+__global__ __launch_bounds__(256) void k2_solve(const double *__restrict__ p, int nb, double *__restrict__ y)
 {
+  // p: pn[j], then pd[j][q]
   __shared__ double red[kNSums];
   double a[kNSums];
 #pragma unroll
   for (int t = 0; t < kNSums; t++) a[t] = 0.0;
   for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    int t = 0;
 #pragma unroll
-    for (int j = 0; j <= kHm; j++) a[t++] += pn[(int64_t)j * nb + b];
-#pragma unroll
-    for (int j = 0; j < kHm; j++)
-#pragma unroll
-      for (int q = 0; q <= j; q++) {
-        a[t++] += p1[(int64_t)(j * kHm + q) * nb + b];
-        a[t++] += p2[(int64_t)(j * kHm + q) * nb + b];
-      }
+    for (int t = 0; t < kNSums; t++) a[t] += p[(int64_t)t * nb + b];
   }
   block_sums<kNSums>(a, kNSums, red);
   if (threadIdx.x != 0) return;
-  double sub[kHm + 1], hc[kHm][kHm];
-  int t = 0;
-  for (int j = 0; j <= kHm; j++) sub[j] = sqrt(red[t++]);
+  double sub[kHm + 1], hc[kHm][kHm], in[kHm];
+  for (int j = 0; j < kHm; j++) {
+    const double n2 = red[j];
+    in[j] = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
+    sub[j] = sqrt(n2) * (j > 0 ? in[j - 1] : 1.0);
+  }
+  const double *d = red + kHm;  // d[j (kHm + 1) + q]
   for (int j = 0; j < kHm; j++)
-    for (int q = 0; q <= j; q++) {
-      hc[q][j] = red[t] + red[t + 1];
-      t += 2;
-    }
+    for (int q = 0; q <= j; q++) hc[q][j] = d[j * (kHm + 1) + q] * in[q] * in[j];
+  const int m = kHm - 1;
+  double left = d[m * (kHm + 1) + kHm] * in[m] * in[m];
+  for (int q = 0; q <= m; q++) left -= hc[q][m] * hc[q][m];
+  sub[kHm] = left > 0.0 ? sqrt(left) : 0.0;
   h2_lstsq(sub, hc, y);
+  for (int q = 0; q < kHm; q++) y[q] *= in[q];
 }
 
 // ---- the whole 2-D correction in one workgroup ------------------------------------
-// On a plane of at most kPlaneMax nodes every kernel of the correction is a
-// launch of a few microseconds of latency: fourteen of them, 4 to 5 us each.
-// One workgroup of 1024 threads does them all: the columns it owns (P per
-// thread) stay in registers, the plane being transformed sits in LDS, and the
-// global sums are block sums.  It takes 20 us at 32^2 and 38 (FP32) or 49 us
-// (FP64) at 64^2; the launches take about 60 us there, and 15 to 20 us of gaps
-// between them.  (One CU does this work: at 128^2 it would take longer than
-// the launches.)  What bounds it is the latency of some 60 barriers and the
-// LDS round trips of the transforms between them.
-constexpr int kPlaneMax = 4096, kPlaneT = 1024, kPlaneP = kPlaneMax / kPlaneT;
-constexpr int kPlanePad = 1024;  // most lines of a plane (axes of 4 nodes and more): one pad value each
+// On a plane of at most kPlaneMax nodes each of the correction's seven launches
+// is 4 to 5 us of latency.  One workgroup of 512 threads does all of them (1024
+// make the barriers dearer: 3 to 6 % of a solve at 16^3, 1 % at 32^3): the
+// columns it owns (P per thread) stay in registers, the plane being transformed
+// sits in LDS, and the global sums are block sums.  What bounds it is the
+// latency of some 60 barriers and the LDS round trips of the transforms between
+// them: 22 us at 32^2, but 38 (FP32) and 49 us (FP64) at 64^2, one CU doing the
+// work.  us of a solve with one workgroup and with the launches: 16^3 FP64 970
+// and 1133, 32^3 FP64 941 and 1062, 64 x 32 x 64 mixed 900 and 955, 64 x 32 x
+// 32 FP64 1110 and 1175; 64^3 mixed 1060 and 1010, 64^3 FP64 1145 and 1023.
+constexpr int kPlaneMax = 2048, kPlaneT = 512, kPlaneP = kPlaneMax / kPlaneT;
+constexpr int kPlanePad = kPlaneMax / 4;  // most lines of a plane (axes of 4 nodes and more): one pad value each
 
 // Radix-4 butterflies on x[0..3] (span 4 q; w1, w2 the forward twiddles), as
 // dif_fwd and dit_inv form them.
@@ -1324,8 +1330,8 @@ __global__ __launch_bounds__(kPlaneT) void k2_plane(int lx, int ly, int nz, int 
                                                     double *__restrict__ y)
 {
   __shared__ cpx<T> s[kPlaneMax + kPlanePad];
-  __shared__ cpx<T> tx[512], ty[512];
-  __shared__ double cs[4 * (kPlanePad + 4)];  // cos, sin of the x and y modes
+  __shared__ cpx<T> tx[kPlanePad / 2], ty[kPlanePad / 2];
+  __shared__ double cs[2 * (kPlanePad + 4)];  // cos, sin of the x and y modes
   __shared__ double red[kHm];
   const int nx = 1 << lx, ny = 1 << ly, nxy = 1 << (lx + ly), ls = nx + 1;
   load_twiddles<T>(tx, twx, nx);
@@ -1493,41 +1499,47 @@ int fft2_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z, T *w3, b
   const bool fused = zline && w3 && ctx->zl_buf && zline_e2_applies(ctx);
   const int nx = ctx->g.nx, ny = ctx->g.ny, nz = ctx->g.nz;
   const int64_t nxy = (int64_t)nx * ny;
-  T *C = (T *)ctx->pc2_buf, *V = C + 9 * nxy, *Z = V + (kFft2Its + 1) * nxy, *w = Z + kFft2Its * nxy;
+  T *C = (T *)ctx->pc2_buf, *U = C + 9 * nxy, *Z = U + kFft2Its * nxy, *w = Z + kFft2Its * nxy;
   cpx<T> *cb = (cpx<T> *)(w + nxy);
   const H2 h = h2_layout(ctx, sizeof(T) == 4);
-  const int nb = h.nb;
-  // z-averaged residual of the first level, mean removed, into V0
+  const int nb = h.nb, nzc = lhs_zchunks(ctx->g, sizeof(T) == 4);
+  // z-averaged residual of the first level
   launch_lhs_zsum<T>(ctx, ctx->prm.lhs_type, (const T *)ctx->mom[0], z, r, h.part, h.pl, fused ? w3 : nullptr);
   Symbol sym = make_symbol(ctx, v19);
   sym.inv_scale = 1.0 / (double)nxy;
   if (nxy <= kPlaneMax) {
     hipLaunchKernelGGL((k2_plane<T>), 1, kPlaneT, 0, ctx->stream, ilog2(nx), ilog2(ny), nz,
-                       lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part, (const T *)C, Z, ctx->tw[0],
+                       nzc, (const double *)h.part, (const T *)C, Z, ctx->tw[0],
                        ctx->tw[1], sym, ctx->trig[0], ctx->trig[1], ctx->trig[2], h.y);
   } else {
-    hipLaunchKernelGGL((k2_r2<T>), nb, 256, 0, ctx->stream, nxy, nz, lhs_zchunks(ctx->g, sizeof(T) == 4), (const double *)h.part,
-                       (const double *)h.pl, h.nlb, V, h.pn);
-    const int Bx = fft2_batch<T>(nx, ny), By = fft2_batch<T>(ny, nx);
+    const int R = ny / nb, lx = ilog2(nx);
+    const size_t lds = fft_lds<T>(nx, R + 2);
+    const int By = fft2_batch<T>(ny, nx);
     for (int j = 0; j < kFft2Its; j++) {
-      T *Vj = V + (int64_t)j * nxy, *Zj = Z + (int64_t)j * nxy;
-      // Zj = F2 Vj: 2-D FFT solve with the kz = 0 symbol
-      hipLaunchKernelGGL((k_fft2_x<T, 0>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
-                         ilog2(nx), ny, Bx, Vj, cb, ctx->tw[0], (const double *)(h.pn + (int64_t)j * nb), nb);
+      T *Zj = Z + (int64_t)j * nxy;
+#define DIR(FIRST)                                                                                                  \
+  hipLaunchKernelGGL((k2_dir<T, FIRST>), nb, 256, fft_lds<T>(nx, R), ctx->stream, lx, R, nxy, j, nz, nzc,           \
+                     (const double *)h.part, (const double *)h.pl, h.nlb, U, (const T *)w, cb, ctx->tw[0], h.pn,    \
+                     (const double *)h.pd)
+      if (j == 0) DIR(true);
+      else DIR(false);
+#undef DIR
+      // 2-D FFT solve with the kz = 0 symbol: along y
       hipLaunchKernelGGL((k_fft_s<T, 3>), (unsigned)(nx / By), kBlock, fft_lds<T>(ny, By), ctx->stream, ilog2(ny),
                          (int64_t)nx, (int64_t)nx, (int64_t)0, By, cb, ctx->tw[1], sym, ctx->trig[0], ctx->trig[1],
                          ctx->trig[2]);
-      hipLaunchKernelGGL((k_fft2_x<T, 1>), (unsigned)((ny + Bx - 1) / Bx), kBlock, fft_lds<T>(nx, Bx), ctx->stream,
-                         ilog2(nx), ny, Bx, Zj, cb, ctx->tw[0], (const double *)nullptr, 0);
-      double *p1 = h.p1 + (int64_t)j * kHm * nb, *p2 = h.p2 + (int64_t)j * kHm * nb;
-      hipLaunchKernelGGL((k2_a2dots<T>), nb, 256, 0, ctx->stream, nx, ny, j, (const T *)C, (const T *)Zj,
-                         (const T *)V, w, p1, nb);
-      hipLaunchKernelGGL((k2_gs_pass<T, 1>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p1, p2, nb);
-      hipLaunchKernelGGL((k2_gs_pass<T, 2>), nb, 256, 0, ctx->stream, nxy, j, V, w, (const double *)p2,
-                         h.pn + (int64_t)(j + 1) * nb, nb);
+      if (lds <= 65536) {
+        hipLaunchKernelGGL((k2_apply<T, true>), nb, 256, lds, ctx->stream, lx, R, ny, j, (const T *)C,
+                           (const cpx<T> *)cb, ctx->tw[0], Zj, (const T *)U, w, h.pd);
+      } else {
+        const int Bx = fft2_batch<T>(nx, ny);
+        hipLaunchKernelGGL((k2_inv_x<T>), (unsigned)((ny + Bx - 1) / Bx), 256, fft_lds<T>(nx, Bx), ctx->stream, lx, ny,
+                           Bx, Zj, (const cpx<T> *)cb, ctx->tw[0]);
+        hipLaunchKernelGGL((k2_apply<T, false>), nb, 256, 0, ctx->stream, lx, R, ny, j, (const T *)C,
+                           (const cpx<T> *)cb, ctx->tw[0], Zj, (const T *)U, w, h.pd);
+      }
     }
-    hipLaunchKernelGGL(k2_solve, 1, 256, 0, ctx->stream, (const double *)h.pn, (const double *)h.p1,
-                       (const double *)h.p2, nb, h.y);
+    hipLaunchKernelGGL(k2_solve, 1, 256, 0, ctx->stream, (const double *)h.pn, nb, h.y);
   }
   if (fused) {
     launch_zline_apply_e2<T>(ctx, (const T *)ctx->zl_buf, ctx->zl_col, w3, z, (const T *)ctx->mom[0], (const T *)Z,
