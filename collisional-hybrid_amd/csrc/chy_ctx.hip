@@ -249,11 +249,14 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
     g[0] = beta;
     int64_t j = 0;
     bool done = false, ahead = false;
-    // Z_j = M^-1 U_j and A Z_j, built in place in slot j + 1
+    int dots = 0;  // partials of the U_q . w that came with the direction
+    // Z_j = M^-1 U_j and w = A Z_j, built in place in slot j + 1
     auto direction = [&](int64_t q) -> int {
-      TRY(pc_apply<T>(ctx, v19, V + q * nc, Z + q * nc));
+      T *Zq = Z + q * nc, *w = V + (q + 1) * nc;
+      TRY(pc_apply<T>(ctx, v19, V + q * nc, Zq));
       timer_start(ctx, "lhs_apply");
-      launch_lhs_apply<T, T, T>(ctx, lt, ctx->solve_transpose, n, Z + q * nc, V + (q + 1) * nc);
+      dots = ctx->solve_transpose ? 0 : launch_lhs_dots<T>(ctx, lt, n, Zq, w, (int)(q + 1), V, nc);
+      if (!dots) launch_lhs_apply<T, T, T>(ctx, lt, ctx->solve_transpose, n, Zq, w);
       timer_stop(ctx, "lhs_apply");
       return CHY_OK;
     };
@@ -279,8 +282,9 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
       const int refine = ctx->prm.ksp_gmres_cgs_refinement;
       const double sj = sc[j];
       double wn;  // |U_{j+1}| before scaling
-      launch_gs_dots<T>(ctx, (int)(j + 1), V, nc, Vn, nc, hdev, sc2);
+      if (!dots) launch_gs_dots<T>(ctx, (int)(j + 1), V, nc, Vn, nc, hdev, sc2);
       if (refine == CHY_CGS_REFINE_ALWAYS) {
+        if (dots) launch_dots_sum(ctx, (int)(j + 1), dots, hdev, sc2);
         launch_gs_update_dots<T>(ctx, (int)(j + 1), V, nc, hdev, Vn, nc, h2dev, sc2);
         launch_gs_update_norm<T>(ctx, (int)(j + 1), V, nc, h2dev, Vn, nc, ndev);
         timer_stop(ctx, "krylov");
@@ -289,7 +293,8 @@ int gmres_inner(chy_ctx *ctx, const double v19[19], const T *rhs, T *e, double r
         for (int64_t q = 0; q <= j; q++) h[q] = sc[q] > 0.0 ? (ctx->h_red[q] + ctx->h_red[(m + 2) + q]) * sj / sc[q] : 0.0;
         wn = sqrt(ctx->h_red[2 * (m + 2)]);
       } else {
-        launch_gs_update_norm<T>(ctx, (int)(j + 1), V, nc, hdev, Vn, nc, ndev);
+        if (dots) launch_gs_sum_update_norm<T>(ctx, (int)(j + 1), V, nc, dots, hdev, sc2, Vn, nc, ndev);
+        else launch_gs_update_norm<T>(ctx, (int)(j + 1), V, nc, hdev, Vn, nc, ndev);
         if (refine == CHY_CGS_REFINE_NEVER) {
           timer_stop(ctx, "krylov");
           TRY(run_ahead(j));

@@ -484,6 +484,7 @@ void k_lhs_tiled(Grid g, int lhs_type, SCoef s, LapRow lap,
 // 72 and FP64 99 -> 199.  col_stencil draws the line between them.  Four planes
 // a group measured best or level for both types (1, 2, 4 and 8 tried).
 constexpr int kColZ = 4;
+constexpr int kColDots = 8;  // most dot products taken with A x
 static inline bool col_stencil(const Grid &g, bool fp32) { return g.nc <= (fp32 ? (int64_t)1 << 23 : (int64_t)1 << 21); }
 
 // Planes per chunk: 1024 blocks of columns, in whole groups, at most kZChunk
@@ -572,10 +573,12 @@ __device__ __forceinline__ T ld_off(const T *__restrict__ base, uint32_t byte_of
 template <typename TN, typename TX, typename TY, typename C, bool DIFF, int OUT, typename TB, int OP>
 __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow lap, const TN *__restrict__ n,
                                                  const TX *__restrict__ x, const TB *__restrict__ b,
-                                                 TY *__restrict__ y, double *__restrict__ pl, TX *__restrict__ d3)
+                                                 TY *__restrict__ y, double *__restrict__ pl, TX *__restrict__ d3,
+                                                 int nv, int64_t vs)
 {
   constexpr bool ZS = OUT == 2 || OUT == 4, KZ = OP == kOpKz;
   constexpr int ZR = kColZ;
+  double dots[OUT == 5 ? kColDots : 1] = {};
   uint32_t bx, by, bz;
   const uint32_t tile = xcd_tile(bx, by, bz);
   const int64_t pstride = (int64_t)g.nx * g.ny;
@@ -624,23 +627,43 @@ __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow
             nf[v][2] = (C)ld_off(np, cyp * (uint32_t)sizeof(TN));
             nf[v][3] = (C)ld_off(np, cym * (uint32_t)sizeof(TN));
           }
-          if (OUT != 0) rb[v] = ld_off(b + pb, c0 * (uint32_t)sizeof(TB));
+          if (OUT != 0 && OUT != 5) rb[v] = ld_off(b + pb, c0 * (uint32_t)sizeof(TB));
         }
       }
+      TY yv[ZR];
 #pragma unroll
       for (int v = 0; v < ZR; v++) {
         const int u = v + 1, k = k0 + v;
+        if (OUT == 5) yv[v] = (TY)0;
         if (k >= z1) break;
         const C acc = row_apply<C, DIFF, OP>(s, lap, nc[u], nf[v], nc[u + 1], nc[u - 1], xc[u], xf[u], xe[v], xc[u + 1],
                                              xc[u - 1], xf[u + 1], xf[u - 1]);
         const int64_t c = (int64_t)c0 + pstride * k;
-        if (OUT == 0) y[c] = (TY)acc;
-        else {
+        if (OUT == 0 || OUT == 5) {
+          y[c] = (TY)acc;
+          yv[v] = (TY)acc;
+        } else {
           const double rv = (double)rb[v] - (double)acc;
           if (OUT == 1 || OUT == 3) y[c] = (TY)rv;
           if (OUT == 4) d3[c] = (TX)rv;
           if (ZS) zs += rv;
           if (OUT == 3) zs += rv * rv;
+        }
+      }
+      if (OUT == 5) {
+#pragma unroll
+        for (int q = 0; q < kColDots; q++) {
+          if (q < nv) {
+            TB bv[ZR];
+#pragma unroll
+            for (int v = 0; v < ZR; v++) {
+              const int k = k0 + v < z1 ? k0 + v : z1 - 1;  // (past the chunk: yv is 0)
+              bv[v] = ld_off(b + q * vs + pstride * k, c0 * (uint32_t)sizeof(TB));
+            }
+#pragma unroll
+            for (int v = 0; v < ZR; v++)
+              if (k0 + v < z1) dots[q] += (double)bv[v] * (double)yv[v];
+          }
         }
       }
     }
@@ -654,6 +677,22 @@ __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0) pl[tile] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+  }
+  if (OUT == 5) {
+    __shared__ double dsum[4][kColDots];
+#pragma unroll
+    for (int q = 0; q < kColDots; q++) {
+      if (q < nv) {
+        double t = dots[q];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+        if ((threadIdx.x & 63) == 0) dsum[threadIdx.x >> 6][q] = t;
+      }
+    }
+    __syncthreads();
+    if (threadIdx.x < nv)
+      pl[(int64_t)tile * nv + threadIdx.x] = ((dsum[0][threadIdx.x] + dsum[1][threadIdx.x]) + dsum[2][threadIdx.x]) +
+                                             dsum[3][threadIdx.x];
   }
 }
 
@@ -690,19 +729,20 @@ static inline bool kz_operator(int lhs_type, const SCoef &s)
 // one; the B-along-z instantiation when it applies.
 template <typename TN, typename TX, typename TY, typename C, bool DIFF, int OUT, typename TB = double, int TW = kTX>
 static void launch_tiled_on(chy_ctx *ctx, const Grid &g, const SCoef &s, const LapRow &L, int lhs_type, const TN *n,
-                            const TX *x, const TB *b, TY *y, double *pl, TX *d3 = nullptr)
+                            const TX *x, const TB *b, TY *y, double *pl, TX *d3 = nullptr, int nv = 0, int64_t vs = 0)
 {
-  if (col_stencil(g, sizeof(C) == 4)) {
+  if (OUT == 5 || col_stencil(g, sizeof(C) == 4)) {
 #define COLK(OP)                                                                                                  \
   hipLaunchKernelGGL((k_lhs_col<TN, TX, TY, C, DIFF, OUT, TB, OP>), col_grid(g), 256, 0, ctx->stream, g, col_chunk(g), \
-                     s, L, n, x, b, y, pl, d3)
+                     s, L, n, x, b, y, pl, d3, nv, vs)
     if (kz_operator(lhs_type, s)) COLK(kOpKz);
     else if (lhs_type == CHY_LHS_FULL) COLK(kOpFull);
     else COLK(kOpConst);
 #undef COLK
     return;
   }
-  if (kz_operator(lhs_type, s))
+  if constexpr (OUT == 5) return;
+  else if (kz_operator(lhs_type, s))
     hipLaunchKernelGGL((k_lhs_tiled<TN, TX, TY, C, DIFF, OUT, TB, TW, true>), tiled_grid(g, TW), kBlock, 0,
                        ctx->stream, g, lhs_type, s, L, n, x, b, y, pl, d3);
   else
@@ -739,6 +779,25 @@ void launch_lhs_apply(chy_ctx *ctx, int lhs_type, bool transpose, const TN *n, c
   else
     launch_tiled<TN, TX, TY, C, fp32, 0>(ctx, lhs_type, n, x, (const double *)nullptr, y, (double *)nullptr);
 }
+
+// y = A x with one partial of V_q . y, q < nv, per block in ctx->red; returns
+// the number of partials, or 0 with nothing launched where the column kernel
+// does not run or would leave more of them than the reduction buffer takes.
+template <typename T>
+int launch_lhs_dots(chy_ctx *ctx, int lhs_type, const T *n, const T *x, T *y, int nv, const T *V, int64_t stride)
+{
+  constexpr bool fp32 = sizeof(T) == 4;
+  using C = typename std::conditional<fp32, float, double>::type;
+  const Grid &g = ctx->g;
+  const dim3 d = col_grid(g);
+  if (nv > kColDots || !col_stencil(g, fp32) || (int64_t)d.x * d.y > kRedBlocks) return 0;
+  const SCoef s = full_scoef(ctx->prm.d, ctx->prm.kappa_e);
+  const LapRow L = lap_row(ctx, lhs_type);
+  launch_tiled_on<T, T, T, C, fp32, 5, T>(ctx, g, s, L, lhs_type, n, x, V, y, ctx->red, nullptr, nv, stride);
+  return (int)(d.x * d.y);
+}
+template int launch_lhs_dots<double>(chy_ctx *, int, const double *, const double *, double *, int, const double *, int64_t);
+template int launch_lhs_dots<float>(chy_ctx *, int, const float *, const float *, float *, int, const float *, int64_t);
 
 int lhs_zchunks(const Grid &g, bool fp32)
 {
@@ -1295,15 +1354,43 @@ __global__ __launch_bounds__(256) void k_mdot4(int nv, const T *__restrict__ A, 
 }
 
 // w -= sum_k h_k V_k, then partial[blk*nv + k] = V_k . w (of the new w), or
-// with NORM the partial of ||w||^2 instead
-template <typename T, int NV, bool NORM>
+// with NORM the partial of ||w||^2 instead.  SUM: h_k is the sum of the nblk
+// partials h[b*nv + k] times sc.s[k], made by every block in the same order;
+// block 0 leaves them in out and its mirror, as k_combine does.
+template <typename T, int NV, bool NORM, bool SUM = false>
 __global__ __launch_bounds__(256) void k_gs4(int nv, const T *__restrict__ V, int64_t stride,
                                              const double *__restrict__ h, T *__restrict__ w, int64_t n4,
-                                             double *__restrict__ partial)
+                                             double *__restrict__ partial, int nblk, DotScale sc,
+                                             double *__restrict__ out, double *__restrict__ mirror)
 {
   __shared__ double hs[NV];
   __shared__ double sh[4][NORM ? 1 : NV];
-  if (threadIdx.x < nv) hs[threadIdx.x] = h[threadIdx.x];
+  if (SUM) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int k0 = 0; k0 < NV; k0 += 4) {
+      const int k = k0 + (threadIdx.x >> 6);
+      if (k < nv) {
+        double t = 0.0;
+#pragma unroll 4
+        for (int b = lane; b < nblk; b += 64) t += h[(int64_t)b * nv + k];
+        t = wave_sum(t);
+        if (lane == 0) {
+          const double v = t * sc.s[k];
+          hs[k] = v;
+          if (blockIdx.x == 0) {
+            out[k] = v;
+            if (mirror) {
+              mirror[k] = v;
+              __threadfence_system();
+            }
+          }
+        }
+      }
+    }
+  } else if (threadIdx.x < nv) {
+    hs[threadIdx.x] = h[threadIdx.x];
+  }
   __syncthreads();
   double acc[NORM ? 1 : NV];
 #pragma unroll
@@ -1374,7 +1461,8 @@ void launch_gs_update_dots(chy_ctx *ctx, int nv, const T *V, int64_t stride, con
   }
   const int64_t n4 = n / 4;
   const unsigned nb = (unsigned)std::min<int64_t>(kRedBlocks, (n4 + kBlock - 1) / kBlock);
-  hipLaunchKernelGGL((k_gs4<T, 8, false>), nb, kBlock, 0, ctx->stream, nv, V, stride, h, w, n4, ctx->red);
+  hipLaunchKernelGGL((k_gs4<T, 8, false>), nb, kBlock, 0, ctx->stream, nv, V, stride, h, w, n4, ctx->red, 0, DotScale(),
+                     (double *)nullptr, (double *)nullptr);
   combine(ctx, ctx->red, (int)nb, nv, out_dev, scale);
 }
 
@@ -1385,9 +1473,47 @@ void launch_gs_update_norm(chy_ctx *ctx, int nv, const T *V, int64_t stride, con
   if (nv > kMaxDots || !quad_ok(n, stride, V, w)) { launch_mgs_norm<T>(ctx, nv, V, stride, h, w, n, norm2_dev); return; }
   const int64_t n4 = n / 4;
   const unsigned nb = (unsigned)std::min<int64_t>(kRedBlocks, (n4 + kBlock - 1) / kBlock);
-  GS_NV(nv, hipLaunchKernelGGL((k_gs4<T, NV, true>), nb, kBlock, 0, ctx->stream, nv, V, stride, h, w, n4, ctx->red));
+  GS_NV(nv, hipLaunchKernelGGL((k_gs4<T, NV, true>), nb, kBlock, 0, ctx->stream, nv, V, stride, h, w, n4, ctx->red, 0,
+                               DotScale(), (double *)nullptr, (double *)nullptr));
   combine(ctx, ctx->red, (int)nb, 1, norm2_dev);
 }
+
+// The dots of launch_lhs_dots' nblk partials, scaled, to out_dev
+void launch_dots_sum(chy_ctx *ctx, int nv, int nblk, double *out_dev, const double *scale)
+{
+  combine(ctx, ctx->red, nblk, nv, out_dev, scale);
+}
+
+// The same, w -= V out and ||w||^2: the update adds the partials itself, in
+// every block.  With the dots taken where w is made, that is two launches of
+// 4.5 us an iteration fewer, for 1 to 3 us more in each of the two kernels.  us
+// of a solve, dots and their sum as launches of their own -> here: 32^3 FP64 926
+// -> 896, 64^3 mixed 1030 -> 994 and FP64 1030 -> 996, 64 x 128 x 64 mixed 1062
+// -> 1025, 128^3 FP64 2075 -> 1985 (2020 with the sum as a launch), mixed 1580
+// -> 1535.
+template <typename T>
+void launch_gs_sum_update_norm(chy_ctx *ctx, int nv, const T *V, int64_t stride, int nblk, double *out_dev,
+                               const double *scale, T *w, int64_t n, double *norm2_dev)
+{
+  if (!quad_ok(n, stride, V, w)) {
+    launch_dots_sum(ctx, nv, nblk, out_dev, scale);
+    launch_gs_update_norm<T>(ctx, nv, V, stride, out_dev, w, n, norm2_dev);
+    return;
+  }
+  const int64_t n4 = n / 4;
+  const unsigned nb = (unsigned)std::min<int64_t>(kRedBlocks, (n4 + kBlock - 1) / kBlock);
+  DotScale sc;
+  sc.on = 1;
+  for (int k = 0; k < kMaxDots; k++) sc.s[k] = k < nv ? scale[k] : 1.0;
+  double *norms = ctx->red + (int64_t)kColDots * kRedBlocks;  // (the dots' partials are read meanwhile)
+  hipLaunchKernelGGL((k_gs4<T, 8, true, true>), nb, kBlock, 0, ctx->stream, nv, V, stride, (const double *)ctx->red, w,
+                     n4, norms, nblk, sc, out_dev, mirror_of(ctx, out_dev, nv));
+  combine(ctx, norms, (int)nb, 1, norm2_dev);
+}
+template void launch_gs_sum_update_norm<double>(chy_ctx *, int, const double *, int64_t, int, double *, const double *,
+                                                double *, int64_t, double *);
+template void launch_gs_sum_update_norm<float>(chy_ctx *, int, const float *, int64_t, int, double *, const double *,
+                                               float *, int64_t, double *);
 
 template <typename T>
 __global__ __launch_bounds__(256) void k_axpby(int64_t n, double a, const T *__restrict__ x, double b, T *__restrict__ y)

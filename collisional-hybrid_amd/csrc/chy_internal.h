@@ -323,6 +323,14 @@ void launch_gs_update_dots(chy_ctx *ctx, int nv, const T *V, int64_t stride, con
 template <typename T>
 void launch_gs_update_norm(chy_ctx *ctx, int nv, const T *V, int64_t stride, const double *h, T *w, int64_t n,
                            double *norm2_dev);
+// y = A x with the partials of V_q . y, q < nv (returns how many, 0: not done);
+// their sums, scaled, to out_dev; the sums, w -= V out and ||w||^2
+template <typename T>
+int launch_lhs_dots(chy_ctx *ctx, int lhs_type, const T *n, const T *x, T *y, int nv, const T *V, int64_t stride);
+void launch_dots_sum(chy_ctx *ctx, int nv, int nblk, double *out_dev, const double *scale);
+template <typename T>
+void launch_gs_sum_update_norm(chy_ctx *ctx, int nv, const T *V, int64_t stride, int nblk, double *out_dev,
+                               const double *scale, T *w, int64_t n, double *norm2_dev);
 template <typename T>
 void launch_axpby(chy_ctx *ctx, int64_t n, double a, const T *x, double b, T *y);
 template <typename TS, typename TD>

@@ -92,6 +92,30 @@ def test_fft_passes_on_axes_of_any_length(N, extra, prec, base):
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
 
 
+# an iteration's dot products come with A z for at most 8 basis vectors, on grids
+# of the column stencil, and are added in the update's kernel where nodes come
+# in fours: 12 iterations (past 8 vectors) on node counts that are and are not
+# multiples of 4, ragged last blocks, and every kind of row; against a solve
+# that takes a second Gram-Schmidt pass and so the separate kernels.  Two
+# converged solves at this tolerance differ by it times the conditioning of the
+# preconditioned operator (below 100), and by the FP64 residual's rounding.
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("N,extra", [((3, 3, 3), "-pc_type jacobi"), ((5, 7, 3), "-pc_type jacobi"),
+                                     ((17, 16, 6), "-pc_type zline"), ((17, 15, 9), "-pc_type zline -B0x 1e-5 -B0y 2e-5"),
+                                     ((16, 16, 8), "-pc_type fft"), ((32, 32, 32), "-pc_type fft -B0x 1e-5 -B0y 2e-5")])
+def test_gmres_dot_products_with_the_operator(N, extra, prec):
+    phis = []
+    for refine in ("NEVER", "ALWAYS"):
+        with context(opts(N, extra=f"{extra} -ksp_rtol 1e-11 -precision {prec} -ksp_max_it 2000 "
+                                   f"-ksp_gmres_cgs_refinement_type REFINE_{refine}")) as ctx:
+            g = grid_of(ctx.prm)
+            ctx.set_moments(vlasov_from(_moments(g, np.random.default_rng(19))))
+            phi, st = ctx.solve_potential()
+            assert st.converged == 1 and st.residual <= 1e-11, (refine, st.iterations, st.residual)
+            phis.append(phi)
+    assert np.abs(phis[0] - phis[1]).max() <= 2e-9 * np.abs(phis[1]).max()
+
+
 # the next direction is launched before the present one's dot products are read,
 # except where the cycle, the iteration limit or the expected convergence ends
 # it: each end of a cycle against the oracle's iterate after as many steps (in
