@@ -2502,8 +2502,8 @@ MG_INST(float)
 #undef MG_INST
 
 // Both once-per-solve column walks of the two-level preconditioners for the
-// full operator (COEF: k_zcoef's z-means, FACT: k_zline_factor's factors,
-// the same arithmetic in the same order), in one walk up each column with the
+// full operator on columns beyond 256 planes (COEF: k_zcoef's z-means, FACT:
+// k_zline_factor's factors, the same arithmetic in the same order), in one walk up each column with the
 // density star of KC planes loaded before any is used; the back sweep of the
 // Sherman-Morrison vector reads KC planes at a time too.
 template <typename T, bool COEF, bool FACT>
@@ -2592,11 +2592,200 @@ __global__ __launch_bounds__(256) void k_zcolumn(Grid g, SCoef s, const T *__res
   }
 }
 
+// The same with the columns cut into segments, as k_zline_seg: NC consecutive
+// columns a block, SG segments of P planes each, a thread a segment, whose rows
+// stay in registers.  The pivots follow cp_k = c_k / (b_k - a_k cp_(k-1)), a
+// fractional linear recurrence: a thread composes the 2x2 maps of its planes
+// (rows scaled by 1/b, so the products stay between 0 and 1 in size), runs
+// through the maps before it as a vector (num, den), and takes its planes with
+// the sequential formulas; the Sherman-Morrison vector and its back sweep are
+// first-order linear recurrences treated alike.  us, one thread a column (bound by
+// the serial chain of divisions and the few blocks) -> segments: 32^3 FP64 31 ->
+// 6.5, 64^3 FP64 61 -> 11.4 and FP32 58 -> 10.8, 128^3 FP64 122 -> 29 and FP32
+// 112 -> 27, 128 x 128 x 256 FP64 241 -> 71, 256^3 FP64 317 -> 296 and FP32 260 ->
+// 187 (the stores of the four factors); factors alone, 64 x 48 x 40 FP64 34 -> 7.8,
+// 96 x 80 x 50 FP32 41 -> 8.3.  More than 8 planes a thread spill; beyond 128
+// planes 32 columns a block (239 us with 16 at 256^3 FP32), below 16 (29 and 34
+// us at 128^3 FP64).  Columns beyond 256 planes keep the walk.
+template <typename T, int NC, int SG, int P, bool COEF, bool FACT>
+__global__ __launch_bounds__(NC * SG) void k_zcolumn_seg(Grid g, SCoef s, const T *__restrict__ n, T *__restrict__ Cz,
+                                                         T *__restrict__ za, T *__restrict__ zi, T *__restrict__ zc,
+                                                         T *__restrict__ zq, double *__restrict__ cag,
+                                                         double *__restrict__ cden)
+{
+  constexpr int kMaps = FACT ? 4 : 0, kSums = COEF ? 9 : 0;
+  __shared__ double sh[kMaps > kSums ? kMaps : kSums][SG][NC], ends[4][NC];
+  uint32_t bx, by, bz;
+  (void)xcd_tile(bx, by, bz);
+  const int plane = g.nx * g.ny, m = g.nz, cx = threadIdx.x % NC, sg = threadIdx.x / NC, k0 = sg * P;
+  const int col = (int)bx * NC + cx;
+  const bool live = col < plane;
+  int i, j, k_;
+  split_cell(g, live ? col : 0, i, j, k_);
+  const int c0 = i + g.nx * j;
+  const int oxp = (i + 1 == g.nx ? 0 : i + 1) + g.nx * j, oxm = (i == 0 ? g.nx - 1 : i - 1) + g.nx * j;
+  const int oyp = i + g.nx * (j + 1 == g.ny ? 0 : j + 1), oym = i + g.nx * (j == 0 ? g.ny - 1 : j - 1);
+  // rows of the thread's planes (loads past the last plane read a valid value that is not used)
+  double a[P], b[P], c[P];
+  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  {
+    T nz_[P + 2], xp[P], xm[P], yp[P], ym[P];
+#pragma unroll
+    for (int u = 0; u < P + 2; u++) nz_[u] = n[c0 + (int64_t)plane * wrapi(k0 - 1 + u < m + 1 ? k0 - 1 + u : m, m)];
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      const int64_t pk = (int64_t)plane * (k0 + u < m ? k0 + u : m - 1);
+      xp[u] = n[oxp + pk]; xm[u] = n[oxm + pk]; yp[u] = n[oyp + pk]; ym[u] = n[oym + pk];
+    }
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      double v[19];
+      row_from_star<double>(s, (double)nz_[u + 1], (double)xp[u], (double)xm[u], (double)yp[u], (double)ym[u],
+                            (double)nz_[u + 2], (double)nz_[u], v);
+      a[u] = v[5]; b[u] = v[18]; c[u] = v[4];
+      if (COEF && k0 + u < m) {
+        constexpr int grp[19] = {5, 3, 7, 1, 4, 4, 8, 2, 6, 0, 5, 5, 3, 3, 7, 7, 1, 1, 4};  // kGroup19
+#pragma unroll
+        for (int q = 0; q < 19; q++) acc[grp[q]] += v[q];
+      }
+    }
+  }
+  if (COEF) {
+#pragma unroll
+    for (int q = 0; q < 9; q++) sh[q][sg][cx] = acc[q];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 9 * NC; e += NC * SG) {
+      const int q = e / NC, cc = e % NC, cq = (int)bx * NC + cc;
+      double t = 0.0;
+#pragma unroll
+      for (int r = 0; r < SG; r++) t += sh[q][r][cc];
+      if (cq < plane) Cz[(int64_t)q * plane + cq] = (T)(t / (double)m);
+    }
+    __syncthreads();
+  }
+  if constexpr (FACT) {
+    // the periodic corner: gamma = -b_0, b_0 -= gamma, b_(m-1) -= c_(m-1) a_0 / gamma
+    if (sg == 0) { ends[0][cx] = a[0]; ends[1][cx] = b[0]; }
+    __syncthreads();
+    const double a0 = ends[0][cx], gm = -ends[1][cx];
+    if (sg == 0) b[0] = b[0] - gm;
+#pragma unroll
+    for (int u = 0; u < P; u++)
+      if (k0 + u == m - 1) b[u] = b[u] - c[u] * a0 / gm;
+    double m00 = 1.0, m01 = 0.0, m10 = 0.0, m11 = 1.0;
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      if (k0 + u < m) {
+        const double ib = 1.0 / b[u], ch = c[u] * ib, ah = a[u] * ib;
+        const double t0 = m10 - ah * m00, t1 = m11 - ah * m01;
+        m00 = ch * m10; m01 = ch * m11;
+        m10 = t0; m11 = t1;
+      }
+    }
+    sh[0][sg][cx] = m00; sh[1][sg][cx] = m01; sh[2][sg][cx] = m10; sh[3][sg][cx] = m11;
+    __syncthreads();
+    double num = 0.0, den = 1.0;
+    for (int t = 0; t < sg; t++) {
+      const double x = sh[0][t][cx] * num + sh[1][t][cx] * den;
+      den = sh[2][t][cx] * num + sh[3][t][cx] * den;
+      num = x;
+    }
+    __syncthreads();  // (the maps are read)
+    double cp = num / den, A = 1.0, B = 0.0, iv[P], q[P];
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      iv[u] = 0.0;
+      q[u] = 0.0;
+      if (k0 + u < m) {
+        const double dn = b[u] - a[u] * cp;
+        iv[u] = 1.0 / dn;
+        const double uk = k0 + u == 0 ? gm : (k0 + u == m - 1 ? c[u] : 0.0);
+        cp = c[u] / dn;
+        c[u] = cp;
+        q[u] = uk * iv[u];
+        const double al = -a[u] * iv[u];
+        A = al * A;
+        B = al * B + q[u];
+      }
+    }
+    sh[0][sg][cx] = A;
+    sh[1][sg][cx] = B;
+    __syncthreads();
+    double y = 0.0;
+    for (int t = 0; t < sg; t++) y = sh[0][t][cx] * y + sh[1][t][cx];
+#pragma unroll
+    for (int u = 0; u < P; u++) {
+      if (k0 + u < m) {
+        y = q[u] - a[u] * iv[u] * y;
+        q[u] = y;
+      }
+    }
+    if (sg == (m - 1) / P) ends[2][cx] = y;
+    // the back sweep x_(m-1) = q_(m-1), x_k = q_k - cp_k x_(k+1)
+    A = 1.0; B = 0.0;
+#pragma unroll
+    for (int u = P - 1; u >= 0; u--) {
+      if (k0 + u == m - 1) { A = 0.0; B = q[u]; }
+      else if (k0 + u < m - 1) { B = q[u] - c[u] * B; A = -c[u] * A; }
+    }
+    sh[2][sg][cx] = A;
+    sh[3][sg][cx] = B;
+    __syncthreads();
+    double x = 0.0;
+    for (int t = SG - 1; t > sg; t--) x = sh[2][t][cx] * x + sh[3][t][cx];
+#pragma unroll
+    for (int u = P - 1; u >= 0; u--) {
+      if (k0 + u < m) {
+        x = k0 + u == m - 1 ? q[u] : q[u] - c[u] * x;
+        q[u] = x;
+      }
+    }
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < P; u++) {
+        if (k0 + u < m) {
+          const int64_t e = col + (int64_t)plane * (k0 + u);
+          za[e] = (T)a[u]; zi[e] = (T)iv[u]; zc[e] = (T)c[u]; zq[e] = (T)q[u];
+        }
+      }
+      if (sg == 0) {
+        const double ag = a0 / gm;
+        cag[col] = ag;
+        cden[col] = 1.0 + x + ag * ends[2][cx];
+      }
+    }
+  }
+}
+
+// The segmented factors of the full operator on grid g where a block holds its
+// columns; false: it does not.
+template <typename T, bool COEF, bool FACT>
+static bool launch_zcolumn_seg(chy_ctx *ctx, const Grid &g, const SCoef &s, const T *n, T *Cz, T *zbuf, double *colbuf)
+{
+  const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
+  if (g.nz > 256) return false;
+#define ZFAC(NC, SG, P)                                                                                                \
+  hipLaunchKernelGGL((k_zcolumn_seg<T, NC, SG, P, COEF, FACT>), (unsigned)((plane + NC - 1) / NC), NC * SG, 0,         \
+                     ctx->stream, g, s, n, Cz, zbuf, FACT ? zbuf + nc : zbuf, FACT ? zbuf + 2 * nc : zbuf,             \
+                     FACT ? zbuf + 3 * nc : zbuf, colbuf, FACT ? colbuf + plane : colbuf)
+  if (g.nz <= 32) ZFAC(16, 8, 4);
+  else if (g.nz <= 64) ZFAC(16, 8, 8);
+  else if (g.nz <= 128) ZFAC(16, 16, 8);
+  else ZFAC(32, 32, 8);
+#undef ZFAC
+  return true;
+}
+
 template <typename T>
 void launch_zcolumn(chy_ctx *ctx, const T *n, T *Cz, T *zbuf, double *colbuf)
 {
   const SCoef s = full_scoef(ctx->prm.d, ctx->prm.kappa_e);
   const int64_t nc = ctx->g.nc, plane = (int64_t)ctx->g.nx * ctx->g.ny;
+  const bool seg = Cz && zbuf ? launch_zcolumn_seg<T, true, true>(ctx, ctx->g, s, n, Cz, zbuf, colbuf)
+                   : Cz       ? launch_zcolumn_seg<T, true, false>(ctx, ctx->g, s, n, Cz, zbuf, colbuf)
+                   : zbuf     ? launch_zcolumn_seg<T, false, true>(ctx, ctx->g, s, n, Cz, zbuf, colbuf)
+                              : true;
+  if (seg) return;
   T *z4[4] = {zbuf, zbuf ? zbuf + nc : nullptr, zbuf ? zbuf + 2 * nc : nullptr, zbuf ? zbuf + 3 * nc : nullptr};
   double *c2[2] = {colbuf, colbuf ? colbuf + plane : nullptr};
 #define ZCOL(A, B)                                                                                              \
@@ -2686,6 +2875,7 @@ void launch_zline_factor_g(chy_ctx *ctx, const Grid &g, const double d[3], int l
   LapRow L;
   uniform_row(lhs_type == CHY_LHS_FULL ? CHY_LHS_IDENTITY : lhs_type, d, ctx->prm.kappa_e, 0.0, L.v);
   const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
+  if (lhs_type == CHY_LHS_FULL && launch_zcolumn_seg<T, false, true>(ctx, g, s, n, nullptr, zbuf, colbuf)) return;
   hipLaunchKernelGGL((k_zline_factor<T>), nblocks(plane), kBlock, 0, ctx->stream, g, lhs_type, s, L, n, zbuf,
                      zbuf + nc, zbuf + 2 * nc, zbuf + 3 * nc, colbuf, colbuf + plane);
 }
