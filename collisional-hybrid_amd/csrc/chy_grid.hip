@@ -2198,8 +2198,8 @@ __global__ __launch_bounds__(NC * SG) void k_zline_seg(Grid g, const T *__restri
 // The multigrid keeps its level fields as [y][x][z]: a group of W lanes owns a
 // column, P consecutive planes a lane (W P >= nz), so that the stencil around a
 // column, the column's z-line system and its solve are contiguous loads and
-// shuffles.  A smoothing sweep is then one launch, x' = x + omega zline^-1 (b -
-// A x), the residual never stored: 6.0 us on 96 x 80 x 50 and 5 on its coarse
+// register moves.  A smoothing sweep is then one launch, x' = x + omega zline^-1 (b
+// - A x), the residual never stored: 4 to 6 us on 96 x 80 x 50 and its coarse
 // levels (FP32), where with x fastest it took a residual pass (4 to 6 us) and a
 // solve (16.6 us walking 96 x 80 columns, 4.6 us on fewer).  A preconditioner
 // application there went from 65 launches to 43.  Whole solves: 96 x 80 x 50
@@ -2254,6 +2254,62 @@ __device__ __forceinline__ void wave_sync()
   __builtin_amdgcn_wave_barrier();
 }
 
+// x of the lane that CTRL (a DPP control) names, other where there is none in
+// the row of 16 lanes (or, for a shift of the whole wave, in the wave)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x, double other)
+{
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(x), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(x), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_value(double x, int l)  // l: the same in every lane
+{
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+
+// Inclusive scan of the affine maps y -> A y + B over groups of W lanes, lower
+// lanes' maps first (UP) or higher lanes' first: four register moves within the
+// rows of 16 lanes, then the row totals of the rows before it.  (Six shuffles
+// of each value through LDS made a sweep take 5.3 us on 64 x 48 x 40 FP64 and 5.6
+// on 96 x 80 x 50 FP32, which now takes 4.5 and 4.9; a solve there 13.2 -> 12.4
+// and 14.9 -> 14.2 ms.)
+template <bool UP, int W>
+__device__ __forceinline__ void affine_scan(double &A, double &B)
+{
+  auto step = [&](auto n) {
+    constexpr int ctrl = (UP ? 0x110 : 0x100) + decltype(n)::value;  // row_shr:n, row_shl:n
+    const double A2 = dpp_move<ctrl>(A, 1.0), B2 = dpp_move<ctrl>(B, 0.0);
+    B = A * B2 + B;
+    A = A * A2;
+  };
+  step(std::integral_constant<int, 1>());
+  step(std::integral_constant<int, 2>());
+  step(std::integral_constant<int, 4>());
+  step(std::integral_constant<int, 8>());
+  if constexpr (W > 16) {
+    const int row = (int)(threadIdx.x & 63) >> 4;
+    // the maps of whole rows, in the order in which they apply: rows 0, 1, 2 (UP) or 3, 2, 1
+    const double a0 = lane_value(A, UP ? 15 : 48), b0 = lane_value(B, UP ? 15 : 48);
+    const double a2 = lane_value(A, UP ? 47 : 16), b2 = lane_value(B, UP ? 47 : 16);
+    double a = 1.0, b = 0.0;
+    if constexpr (W == 32) {
+      if (UP) { if (row & 1) { a = row == 1 ? a0 : a2; b = row == 1 ? b0 : b2; } }
+      else if (!(row & 1)) { a = row == 2 ? a0 : a2; b = row == 2 ? b0 : b2; }
+    } else {
+      const double a1 = lane_value(A, UP ? 31 : 32), b1 = lane_value(B, UP ? 31 : 32);
+      const double a10 = a1 * a0, b10 = a1 * b0 + b1, a210 = a2 * a10, b210 = a2 * b10 + b2;
+      const int after = UP ? row : 3 - row;  // rows whose maps come first
+      a = after == 0 ? 1.0 : after == 1 ? a0 : after == 2 ? a10 : a210;
+      b = after == 0 ? 0.0 : after == 1 ? b0 : after == 2 ? b10 : b210;
+    }
+    B = A * b + B;
+    A = A * a;
+  }
+}
+
 // The cyclic z-line solve of the column held by W lanes (lane L: planes L P ..
 // L P + P - 1), r in and the solution in r.  The forward and back
 // substitutions are first-order linear recurrences, y_k = alpha_k y_(k-1) +
@@ -2273,12 +2329,8 @@ __device__ __forceinline__ void zline_lanes(int L, int m, double (&r)[P], const 
       B = al * B + be;
     }
   }
-#pragma unroll
-  for (int off = 1; off < W; off <<= 1) {  // inclusive scan: lower lanes' maps first
-    const double A2 = __shfl_up(A, off, W), B2 = __shfl_up(B, off, W);
-    if (L >= off) { B = A * B2 + B; A = A * A2; }
-  }
-  double yv = __shfl_up(B, 1, W);  // the exclusive prefix applied to y_(-1) = 0
+  affine_scan<true, W>(A, B);
+  double yv = dpp_move<0x138>(B, 0.0);  // (wave_shr:1) the exclusive prefix applied to y_(-1) = 0
   if (L == 0) yv = 0.0;
 #pragma unroll
   for (int u = 0; u < P; u++) {
@@ -2287,7 +2339,7 @@ __device__ __forceinline__ void zline_lanes(int L, int m, double (&r)[P], const 
       r[u] = yv;
     }
   }
-  const double ylast = __shfl(yv, (m - 1) / P, W);
+  const double ylast = W == 64 ? lane_value(yv, (m - 1) / P) : __shfl(yv, (m - 1) / P, W);
   // backward: x_(m-1) = y_(m-1), x_k = y_k - c_k x_(k+1); higher planes first
   A = 1.0; B = 0.0;
 #pragma unroll
@@ -2296,12 +2348,8 @@ __device__ __forceinline__ void zline_lanes(int L, int m, double (&r)[P], const 
     if (k == m - 1) { A = 0.0; B = ylast; }
     else if (k < m - 1) { B = -c[u] * B + r[u]; A = -c[u] * A; }
   }
-#pragma unroll
-  for (int off = 1; off < W; off <<= 1) {  // higher lanes' maps first
-    const double A2 = __shfl_down(A, off, W), B2 = __shfl_down(B, off, W);
-    if (L + off < W) { B = A * B2 + B; A = A * A2; }
-  }
-  double xv = __shfl_down(B, 1, W);
+  affine_scan<false, W>(A, B);
+  double xv = dpp_move<0x130>(B, 0.0);  // (wave_shl:1)
   if (L == W - 1) xv = 0.0;
 #pragma unroll
   for (int u = P - 1; u >= 0; u--) {
@@ -2309,7 +2357,7 @@ __device__ __forceinline__ void zline_lanes(int L, int m, double (&r)[P], const 
     if (k == m - 1) xv = ylast;
     else if (k < m - 1) { xv = r[u] - c[u] * xv; r[u] = xv; }
   }
-  const double f = (__shfl(xv, 0, W) + cag * ylast) / cden;
+  const double f = ((W == 64 ? lane_value(xv, 0) : __shfl(xv, 0, W)) + cag * ylast) / cden;
 #pragma unroll
   for (int u = 0; u < P; u++) r[u] -= f * q[u];
 }
