@@ -271,6 +271,29 @@ __device__ __forceinline__ float mean_rel_speed_f(float vx, float vy, float vz, 
 // ---- wave-level helpers (64-wide wavefronts) -----------------------------------
 __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
+// Orders a wave's own LDS accesses (which the hardware keeps in order)
+__device__ __forceinline__ void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// x of the lane that CTRL (a DPP control) names, other where there is none in
+// the row of 16 lanes (or, for a shift of the whole wave, in the wave)
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double x, double other)
+{
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(x), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(x), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double lane_value(double x, int l)  // l: the same in every lane
+{
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                          __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+
 // Run-length aggregation of integer atomics over lanes holding equal keys in
 // consecutive lanes: returns, for each active lane, (head lane, run length).
 // Inactive lanes must pass key = -1.

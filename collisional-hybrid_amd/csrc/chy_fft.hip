@@ -596,8 +596,9 @@ __device__ __forceinline__ void dftR(cpx<T> (&v)[R])
 
 // The four-step transform of the line held by this thread's group (thread j
 // of TH; its LDS rows start at gbase).  tws: W_N^m, m < N/2 (forward).  Every
-// thread of the block calls it (two barriers).
-template <typename T, bool INV, int TH, int R>
+// thread of the block calls it (two barriers); with WAVE, whole waves that hold
+// their lines' threads, each ordering its own LDS accesses.
+template <typename T, bool INV, int TH, int R, bool WAVE = false>
 __device__ __forceinline__ void fft_line(cpx<T> (&v)[R], int j, T *lre, T *lim, int gbase, const cpx<T> *tws)
 {
   constexpr int N = TH * R, H = N / 2, SK = TH + 1;
@@ -615,7 +616,7 @@ __device__ __forceinline__ void fft_line(cpx<T> (&v)[R], int j, T *lre, T *lim, 
     lre[gbase + k1 * SK + j] = v[k1].x;
     lim[gbase + k1 * SK + j] = v[k1].y;
   }
-  __syncthreads();
+  if (WAVE) wave_sync(); else __syncthreads();
 #pragma unroll
   for (int c = 0; c < R / TH; c++) {
     cpx<T> u[TH];
@@ -626,7 +627,7 @@ __device__ __forceinline__ void fft_line(cpx<T> (&v)[R], int j, T *lre, T *lim, 
 #pragma unroll
     for (int k2 = 0; k2 < TH; k2++) v[c + (R / TH) * k2] = u[k2];
   }
-  __syncthreads();
+  if (WAVE) wave_sync(); else __syncthreads();
 }
 
 // Strided N-point pass over `lines` lines: line l = a + A c (A = 2^lA) at a + c
@@ -1200,6 +1201,27 @@ __device__ __forceinline__ void h2_lstsq(const double (&sub)[kHm + 1], const dou
   for (int q = 0; q < kHm; q++) y[q] = yy[q];
 }
 
+// The coefficients y[q] of the Z_q from red: |U_j|^2, j < kHm, then rows j of
+// U_q . w (q <= j) and |w|^2 (see h2_layout).
+__device__ __forceinline__ void h2_coeffs(const double *red, double *y)
+{
+  double sub[kHm + 1], hc[kHm][kHm], in[kHm];
+  for (int j = 0; j < kHm; j++) {
+    const double n2 = red[j];
+    in[j] = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
+    sub[j] = sqrt(n2) * (j > 0 ? in[j - 1] : 1.0);
+  }
+  const double *d = red + kHm;  // d[j (kHm + 1) + q]
+  for (int j = 0; j < kHm; j++)
+    for (int q = 0; q <= j; q++) hc[q][j] = d[j * (kHm + 1) + q] * in[q] * in[j];
+  const int m = kHm - 1;
+  double left = d[m * (kHm + 1) + kHm] * in[m] * in[m];
+  for (int q = 0; q <= m; q++) left -= hc[q][m] * hc[q][m];
+  sub[kHm] = left > 0.0 ? sqrt(left) : 0.0;
+  h2_lstsq(sub, hc, y);
+  for (int q = 0; q < kHm; q++) y[q] *= in[q];
+}
+
 // Hessenberg columns from the partials, Givens QR and back substitution
 // (one block): the coefficients y[q] of the Z_q, q < kHm (zero past a
 // breakdown).  The normalised basis is U_q / n_q, n_q = |U_q|; the last
@@ -1218,35 +1240,21 @@ __global__ __launch_bounds__(256) void k2_solve(const double *__restrict__ p, in
     for (int t = 0; t < kNSums; t++) a[t] += p[(int64_t)t * nb + b];
   }
   block_sums<kNSums>(a, kNSums, red);
-  if (threadIdx.x != 0) return;
-  double sub[kHm + 1], hc[kHm][kHm], in[kHm];
-  for (int j = 0; j < kHm; j++) {
-    const double n2 = red[j];
-    in[j] = n2 > 0.0 ? 1.0 / sqrt(n2) : 0.0;
-    sub[j] = sqrt(n2) * (j > 0 ? in[j - 1] : 1.0);
-  }
-  const double *d = red + kHm;  // d[j (kHm + 1) + q]
-  for (int j = 0; j < kHm; j++)
-    for (int q = 0; q <= j; q++) hc[q][j] = d[j * (kHm + 1) + q] * in[q] * in[j];
-  const int m = kHm - 1;
-  double left = d[m * (kHm + 1) + kHm] * in[m] * in[m];
-  for (int q = 0; q <= m; q++) left -= hc[q][m] * hc[q][m];
-  sub[kHm] = left > 0.0 ? sqrt(left) : 0.0;
-  h2_lstsq(sub, hc, y);
-  for (int q = 0; q < kHm; q++) y[q] *= in[q];
+  if (threadIdx.x == 0) h2_coeffs(red, y);
 }
 
 // ---- the whole 2-D correction in one workgroup ------------------------------------
 // On a plane of at most kPlaneMax nodes each of the correction's seven launches
-// is 4 to 5 us of latency.  One workgroup of 512 threads does all of them (1024
-// make the barriers dearer: 3 to 6 % of a solve at 16^3, 1 % at 32^3): the
-// columns it owns (P per thread) stay in registers, the plane being transformed
-// sits in LDS, and the global sums are block sums.  What bounds it is the
-// latency of some 60 barriers and the LDS round trips of the transforms between
-// them: 22 us at 32^2, but 38 (FP32) and 49 us (FP64) at 64^2, one CU doing the
-// work.  us of a solve with one workgroup and with the launches: 16^3 FP64 970
-// and 1133, 32^3 FP64 941 and 1062, 64 x 32 x 64 mixed 900 and 955, 64 x 32 x
-// 32 FP64 1110 and 1175; 64^3 mixed 1060 and 1010, 64^3 FP64 1145 and 1023.
+// is 4 to 5 us of latency.  One workgroup does all of them: the columns it owns (P
+// per thread) stay in registers, the plane being transformed sits in LDS, and
+// the global sums are block sums.  k2_plane_q below takes the planes whose axes
+// have 16 to 64 points, this kernel those with shorter or longer ones.  What
+// bounds it is the latency of some 60 barriers and the LDS round trips of the
+// transforms between them: 20 us at 32^2, but 38 (FP32) and 49 us (FP64) at 64^2,
+// one CU doing the work.  512 threads (1024 make the barriers dearer: 3 to 6 % of
+// a solve at 16^3).  us of a solve with one workgroup and with the launches:
+// 16^3 FP64 970 and 1133, 32^3 FP64 941 and 1062, 64 x 32 x 64 mixed 900 and 955;
+// 64^3 mixed 1060 and 1010, 64^3 FP64 1145 and 1023.
 constexpr int kPlaneMax = 2048, kPlaneT = 512, kPlaneP = kPlaneMax / kPlaneT;
 constexpr int kPlanePad = kPlaneMax / 4;  // most lines of a plane (axes of 4 nodes and more): one pad value each
 
@@ -1461,6 +1469,191 @@ __global__ __launch_bounds__(kPlaneT) void k2_plane(int lx, int ly, int nz, int 
   if (threadIdx.x == 0) h2_lstsq(sub, hc, y);
 }
 
+// The same on planes whose axes have 16, 32 or 64 points (NX = THX RX, NY = THY
+// RY), with the four-step transforms in registers: a line's threads are lanes of
+// one wave, so the transforms themselves need no barrier, only the turn from
+// rows to columns does; the basis is unnormalised, as in the launches below, so
+// that three block sums do; the 2-D coefficients and the symbol are loaded and
+// made once.  LDS: the plane as rows (SX apart) or as columns (SY apart), with
+// room for a line's exchange in its own place.  us, k2_plane -> here: 16^2 FP64
+// 14.9 -> 9.7, 32^2 FP64 20.4 -> 15.7 and FP32 18.4 -> 14.2, 64 x 32 FP64 27.9 ->
+// 21.4; a solve on 32^3 FP64 885 -> 820, on 16^3 FP64 908 -> 845.  (64^2 took 59
+// and 42 us, more than the launches' 31: it spills.)
+template <typename T, int THX, int RX, int THY, int RY>
+__global__ __launch_bounds__((std::min(512, std::max(64, THX * RX * THY * RY / 4))))
+void k2_plane_q(int nz, int nzc, const double *__restrict__ part, const T *__restrict__ C, T *__restrict__ Z,
+                const double *__restrict__ twx, const double *__restrict__ twy, Symbol sym,
+                const double *__restrict__ trx, const double *__restrict__ try_, const double *__restrict__ trz,
+                double *__restrict__ y)
+{
+  constexpr int NX = THX * RX, NY = THY * RY, NXY = NX * NY;
+  constexpr int NT = NXY / 4 < 64 ? 64 : NXY / 4 > 512 ? 512 : NXY / 4, P = NXY / NT, NW = NT / 64;
+  constexpr int SX = (RX * (THX + 1) > NX ? RX * (THX + 1) : NX) | 1;
+  constexpr int SY = (RY * (THY + 1) > NY ? RY * (THY + 1) : NY) | 1;
+  constexpr int L = NY * SX > NX * SY ? NY * SX : NX * SY, kN = kHm + 2;
+  static_assert(NY * THX <= NT && NX * THY <= NT, "a thread's share of a line fits");
+  constexpr bool kKeepC = P * 9 * (int)sizeof(T) <= 320;  // the coefficients in registers (at most 80)
+  __shared__ T pre[L], pim[L];
+  __shared__ cpx<T> tx[NX / 2], ty[NY / 2];
+  __shared__ double sums[2][NW][kN];
+  const int t = (int)threadIdx.x, lane = t & 63, wid = t >> 6;
+  // block-wide sums of v[0 .. n): every thread adds the waves' sums in the same order
+  int flip = 0;
+  auto block_sum = [&](double *v, int n) {
+#pragma unroll
+    for (int q = 0; q < kN; q++) {
+      if (q < n) {
+        double x = v[q];
+        x += dpp_move<0x111>(x, 0.0);  // row_shr:1, 2, 4, 8: lane 15 of a row has its sum
+        x += dpp_move<0x112>(x, 0.0);
+        x += dpp_move<0x114>(x, 0.0);
+        x += dpp_move<0x118>(x, 0.0);
+        const double w = (lane_value(x, 15) + lane_value(x, 31)) + (lane_value(x, 47) + lane_value(x, 63));
+        if (lane == 0) sums[flip][wid][q] = w;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kN; q++) {
+      if (q < n) {
+        double x = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; w++) x += sums[flip][w][q];
+        v[q] = x;
+      }
+    }
+    flip ^= 1;
+  };
+  T U[kHm][P], Ck[kKeepC ? P : 1][9], w[P];
+  double r2[P], v[kN];
+  v[0] = 0.0;
+#pragma unroll
+  for (int p = 0; p < P; p++) r2[p] = 0.0;
+#pragma unroll 4
+  for (int zc = 0; zc < nzc; zc++) {
+#pragma unroll
+    for (int p = 0; p < P; p++) r2[p] += part[(int64_t)zc * NXY + t + NT * p];
+  }
+  if constexpr (kKeepC) {
+#pragma unroll
+    for (int p = 0; p < P; p++)
+#pragma unroll
+      for (int o = 0; o < 9; o++) Ck[p][o] = C[o * NXY + t + NT * p];
+  }
+  load_twiddles<T>(tx, twx, NX);
+  load_twiddles<T>(ty, twy, NY);
+  // the thread's lines: row t / THX, its elements j + THX m; column kx = t / THY
+  const int row = t / THX, jx = t % THX, kx = t / THY, jy = t % THY;
+  const bool xl = t < NY * THX, yl = t < NX * THY;
+  double f[RY];  // the kz = 0 symbol's factors at the thread's (kx, ky)
+#pragma unroll
+  for (int m = 0; m < RY; m++) f[m] = yl ? symbol_factor(sym, kx, jy + THY * m, 0, trx, try_, trz) : 0.0;
+#pragma unroll
+  for (int p = 0; p < P; p++) v[0] += r2[p];
+  block_sum(v, 1);
+  const double inz = 1.0 / (double)nz, mean = v[0] * inz / (double)NXY;
+#pragma unroll
+  for (int p = 0; p < P; p++) U[0][p] = (T)(r2[p] * inz - mean);
+  double red[kNSums];
+#pragma unroll
+  for (int j = 0; j < kHm; j++) {
+    // Z_j = F2 U_j
+#pragma unroll
+    for (int p = 0; p < P; p++) pre[(t + NT * p) / NX * SX + (t + NT * p) % NX] = U[j][p];
+    __syncthreads();
+    {
+      cpx<T> a[RX];
+      if (xl) {
+#pragma unroll
+        for (int m = 0; m < RX; m++) a[m] = {pre[row * SX + jx + THX * m], (T)0};
+        wave_sync();
+        fft_line<T, false, THX, RX, true>(a, jx, pre, pim, row * SX, tx);
+      }
+      __syncthreads();
+      if (xl) {
+#pragma unroll
+        for (int m = 0; m < RX; m++) {
+          pre[(jx + THX * m) * SY + row] = a[m].x;
+          pim[(jx + THX * m) * SY + row] = a[m].y;
+        }
+      }
+      __syncthreads();
+    }
+    {
+      cpx<T> a[RY];
+      if (yl) {
+#pragma unroll
+        for (int m = 0; m < RY; m++) a[m] = {pre[kx * SY + jy + THY * m], pim[kx * SY + jy + THY * m]};
+        wave_sync();
+        fft_line<T, false, THY, RY, true>(a, jy, pre, pim, kx * SY, ty);
+#pragma unroll
+        for (int m = 0; m < RY; m++) a[m] = {(T)((double)a[m].x * f[m]), (T)((double)a[m].y * f[m])};
+        fft_line<T, true, THY, RY, true>(a, jy, pre, pim, kx * SY, ty);
+      }
+      __syncthreads();
+      if (yl) {
+#pragma unroll
+        for (int m = 0; m < RY; m++) {
+          pre[(jy + THY * m) * SX + kx] = a[m].x;
+          pim[(jy + THY * m) * SX + kx] = a[m].y;
+        }
+      }
+      __syncthreads();
+    }
+    if (xl) {
+      cpx<T> a[RX];
+#pragma unroll
+      for (int m = 0; m < RX; m++) a[m] = {pre[row * SX + jx + THX * m], pim[row * SX + jx + THX * m]};
+      wave_sync();
+      fft_line<T, true, THX, RX, true>(a, jx, pre, pim, row * SX, tx);
+#pragma unroll
+      for (int m = 0; m < RX; m++) pre[row * SX + jx + THX * m] = a[m].x;
+    }
+    __syncthreads();
+    // w = A2 Z_j and its products with U_0 .. U_j
+#pragma unroll
+    for (int q = 0; q < kN; q++) v[q] = 0.0;
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      const int col = t + NT * p, i = col % NX, r = col / NX;
+      const int xs[3] = {(i - 1) & (NX - 1), i, (i + 1) & (NX - 1)};
+      const int ys[3] = {((r - 1) & (NY - 1)) * SX, r * SX, ((r + 1) & (NY - 1)) * SX};
+      double acc = 0.0;
+#pragma unroll
+      for (int o = 0; o < 9; o++)
+        acc += (double)(kKeepC ? Ck[kKeepC ? p : 0][o] : C[o * NXY + col]) * (double)pre[ys[o / 3] + xs[o % 3]];
+      w[p] = (T)acc;
+      Z[j * NXY + col] = pre[r * SX + i];
+#pragma unroll
+      for (int q = 0; q <= j; q++) v[q] += (double)U[q][p] * (double)w[p];
+      v[kHm] += (double)w[p] * (double)w[p];
+      v[kHm + 1] += (double)U[j][p] * (double)U[j][p];
+    }
+    block_sum(v, kN);  // (its barrier also ends the reads of the plane)
+    red[j] = v[kHm + 1];
+#pragma unroll
+    for (int q = 0; q <= kHm; q++) red[kHm + j * (kHm + 1) + q] = v[q];
+    if (j + 1 < kHm) {
+#pragma unroll
+      for (int p = 0; p < P; p++) {
+        double x = (double)w[p];
+#pragma unroll
+        for (int q = 0; q <= j; q++)
+          if (red[q] > 0.0) x -= v[q] / red[q] * (double)U[q][p];
+        U[j + 1 < kHm ? j + 1 : 0][p] = (T)x;
+      }
+    }
+  }
+  if (t == 0) h2_coeffs(red, y);
+}
+
+// Planes that k2_plane_q takes
+static bool plane_q(int nx, int ny)
+{
+  auto axis = [](int n) { return n == 16 || n == 32 || n == 64; };
+  return axis(nx) && axis(ny) && nx * ny <= kPlaneMax;
+}
+
 // z[k * nxy + col] += sum_q y_q Z_q[col] over kExtZ planes per block
 template <typename T>
 __global__ __launch_bounds__(256) void k2_ext(int64_t nxy, int nz, const T *__restrict__ Z, const double *__restrict__ y,
@@ -1507,7 +1700,23 @@ int fft2_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z, T *w3, b
   launch_lhs_zsum<T>(ctx, ctx->prm.lhs_type, (const T *)ctx->mom[0], z, r, h.part, h.pl, fused ? w3 : nullptr);
   Symbol sym = make_symbol(ctx, v19);
   sym.inv_scale = 1.0 / (double)nxy;
-  if (nxy <= kPlaneMax) {
+  if (plane_q(nx, ny)) {
+#define PLANE(THX, RX, THY, RY)                                                                                       \
+  hipLaunchKernelGGL((k2_plane_q<T, THX, RX, THY, RY>), 1, std::min(512, std::max(64, nx * ny / 4)), 0, ctx->stream, nz, \
+                     nzc, (const double *)h.part, (const T *)C, Z, ctx->tw[0], ctx->tw[1], sym, ctx->trig[0],          \
+                     ctx->trig[1], ctx->trig[2], h.y)
+#define PLANE_X(THY, RY)                          \
+  do {                                            \
+    if (nx == 16) PLANE(4, 4, THY, RY);           \
+    else if (nx == 32) PLANE(4, 8, THY, RY);      \
+    else if constexpr (THY * RY < 64) PLANE(8, 8, THY, RY); \
+  } while (0)
+    if (ny == 16) PLANE_X(4, 4);
+    else if (ny == 32) PLANE_X(4, 8);
+    else PLANE_X(8, 8);
+#undef PLANE_X
+#undef PLANE
+  } else if (nxy <= kPlaneMax) {
     hipLaunchKernelGGL((k2_plane<T>), 1, kPlaneT, 0, ctx->stream, ilog2(nx), ilog2(ny), nz,
                        nzc, (const double *)h.part, (const T *)C, Z, ctx->tw[0],
                        ctx->tw[1], sym, ctx->trig[0], ctx->trig[1], ctx->trig[2], h.y);

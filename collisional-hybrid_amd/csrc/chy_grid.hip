@@ -2247,29 +2247,6 @@ __device__ __forceinline__ C zf_row(const Grid &g, const SCoef &s, const LapRow 
   return row_apply<C, DIFF, OP>(s, lap, n0, nf, nzp, nzm, (C)x[q.c + k], xf, xe, (C)x[q.c + kp], (C)x[q.c + km], xfp, xfm);
 }
 
-// Orders a wave's own LDS accesses (which the hardware keeps in order)
-__device__ __forceinline__ void wave_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
-// x of the lane that CTRL (a DPP control) names, other where there is none in
-// the row of 16 lanes (or, for a shift of the whole wave, in the wave)
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double x, double other)
-{
-  const int lo = __builtin_amdgcn_update_dpp(__double2loint(other), __double2loint(x), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(other), __double2hiint(x), CTRL, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-
-__device__ __forceinline__ double lane_value(double x, int l)  // l: the same in every lane
-{
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
-                          __builtin_amdgcn_readlane(__double2loint(x), l));
-}
-
 // Inclusive scan of the affine maps y -> A y + B over groups of W lanes, lower
 // lanes' maps first (UP) or higher lanes' first: four register moves within the
 // rows of 16 lanes, then the row totals of the rows before it.  (Six shuffles

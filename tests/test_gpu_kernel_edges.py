@@ -37,15 +37,17 @@ def test_stencil_is_the_oracles_bit_for_bit(N, extra):
 
 
 # the one-workgroup 2-D correction: planes of 16 to 2048 nodes with even and
-# odd log2 lengths and the longest lines it takes; beyond it the separate
+# odd log2 lengths and the longest lines it takes, every pair of 16, 32 and 64
+# points in registers up to that size; beyond it the separate
 # launches, at one and several rows a block, and with x lines whose inverse
 # (2048 points in FP64) is a launch of its own.  The symbol of the FFT stage is a
 # sum that cancels towards the weakest mode: lambda_min / A0 = (1 - cos(2 pi /
 # N)) / (2 + 1 + Kz^2), and its 8 roundings on each side, in another order,
 # bound the agreement with the oracle.
 @pytest.mark.parametrize("prec,base", [("fp64", 1e-12), ("mixed", 2e-5)])
-@pytest.mark.parametrize("N", [(4, 4, 4), (8, 4, 4), (4, 8, 8), (32, 16, 8), (16, 32, 4), (64, 64, 4), (64, 32, 4), (4, 512, 4),
-                               (512, 4, 4), (4, 1024, 4), (1024, 4, 4), (128, 64, 4), (16, 256, 4), (2048, 4, 4)])
+@pytest.mark.parametrize("N", [(4, 4, 4), (8, 4, 4), (4, 8, 8), (32, 16, 8), (16, 32, 4), (64, 64, 4), (64, 32, 4),
+                               (4, 512, 4), (512, 4, 4), (4, 1024, 4), (1024, 4, 4), (128, 64, 4), (16, 256, 4), (2048, 4, 4),
+                               (16, 16, 4), (32, 32, 32), (64, 16, 4), (16, 64, 8), (32, 64, 4), (8, 256, 4)])
 def test_two_level_correction_on_any_plane(N, prec, base):
     rng = np.random.default_rng(12)
     with context(opts(N, extra=f"-pc_type fft2 -precision {prec}")) as ctx:
