@@ -790,6 +790,144 @@ __global__ __launch_bounds__((q_block<T, TH, R>())) void k_rfftq_x(int64_t nline
   }
 }
 
+// The x and y passes of one plane in one launch: a block holds the plane's row
+// pairs, then its columns of the half spectrum, in LDS (a line's exchange takes
+// place in its own row, SX or SY apart; its threads are lanes of one wave).
+// MODE 0: real rows -> half spectrum, natural order along x and y, as k_rfftq_x<0>
+// and k_fftq_s<0> leave it; MODE 1 the reverse.  On small grids a pass is one
+// launch's latency, so two in one are the faster: us forward and back, four
+// launches -> two: 16^3 FP64 11.2 -> 6.7, 32^3 FP64 15.9 -> 8.3 and FP32 14.3 ->
+// 7.8, 64^3 FP64 18.1 -> 12.9 and FP32 15.1 -> 11.4; a solve on 16^3 FP64 843 -> 772,
+// 32^3 FP64 815 -> 755, 64^3 FP64 953 -> 919, 64 x 64 x 256 mixed 1067 -> 1012.  (A
+// plane of 64 x 128 fills a block for as long as the launches take: 21.0 and
+// 21.1 us.)
+template <typename T, int MODE, int THX, int RX, int THY, int RY>
+__global__ __launch_bounds__((std::max(64, std::max(RY * THY / 2 * THX, THX * RX / 2 * THY))))
+void k_fft_xy(const T *__restrict__ rin, cpx<T> *__restrict__ buf, T *__restrict__ rout,
+              const double *__restrict__ twx, const double *__restrict__ twy, int64_t pstride)
+{
+  constexpr int NX = THX * RX, NY = THY * RY, H = NX / 2;
+  constexpr int SX = (RX * (THX + 1) > NX ? RX * (THX + 1) : NX) | 1;
+  constexpr int SY = (RY * (THY + 1) > NY ? RY * (THY + 1) : NY) | 1;
+  constexpr int L = NY / 2 * SX > H * SY ? NY / 2 * SX : H * SY;
+  __shared__ T pre[L], pim[L];
+  __shared__ cpx<T> tx[NX / 2], ty[NY / 2];
+  const int t = (int)threadIdx.x, g = t / THX, jx = t % THX, kx = t / THY, jy = t % THY;
+  const bool xl = t < NY / 2 * THX, yl = t < H * THY;
+  cpx<T> *pb = buf + (int64_t)blockIdx.x * pstride;
+  const int64_t r0 = (int64_t)blockIdx.x * NX * NY + (int64_t)2 * g * NX;
+  cpx<T> ax[RX], ay[RY];
+  if (MODE == 0) {
+    if (xl) {
+#pragma unroll
+      for (int m = 0; m < RX; m++) ax[m] = {rin[r0 + jx + THX * m], rin[r0 + NX + jx + THX * m]};
+    }
+  } else if (yl) {
+#pragma unroll
+    for (int m = 0; m < RY; m++) ay[m] = pb[kx + H * (jy + THY * m)];
+  }
+  load_twiddles<T>(tx, twx, NX);
+  load_twiddles<T>(ty, twy, NY);
+  __syncthreads();
+  T *re = pre + g * SX, *im = pim + g * SX;
+  if (MODE == 0) {
+    cpx<T> xa[RX / 2], xb[RX / 2];
+    if (xl) {
+      fft_line<T, false, THX, RX, true>(ax, jx, pre, pim, g * SX, tx);
+#pragma unroll
+      for (int m = 0; m < RX; m++) { re[jx + THX * m] = ax[m].x; im[jx + THX * m] = ax[m].y; }
+      wave_sync();
+#pragma unroll
+      for (int m = 0; m < RX / 2; m++) {
+        const int k = jx + THX * m;
+        const T zx = re[k], zy = im[k];
+        if (k == 0) {
+          xa[m] = {zx, re[H]};
+          xb[m] = {zy, im[H]};
+        } else {
+          const T mx = re[NX - k], my = im[NX - k];
+          xa[m] = {(T)0.5 * (zx + mx), (T)0.5 * (zy - my)};
+          xb[m] = {(T)0.5 * (zy + my), (T)0.5 * (mx - zx)};
+        }
+      }
+    }
+    __syncthreads();
+    if (xl) {
+#pragma unroll
+      for (int m = 0; m < RX / 2; m++) {
+        const int c = (jx + THX * m) * SY + 2 * g;
+        pre[c] = xa[m].x; pim[c] = xa[m].y;
+        pre[c + 1] = xb[m].x; pim[c + 1] = xb[m].y;
+      }
+    }
+    __syncthreads();
+    if (yl) {
+#pragma unroll
+      for (int m = 0; m < RY; m++) ay[m] = {pre[kx * SY + jy + THY * m], pim[kx * SY + jy + THY * m]};
+      wave_sync();
+      fft_line<T, false, THY, RY, true>(ay, jy, pre, pim, kx * SY, ty);
+#pragma unroll
+      for (int m = 0; m < RY; m++) pb[kx + H * (jy + THY * m)] = ay[m];
+    }
+  } else {
+    if (yl) fft_line<T, true, THY, RY, true>(ay, jy, pre, pim, kx * SY, ty);
+    __syncthreads();
+    if (yl) {  // row 2 g at the front of pair g's place, row 2 g + 1 H further
+#pragma unroll
+      for (int m = 0; m < RY; m++) {
+        const int row = jy + THY * m, c = (row >> 1) * SX + (row & 1) * H + kx;
+        pre[c] = ay[m].x; pim[c] = ay[m].y;
+      }
+    }
+    __syncthreads();
+    if (xl) {
+#pragma unroll
+      for (int m = 0; m < RX; m++) {
+        const int k = jx + THX * m;
+        if (k == 0) ax[m] = {re[0], re[H]};
+        else if (k == H) ax[m] = {im[0], im[H]};
+        else if (k < H) ax[m] = {re[k] - im[H + k], im[k] + re[H + k]};
+        else ax[m] = {re[NX - k] + im[H + NX - k], re[H + NX - k] - im[NX - k]};
+      }
+      wave_sync();
+      fft_line<T, true, THX, RX, true>(ax, jx, pre, pim, g * SX, tx);
+#pragma unroll
+      for (int m = 0; m < RX; m++) {
+        rout[r0 + jx + THX * m] = ax[m].x;
+        rout[r0 + NX + jx + THX * m] = ax[m].y;
+      }
+    }
+  }
+}
+
+// Planes that k_fft_xy takes
+static bool fft_xy_plane(int nx, int ny)
+{
+  auto axis = [](int n) { return n == 16 || n == 32 || n == 64; };
+  return axis(nx) && axis(ny);
+}
+
+template <typename T, int MODE>
+static void launch_fft_xy(chy_ctx *ctx, const T *rin, cpx<T> *buf, T *rout, int64_t pstride)
+{
+  const int nx = ctx->g.nx, ny = ctx->g.ny;
+#define XY(THX, RX, THY, RY)                                                                                   \
+  hipLaunchKernelGGL((k_fft_xy<T, MODE, THX, RX, THY, RY>), (unsigned)ctx->g.nz,                               \
+                     std::max(64, std::max(RY * THY / 2 * THX, THX * RX / 2 * THY)), 0, ctx->stream, rin, buf, \
+                     rout, ctx->tw[0], ctx->tw[1], pstride)
+#define XY_X(THY, RY)                     \
+  do {                                    \
+    if (nx == 16) XY(4, 4, THY, RY);      \
+    else if (nx == 32) XY(4, 8, THY, RY); \
+    else XY(8, 8, THY, RY);               \
+  } while (0)
+  if (ny == 16) XY_X(4, 4);
+  else if (ny == 32) XY_X(4, 8);
+  else XY_X(8, 8);
+#undef XY_X
+#undef XY
+}
+
 static bool pow2(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // Axis lengths of the four-step kernels: 16 to 512 points (512 in FP32 only:
@@ -877,7 +1015,10 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
 #define FFTQ(MODE, n, LINES, LA, EXTRA, ES, CS, TW)                                                                    \
   Q_AXIS(T, n, hipLaunchKernelGGL((k_fftq_s<T, MODE, TH, R>), blocks(LINES, NL) + EXTRA, NL * TH, 0, ctx->stream,      \
                                   (int64_t)(LINES), LA, ES, CS, buf, TW, sym, ctx->trig[0], ctx->trig[1], ctx->trig[2]))
-  if (xq) {  // x forward: real lines -> half spectra (kx < nx/2, slot 0 packs kx = 0, nx/2)
+  const bool xy = fft_xy_plane(nx, ny);
+  if (xy) {
+    launch_fft_xy<T, 0>(ctx, r, buf, (T *)nullptr, P);
+  } else if (xq) {  // x forward: real lines -> half spectra (kx < nx/2, slot 0 packs kx = 0, nx/2)
     RFFTQ(0, r, (T *)nullptr);
   } else {
     const int B = rfft_batch<T>(hx, nlines);
@@ -885,7 +1026,8 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
                        ilog2(nx), nlines, B, r, buf, (T *)nullptr, ctx->tw[0], 1.0, ilog2(ny), P);
   }
   // y forward: lines (kx, iz); A = nx/2 contiguous, c = iz with stride P
-  if (yq) {
+  if (xy) {
+  } else if (yq) {
     FFTQ(0, ny, (int64_t)hx * nz, lhx, 0u, (int64_t)hx, P, ctx->tw[1]);
   } else {
     const int n = ny, B = fft_batch<T>(n, hx);
@@ -907,7 +1049,9 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
                          sym, ctx->trig[0], ctx->trig[1], ctx->trig[2]);
     }
   }
-  if (yq) {  // y inverse
+  if (xy) {
+    launch_fft_xy<T, 1>(ctx, (const T *)nullptr, buf, z, P);
+  } else if (yq) {  // y inverse
     FFTQ(1, ny, (int64_t)hx * nz, lhx, 0u, (int64_t)hx, P, ctx->tw[1]);
   } else {
     const int n = ny, B = fft_batch<T>(n, hx);
@@ -915,7 +1059,8 @@ int fft_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z)
                        (int64_t)hx, (int64_t)hx, P, B, buf, ctx->tw[1], sym, ctx->trig[0], ctx->trig[1],
                        ctx->trig[2]);
   }
-  if (xq) {  // x inverse: half spectra -> real lines
+  if (xy) {
+  } else if (xq) {  // x inverse: half spectra -> real lines
     RFFTQ(1, (const T *)nullptr, z);
   } else {
     const int B = rfft_batch<T>(hx, nlines);

@@ -74,7 +74,9 @@ def test_two_level_correction_on_any_plane(N, prec, base):
 @pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5"])
 @pytest.mark.parametrize("N", [(16, 4, 4), (4, 16, 4), (4, 4, 16), (16, 16, 32), (32, 32, 16), (64, 16, 8), (8, 64, 16),
                                (32, 8, 64), (128, 32, 4), (16, 128, 8), (4, 8, 128), (64, 64, 64), (256, 16, 4),
-                               (8, 256, 16), (4, 4, 256), (512, 4, 16), (4, 512, 4), (8, 4, 512)])
+                               (8, 256, 16), (4, 4, 256), (512, 4, 16), (4, 512, 4), (8, 4, 512),
+                               # both axes of 16 to 64 points: the plane in one launch
+                               (16, 32, 4), (16, 64, 8), (32, 16, 16), (32, 64, 4), (64, 32, 16), (64, 64, 4)])
 def test_fft_passes_on_axes_of_any_length(N, extra, prec, base):
     rng = np.random.default_rng(17)
     with context(opts(N, extra=f"-pc_type fft -precision {prec} {extra}")) as ctx:
