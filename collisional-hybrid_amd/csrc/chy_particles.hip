@@ -545,22 +545,49 @@ __global__ __launch_bounds__(256) void k_scan_tiles(int64_t nt, uint32_t *__rest
 }
 
 // Per-tile scan; writes offsets[0..n) and the cursor copy; offsets[n] = total.
+// The tile passes through LDS, so that a thread takes 16 consecutive counts and
+// the tile needs one block scan while memory is read and written in whole
+// lines.  us, with a block scan and a round trip to memory for each 256 counts ->
+// now: 32^3 and 64^3 12.8 -> 4.5, 256^3 40 -> 32.
 __global__ __launch_bounds__(256) void k_tile_scan(int64_t n, const uint32_t *__restrict__ in,
                                                    const uint32_t *__restrict__ tsum, uint32_t *__restrict__ offs,
                                                    uint32_t *__restrict__ cursor, uint32_t total)
 {
-  __shared__ uint32_t sh[4];
+  constexpr int K = kScanTile / 256;
+  __shared__ uint32_t sh[4], w[kScanTile + 256];  // (a pad value every K)
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
-  uint32_t carry = tsum[blockIdx.x];
-  for (int q0 = 0; q0 < kScanTile; q0 += 256) {
-    const int64_t i = base + q0 + threadIdx.x;
-    const uint32_t v = i < n ? in[i] : 0u;
-    uint32_t tot;
-    const uint32_t ex = block_exscan(v, tot, sh);
-    if (i < n) { offs[i] = carry + ex; cursor[i] = carry + ex; }
-    carry += tot;
+  const int t = (int)threadIdx.x;
+  uint32_t v[K];
+#pragma unroll
+  for (int u = 0; u < K; u++) {
+    const int64_t i = base + t + 256 * u;
+    v[u] = i < n ? in[i] : 0u;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) offs[n] = total;
+#pragma unroll
+  for (int u = 0; u < K; u++) w[(t + 256 * u) + (t + 256 * u) / K] = v[u];
+  __syncthreads();
+  uint32_t sum = 0;
+#pragma unroll
+  for (int u = 0; u < K; u++) {
+    const uint32_t c = w[(K + 1) * t + u];
+    v[u] = sum;
+    sum += c;
+  }
+  uint32_t tot;
+  const uint32_t ex = tsum[blockIdx.x] + block_exscan(sum, tot, sh);
+#pragma unroll
+  for (int u = 0; u < K; u++) w[(K + 1) * t + u] = ex + v[u];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < K; u++) {
+    const int64_t i = base + t + 256 * u;
+    if (i < n) {
+      const uint32_t q = w[(t + 256 * u) + (t + 256 * u) / K];
+      offs[i] = q;
+      cursor[i] = q;
+    }
+  }
+  if (blockIdx.x == 0 && t == 0) offs[n] = total;
 }
 
 // Scatter: slot = cursor[key]++ (run-aggregated), perm[slot] = p.

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import orc
-from gpu_cases import (as_particles, context, grid_of, opts, push_params_of, random_particles, relmax, upload,
+from gpu_cases import (as_particles, context, grid_of, opts, oracle_sorted, push_params_of, random_particles, relmax, upload,
                        vlasov_from)
 
 pytestmark = pytest.mark.gpu
@@ -255,3 +255,22 @@ def test_fp64_push_of_any_number_of_ions(N, n, nui):
     assert (st.accepted, st.refused) == (stats[0], stats[1])
     for a in ("x", "y", "z", "vx", "vy", "vz"):
         assert relmax(getattr(after, a), getattr(nxt, a)) <= 1e-12
+
+
+# tiles of 4096 cells, 16 a thread: a part of one, one short by a cell, a whole
+# one, and further tiles that end within a thread's cells
+@pytest.mark.parametrize("N", [(3, 3, 3), (63, 13, 5), (16, 16, 16), (17, 241, 3), (41, 20, 11), (3, 1371, 3)])
+def test_cell_offsets_at_the_edges_of_scan_tiles(N):
+    rng = np.random.default_rng(20)
+    n = 3 * N[0] * N[1] * N[2] + 1
+    with context(opts(N), capacity=n) as ctx:
+        g = grid_of(ctx.prm)
+        p = random_particles(g, n, rng)
+        upload(ctx, p)
+        got = as_particles(ctx.get_particles())
+        v = ctx.collect_moments()
+    ps, offs = oracle_sorted(g, p)
+    assert np.array_equal(got.pid, ps.pid)
+    ref = orc.deposit_sorted(g, ps, offs)
+    for a in range(4):
+        assert np.array_equal(v[:, a], ref[a])
