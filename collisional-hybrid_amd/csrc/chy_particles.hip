@@ -173,8 +173,8 @@ __device__ __forceinline__ void flush_scatter_counts(unsigned long long *cs, uin
 // stores, its loads and its corners in turn, and 61 % of the waves' time went
 // into waiting at a few hundred GB/s.  With the next ion's loads issued before
 // this one's stores, its arguments reloaded instead of spilled and arithmetic
-// for the arguments that occur (chy_device.h: 2154 -> 1164 vector instructions
-// in all) it went from 11.43 to 8.63 ms on 268 M ions and from 3.20 to 2.24 on
+// for the arguments that occur (chy_device.h: 2154 -> 1268 vector instructions
+// in all) it went from 11.43 to 9.09 ms on 268 M ions and from 3.20 to 2.35 on
 // 67 M, of which the instructions make up about two thirds.  (The arithmetic
 // alone gained 4 %; four waves per SIMD instead of three cost spills.)
 // The kernel's (only) argument in its constant segment, by a pointer of which
