@@ -424,7 +424,7 @@ int64_t fft2_buf_elems(const chy_ctx *ctx);  // elements of T in pc2_buf
 int64_t fft2_h_elems(const chy_ctx *ctx);    // doubles in pc2_h
 // fft2z: the z-line correction of the fft2 residual.  zbuf: 4 nc values of T
 // (factors), colbuf: 2 (nx ny) doubles, made by launch_zline_factor once per
-// solve; launch_zline_apply adds the z-line solve of res to z (res is used as
+// solve; launch_zline_apply adds the z-line solve of res to z (res may be used as
 // scratch); launch_residual_t: res = b - A(n) x in precision T.
 template <typename T>
 void launch_zline_factor(chy_ctx *ctx, int lhs_type, const T *n, T *zbuf, double *colbuf);
