@@ -309,6 +309,16 @@ __device__ __forceinline__ double lane_value(double x, int l)  // l: the same in
                           __builtin_amdgcn_readlane(__double2loint(x), l));
 }
 
+// Sum over the wave's 64 lanes (all active), the same in every lane
+__device__ __forceinline__ double wave_total(double x)
+{
+  x += dpp_move<0x111>(x, 0.0);  // row_shr:1, 2, 4, 8: lane 15 of a row has its sum
+  x += dpp_move<0x112>(x, 0.0);
+  x += dpp_move<0x114>(x, 0.0);
+  x += dpp_move<0x118>(x, 0.0);
+  return (lane_value(x, 15) + lane_value(x, 31)) + (lane_value(x, 47) + lane_value(x, 63));
+}
+
 // Run-length aggregation of integer atomics over lanes holding equal keys in
 // consecutive lanes: returns, for each active lane, (head lane, run length).
 // Inactive lanes must pass key = -1.

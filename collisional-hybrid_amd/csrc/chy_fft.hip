@@ -1151,9 +1151,7 @@ __device__ __forceinline__ void block_sums(double (&v)[NV], int nv, double *out)
 #pragma unroll
   for (int q = 0; q < NV; q++) {
     if (q < nv) {
-      double t = v[q];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
+      const double t = wave_total(v[q]);
       if ((threadIdx.x & 63) == 0) sh[w][q] = t;
     }
   }
@@ -1373,18 +1371,16 @@ __device__ __forceinline__ void h2_coeffs(const double *red, double *y)
 // subdiagonal entry, the norm of what is left of w, comes from |w|^2 less the
 // parts taken out.
 constexpr int kNSums = kHm * (kHm + 2);
-__global__ __launch_bounds__(256) void k2_solve(const double *__restrict__ p, int nb, double *__restrict__ y)
+__global__ __launch_bounds__(64 * kNSums) void k2_solve(const double *__restrict__ p, int nb, double *__restrict__ y)
 {
-  // p: pn[j], then pd[j][q]
+  // p: pn[j], then pd[j][q]; a wave a sum
   __shared__ double red[kNSums];
-  double a[kNSums];
-#pragma unroll
-  for (int t = 0; t < kNSums; t++) a[t] = 0.0;
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-#pragma unroll
-    for (int t = 0; t < kNSums; t++) a[t] += p[(int64_t)t * nb + b];
-  }
-  block_sums<kNSums>(a, kNSums, red);
+  const int w = threadIdx.x >> 6;
+  double a = 0.0;
+  for (int b = threadIdx.x & 63; b < nb; b += 64) a += p[(int64_t)w * nb + b];
+  a = wave_total(a);
+  if ((threadIdx.x & 63) == 0) red[w] = a;
+  __syncthreads();
   if (threadIdx.x == 0) h2_coeffs(red, y);
 }
 
@@ -1648,12 +1644,7 @@ void k2_plane_q(int nz, int nzc, const double *__restrict__ part, const T *__res
 #pragma unroll
     for (int q = 0; q < kN; q++) {
       if (q < n) {
-        double x = v[q];
-        x += dpp_move<0x111>(x, 0.0);  // row_shr:1, 2, 4, 8: lane 15 of a row has its sum
-        x += dpp_move<0x112>(x, 0.0);
-        x += dpp_move<0x114>(x, 0.0);
-        x += dpp_move<0x118>(x, 0.0);
-        const double w = (lane_value(x, 15) + lane_value(x, 31)) + (lane_value(x, 47) + lane_value(x, 63));
+        const double w = wave_total(v[q]);
         if (lane == 0) sums[flip][wid][q] = w;
       }
     }
@@ -1893,7 +1884,7 @@ int fft2_pc_apply(chy_ctx *ctx, const double v19[19], const T *r, T *z, T *w3, b
                            (const cpx<T> *)cb, ctx->tw[0], Zj, (const T *)U, w, h.pd);
       }
     }
-    hipLaunchKernelGGL(k2_solve, 1, 256, 0, ctx->stream, (const double *)h.pn, nb, h.y);
+    hipLaunchKernelGGL(k2_solve, 1, 64 * kNSums, 0, ctx->stream, (const double *)h.pn, nb, h.y);
   }
   if (fused) {
     launch_zline_apply_e2<T>(ctx, (const T *)ctx->zl_buf, ctx->zl_col, w3, z, (const T *)ctx->mom[0], (const T *)Z,
