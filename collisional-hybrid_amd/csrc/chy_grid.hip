@@ -457,8 +457,7 @@ void k_lhs_tiled(Grid g, int lhs_type, SCoef s, LapRow lap,
         t += zs[rr];
       }
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+    t = wave_total(t);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0) pl[tile] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
@@ -672,8 +671,7 @@ __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow
   if (ZS || OUT == 3) {
     __shared__ double wsum[4];
     double t = zs;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+    t = wave_total(t);
     if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0) pl[tile] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
@@ -684,8 +682,7 @@ __global__ __launch_bounds__(256) void k_lhs_col(Grid g, int zc, SCoef s, LapRow
     for (int q = 0; q < kColDots; q++) {
       if (q < nv) {
         double t = dots[q];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) t += __shfl_down(t, o, 64);
+        t = wave_total(t);
         if ((threadIdx.x & 63) == 0) dsum[threadIdx.x >> 6][q] = t;
       }
     }
@@ -1051,13 +1048,6 @@ void launch_rhs(chy_ctx *ctx, int rhs_type, const T *n, const T *gx, const T *gy
 // ---- deterministic reductions ---------------------------------------------------
 constexpr int kMaxDots = 32;
 
-__device__ __forceinline__ double wave_sum(double v)
-{
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-  return v;
-}
-
 // partial[blk*nv + k] = sum over this block's grid-stride range of A_k . b
 template <typename T, int NV>
 __global__ __launch_bounds__(256) void k_mdot(int nv, const T *__restrict__ A, int64_t stride, const T *__restrict__ b,
@@ -1077,7 +1067,7 @@ __global__ __launch_bounds__(256) void k_mdot(int nv, const T *__restrict__ A, i
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     if (k < nv) {
-      const double s = wave_sum(acc[k]);
+      const double s = wave_total(acc[k]);
       if ((threadIdx.x & 63) == 0) sh[wid][k] = s;
     }
   }
@@ -1106,7 +1096,7 @@ __global__ __launch_bounds__(256) void k_combine(const double *__restrict__ part
   for (int k = 0; k < nv; k++) {
     double acc = 0.0;
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) acc += partial[(int64_t)b * nv + k];
-    const double s = wave_sum(acc);
+    const double s = wave_total(acc);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -1153,7 +1143,7 @@ __global__ __launch_bounds__(256) void k_chunk_sum(const double *__restrict__ pa
   double acc = 0.0;
 #pragma unroll 8
   for (int64_t b = lo + threadIdx.x; b < hi; b += blockDim.x) acc += partial[b];
-  const double t = wave_sum(acc);
+  const double t = wave_total(acc);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = t;
   __syncthreads();
   if (threadIdx.x == 0) out[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
@@ -1197,7 +1187,7 @@ __global__ __launch_bounds__(256) void k_sum(const T *__restrict__ a, int64_t n,
   double acc = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     acc += (double)a[i];
-  const double s = wave_sum(acc);
+  const double s = wave_total(acc);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
@@ -1282,7 +1272,7 @@ __global__ __launch_bounds__(256) void k_mgs_norm(int nv, const T *__restrict__ 
     w[i] = r;
     nn += (double)r * (double)r;
   }
-  const double s = wave_sum(nn);
+  const double s = wave_total(nn);
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
   __syncthreads();
   if (threadIdx.x == 0) partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
@@ -1319,7 +1309,7 @@ __device__ __forceinline__ void block_partials(const double (&acc)[NV], int nv, 
 #pragma unroll
   for (int k = 0; k < NV; k++) {
     if (k < nv) {
-      const double s = wave_sum(acc[k]);
+      const double s = wave_total(acc[k]);
       if ((threadIdx.x & 63) == 0) sh[wid][k] = s;
     }
   }
@@ -1374,7 +1364,7 @@ __global__ __launch_bounds__(256) void k_gs4(int nv, const T *__restrict__ V, in
         double t = 0.0;
 #pragma unroll 4
         for (int b = lane; b < nblk; b += 64) t += h[(int64_t)b * nv + k];
-        t = wave_sum(t);
+        t = wave_total(t);
         if (lane == 0) {
           const double v = t * sc.s[k];
           hs[k] = v;
