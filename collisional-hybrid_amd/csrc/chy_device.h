@@ -101,7 +101,7 @@ __host__ __device__ __forceinline__ double div_rn(double a, double d, double rd)
   return __builtin_fma(__builtin_fma(-q, d, a), rd, q);
 }
 
-// a / b for normal b whose quotient neither over- nor underflows: the hardware's
+// a / b for normal b (not 0) whose quotient neither over- nor underflows: the hardware's
 // reciprocal refined twice, then one exact remainder (the last bit may differ
 // from a / b's where that is a near tie)
 __device__ __forceinline__ double div_normal(double a, double b)

@@ -84,6 +84,9 @@ template <typename T> __device__ __forceinline__ T kin_sqrt(T x) { return sqrt_n
 template <> __device__ __forceinline__ float kin_sqrt<float>(float x) { return __builtin_amdgcn_sqrtf(fmaxf(x, 0.0f)); }
 template <typename T> __device__ __forceinline__ T kin_div(T a, T b) { return div_normal(a, b); }
 template <> __device__ __forceinline__ float kin_div<float>(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+// the same for a divisor that may be 0 (a / 0 is infinite; div_normal's is NaN)
+template <typename T> __device__ __forceinline__ T kin_div_any(T a, T b) { return a / b; }
+template <> __device__ __forceinline__ float kin_div_any<float>(float a, float b) { return kin_div<float>(a, b); }
 // sine and cosine of 2 pi u, 0 <= u <= 1
 __device__ __forceinline__ void kin_sincos2pi(double u, double &s, double &c) { sincos2pi(u, s, c); }
 __device__ __forceinline__ void kin_sincos2pi(float u, float &s, float &c)
@@ -200,7 +203,7 @@ __device__ __forceinline__ int scatter_n(const PC &pc, uint32_t pid, T vnx, T vn
   const T ux2 = ux1 * cosphi - uy1 * sinphi, uy2 = ux1 * sinphi + uy1 * cosphi, uz2 = uz1;
   const T vfx = vcx + vcr * ux2, vfy = vcy + vcr * uy2, vfz = vcz + vcr * uz2;
   const T vfr = kin_sqrt<T>(vfx * vfx + vfy * vfy + vfz * vfz);
-  if (kin_div<T>(vfr, (T)pc.viT) > (T)10.0) return 2;
+  if (kin_div_any<T>(vfr, (T)pc.viT) > (T)10.0) return 2;  // viT is 0 for ions without a thermal speed
   vx = vfx; vy = vfy; vz = vfz;
   return 1;
 }

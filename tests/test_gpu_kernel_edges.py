@@ -274,3 +274,32 @@ def test_cell_offsets_at_the_edges_of_scan_tiles(N):
     ref = orc.deposit_sorted(g, ps, offs)
     for a in range(4):
         assert np.array_equal(v[:, a], ref[a])
+
+
+# ions without a thermal speed: the final speed of a scattering is then more than
+# ten times it however small, and every scattering is refused (a drift gives
+# them collisions); the oracle divides by zero
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_ions_without_a_thermal_speed_refuse_every_scattering(prec):
+    rng = np.random.default_rng(21)
+    n = 4000
+    with context(opts((6, 5, 4), extra=f"-precision {prec} -Ti 0 -vi0x 500 -nui 1e4 -seed 5 --collision-refusal-limit 0 "
+                                       f"-Np {n}"), capacity=n) as ctx:
+        assert ctx.prm.viT_r == 0.0
+        g = grid_of(ctx.prm)
+        upload(ctx, random_particles(g, n, rng))
+        phi = 0.01 * rng.standard_normal(g.nc)
+        ctx.set_potential(phi)
+        before = as_particles(ctx.get_particles())
+        S = orc.normaliser(before, list(ctx.prm.vn0), ctx.prm.vnT)
+        _, P = push_params_of(ctx.prm, step=0)
+        st = ctx.update_velocities()
+        after = as_particles(ctx.get_particles())
+    nxt, _, _, _, stats = orc.step(g, P, before, phi, S, list(ctx.prm.E0))
+    assert stats[0] == 0 and stats[1] > n // 20
+    assert st.accepted == 0 and st.refused > n // 20
+    if prec == "fp64":
+        back, want = np.argsort(after.pid), np.argsort(nxt.pid)
+        assert st.refused == stats[1]
+        for a in ("vx", "vy", "vz"):
+            assert relmax(getattr(after, a)[back], getattr(nxt, a)[want]) <= 1e-12
