@@ -214,14 +214,18 @@ __device__ __forceinline__ double sqrt_normal(double x)
 
 // ---- periodic cells ----------------------------------------------------------
 // Cell of an absolute coordinate, clamped to [0, n-1]; f = fraction in cell.
-__device__ __forceinline__ void cell_coord(double x, double p0, double d, double rd, int n, int &i, double &f)
+__device__ __forceinline__ void cell_split(double xi, int n, int &i, double &f)
 {
-  const double xi = div_rn(x - p0, d, rd);
   int ii = (int)xi;
   if (ii > n - 1) ii = n - 1;
   if (ii < 0) ii = 0;
   i = ii;
   f = xi - (double)ii;
+}
+
+__device__ __forceinline__ void cell_coord(double x, double p0, double d, double rd, int n, int &i, double &f)
+{
+  cell_split(div_rn(x - p0, d, rd), n, i, f);
 }
 
 // Periodic wrap into [p0, p1); a coordinate more than one period away is
