@@ -10,6 +10,8 @@
 // 700,001 ions 10.8 -> 5.8, getting them 17.4 -> 10.1.
 #include <algorithm>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <system_error>
 #include <thread>
 
@@ -254,9 +256,10 @@ struct IonStage {
   uint32_t *pid;
 };
 
+constexpr size_t kIon = 2 * sizeof(Vec4<double>) + sizeof(double) + sizeof(uint32_t);
+
 static int ion_stage(chy_ctx *ctx, int64_t np, IonStage &s)
 {
-  constexpr size_t kIon = 2 * sizeof(Vec4<double>) + sizeof(double) + sizeof(uint32_t);
   void *st;
   size_t got;
   TRY(stage_get(ctx, kIon * (size_t)np, &st, &got));
@@ -295,6 +298,31 @@ int ions_upload(chy_ctx *ctx, int64_t np, const double *pos, const double *vel, 
   return CHY_OK;
 }
 
+// The staged arrays (all ions in one piece) that are wanted in one copy, where
+// there are several and all of them together take at most kMost: a copy and its
+// wait are some 20 us whatever they move.  us for all four weighted mixed arrays,
+// a copy each -> one: 300 ions 82 -> 24, 3000 65 -> 33, 6800 66 -> 49; at 7000
+// they would be level soon.  (FP64 weights and ids are not staged.)
+static int ions_small(chy_ctx *ctx, const IonStage &s, double *pos, double *vel, double *w, uint32_t *pid, bool &done)
+{
+  constexpr size_t kMost = (size_t)512 << 10;
+  const size_t n = (size_t)s.per;
+  done = false;
+  if (kIon * n > kMost || (pos != nullptr) + (vel != nullptr) + (w != nullptr) + (pid != nullptr) < 2) return CHY_OK;
+  std::unique_ptr<unsigned char[]> h(new (std::nothrow) unsigned char[kIon * n]);
+  if (!h) return CHY_OK;
+  TRY(copy_to_host(ctx, h.get(), s.pos, kIon * n));
+  auto part = [&](void *dst, const void *dev, size_t bytes) {
+    if (dst) memcpy(dst, h.get() + ((const unsigned char *)dev - (const unsigned char *)s.pos), bytes);
+  };
+  part(pos, s.pos, sizeof(Vec4<double>) * n);
+  part(vel, s.vel, sizeof(Vec4<double>) * n);
+  part(w, s.w, sizeof(double) * n);
+  part(pid, s.pid, sizeof(uint32_t) * n);
+  done = true;
+  return CHY_OK;
+}
+
 int ions_download(chy_ctx *ctx, int64_t np, double *pos, double *vel, double *w, uint32_t *pid)
 {
   const bool own_w = ctx->weighted;  // unit weights are filled in below
@@ -309,6 +337,9 @@ int ions_download(chy_ctx *ctx, int64_t np, double *pos, double *vel, double *w,
                            s.w, s.pid);
       else
         hipLaunchKernelGGL(k_ions_out_fp64, nb, 256, 0, ctx->stream, n, i0, ctx->pd[ctx->cur], s.pos, s.vel);
+      bool done = false;
+      if (ctx->mixed && n == np) TRY(ions_small(ctx, s, pos, vel, own_w ? w : nullptr, pid, done));
+      if (done) break;
       if (pos) TRY(copy_to_host(ctx, pos + 4 * i0, s.pos, sizeof(Vec4<double>) * n));
       if (vel) TRY(copy_to_host(ctx, vel + 4 * i0, s.vel, sizeof(Vec4<double>) * n));
       if (ctx->mixed) {

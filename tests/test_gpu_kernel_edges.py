@@ -1,8 +1,11 @@
 """Kernels at the sizes where their tiling can go wrong: block edges,
 remainders, the smallest grids and both sides of each dispatch rule."""
+import time
+
 import numpy as np
 import pytest
 
+import chybrid
 import orc
 from gpu_cases import (as_particles, context, grid_of, opts, oracle_sorted, push_params_of, random_particles, relmax, upload,
                        vlasov_from)
@@ -303,3 +306,42 @@ def test_ions_without_a_thermal_speed_refuse_every_scattering(prec):
         assert st.refused == stats[1]
         for a in ("vx", "vy", "vz"):
             assert relmax(getattr(after, a)[back], getattr(nxt, a)[want]) <= 1e-12
+
+
+# mixed: the arrays of up to 6898 ions come in one copy, of more in one each; both
+# sides of the line, and a caller that wants some of them.  A copy's latency
+# is all that few ions cost, so all four arrays take about what one does
+@pytest.mark.parametrize("n", [1, 300, 6898, 6899])
+def test_arrays_of_a_few_ions_come_in_one_copy(n):
+    rng = np.random.default_rng(22)
+    with context(opts((5, 4, 6), extra="-precision mixed"), capacity=n, weighted=True) as ctx:
+        p = random_particles(grid_of(ctx.prm), n, rng, weights=True)
+        upload(ctx, p)
+        d = ctx.get_particles()
+        get = chybrid.lib().chy_get_particles
+        full = [np.empty((n, 4)), np.empty((n, 4)), np.empty(n), np.empty(n, np.uint32)]
+        for want in ((0, 1, 2, 3), (3,), (1,), (0, 2), (1, 3)):
+            out = [np.full_like(a, 7) for a in full]
+            assert get(ctx._p, *[out[q].ctypes.data if q in want else None for q in range(4)]) == 0
+            got = dict(zip(("pos", "vel", "w", "pid"), out))
+            for q, name in enumerate(("pos", "vel", "w", "pid")):
+                if q not in want:
+                    assert (got[name] == 7).all()
+                elif q < 2:
+                    for a, axis in enumerate("xyz"):
+                        assert np.array_equal(got[name][:, a], d[("" if q == 0 else "v") + axis])
+                else:
+                    assert np.array_equal(got[name], d[name])
+
+        def least(ptrs):
+            t = []
+            for _ in range(300):
+                t0 = time.perf_counter()
+                get(ctx._p, *ptrs)
+                t.append(time.perf_counter() - t0)
+            return min(t)
+
+        if n <= 300:
+            all_four = least([a.ctypes.data for a in full])
+            one = least([None, None, None, full[3].ctypes.data])
+            assert all_four <= 2 * one, (all_four, one)
