@@ -22,7 +22,8 @@ namespace chy {
 // Device scratch for `bytes` of a layout change, less when the caller's loop
 // has to take several pieces: the Krylov basis, which holds nothing between
 // solves, or for many ions on a small grid a buffer of at most kStageBytes that
-// the context then keeps.
+// the context then keeps (the basis again, in small pieces, where the device
+// has no memory left for one).
 static int stage_get(chy_ctx *ctx, size_t bytes, void **p, size_t *got)
 {
   constexpr size_t kEnough = (size_t)16 << 20;
@@ -36,10 +37,15 @@ static int stage_get(chy_ctx *ctx, size_t bytes, void **p, size_t *got)
     if (ctx->stage) (void)hipFree(ctx->stage);
     ctx->stage = nullptr;
     ctx->stage_bytes = 0;
-    unsigned char *q = nullptr;
-    TRY(dalloc(ctx, &q, (int64_t)want));
-    ctx->stage = q;
-    ctx->stage_bytes = want;
+    if (hipMalloc(&ctx->stage, want) == hipSuccess) {
+      ctx->stage_bytes = want;
+    } else {
+      ctx->stage = nullptr;
+      (void)hipGetLastError();
+      *p = ctx->V;
+      *got = ctx->V_bytes;
+      return CHY_OK;
+    }
   }
   *p = ctx->stage;
   *got = ctx->stage_bytes;

@@ -1,5 +1,8 @@
 """Kernels at the sizes where their tiling can go wrong: block edges,
 remainders, the smallest grids and both sides of each dispatch rule."""
+import os
+import subprocess
+import sys
 import time
 
 import numpy as np
@@ -345,3 +348,49 @@ def test_arrays_of_a_few_ions_come_in_one_copy(n):
             all_four = least([a.ctypes.data for a in full])
             one = least([None, None, None, full[3].ctypes.data])
             assert all_four <= 2 * one, (all_four, one)
+
+
+# many ions on a small grid, with no device memory to be had for their staging (an
+# allocator that refuses it, put before the runtime's in a process of its own):
+# the ions go in and come back in small pieces
+_NO_STAGE = r"""
+import ctypes, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path[:0] = sys.argv[2:5]
+import numpy as np
+import chybrid
+from gpu_cases import context, grid_of, opts, random_particles, upload
+n = 30000
+for prec in ("fp64", "mixed"):
+    with context(opts((4, 4, 4), extra="-precision " + prec), capacity=n, weighted=True) as ctx:
+        p = random_particles(grid_of(ctx.prm), n, np.random.default_rng(23), weights=True)
+        p.pid = np.arange(n, dtype=np.uint32)[::-1].copy()
+        ctypes.c_size_t.in_dll(shim, "fail_from").value = 1
+        upload(ctx, p)
+        d = ctx.get_particles()
+        refused = ctypes.c_size_t.in_dll(shim, "refused").value
+        ctypes.c_size_t.in_dll(shim, "fail_from").value = 0
+    assert refused > 0
+    back, want = np.argsort(d["pid"]), np.argsort(p.pid)
+    for name in ("vx", "vy", "vz", "w"):
+        v = getattr(p, name)[want]
+        assert np.array_equal(d[name][back], v if prec == "fp64" else v.astype(np.float32).astype(np.float64))
+    for name in "xyz":
+        assert np.abs(d[name][back] - getattr(p, name)[want]).max() <= (0 if prec == "fp64" else 2.0 ** -24 * 0.05)
+print("STAGED")
+"""
+
+
+def test_ions_are_staged_without_device_memory_to_spare(tmp_path):
+    src, so = tmp_path / "shim.c", tmp_path / "shim.so"
+    src.write_text("#include <dlfcn.h>\n#include <stddef.h>\nsize_t fail_from, refused;\n"
+                   "int hipMalloc(void **p, size_t n)\n{\n  static int (*next)(void **, size_t);\n"
+                   "  if (fail_from && n >= fail_from) { refused++; *p = 0; return 2; }\n"
+                   "  if (!next) next = (int (*)(void **, size_t))dlsym(dlopen(\"libamdhip64.so.7\", RTLD_NOW), \"hipMalloc\");\n"
+                   "  return next(p, n);\n}\n")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"], check=True)
+    here = os.path.dirname(os.path.abspath(__file__))
+    root = os.path.dirname(here)
+    p = subprocess.run([sys.executable, "-c", _NO_STAGE, str(so), here, os.path.join(root, "oracle"),
+                        os.path.join(root, "collisional-hybrid_amd")], capture_output=True, text=True, timeout=100)
+    assert p.returncode == 0 and "STAGED" in p.stdout, p.stderr[-2000:]
