@@ -157,8 +157,8 @@ struct chy_ctx {
   chy_collision_stats *push_stats = nullptr;
   double *h_scale = nullptr;    // pinned: squared scales of the Krylov basis (GMRES)
   // FFT preconditioner
-  void *fft_buf = nullptr;      // complex work array
-  void *pc_buf = nullptr;       // z-line / Chebyshev / two-level scratch, 3 vectors (T)
+  void *fft_buf = nullptr;      // complex work array (multigrid: fields of the finest level)
+  void *pc_buf = nullptr;       // z-line / Chebyshev / two-level / multigrid scratch, 3 vectors (T)
   void *pc2_buf = nullptr;      // two-level FFT preconditioner: x-y fields (T)
   double *pc2_h = nullptr;      // its double workspace: column sums, partial sums
   void *zl_buf = nullptr;       // fft2z: z-line factors (4 nc values of T)

@@ -39,7 +39,6 @@ struct Mg {
   int nlev = 0;
   MgLevel lv[kMgMax];
   bool zfast = false;   // level fields as [y][x][z] (at most kMgMaxPlanes planes)
-  void *tmp = nullptr;  // z-line factors of a level before their transposition
 };
 
 // c = x-y full weighting of f (weights 1/4, 1/2, 1/4 along x and y, periodic).
@@ -182,10 +181,10 @@ int mg_setup(chy_ctx *ctx)
   M->nlev = level_sizes(p.N[0], p.N[1], sz);
   M->zfast = p.N[2] <= kMgMaxPlanes;
   const size_t ts = ctx->mixed ? 4 : 8;
-  if (M->zfast) {
-    unsigned char *q = nullptr;
-    TRY(dalloc(ctx, &q, (int64_t)ts * 4 * ctx->g.nc)); M->tmp = q;
-  }
+  // The finest level's fields but its factors lie in work arrays that the
+  // other preconditioners use: its density in the FFT's second half (a transposed
+  // solve's FFT overwrites it, and the next solve makes it anew).
+  unsigned char *pcb = (unsigned char *)ctx->pc_buf, *ffb = (unsigned char *)ctx->fft_buf;
   for (int l = 0; l < M->nlev; l++) {
     MgLevel &L = M->lv[l];
     Grid &g = L.g;
@@ -201,14 +200,17 @@ int mg_setup(chy_ctx *ctx)
     for (int a = 0; a < 3; a++) { g.d[a] = L.d[a]; g.rd[a] = 1.0 / L.d[a]; }
     const int64_t nc = g.nc, plane = (int64_t)g.nx * g.ny;
     unsigned char *q = nullptr;
-    TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.r = q;
     TRY(dalloc(ctx, &q, (int64_t)ts * 4 * nc)); L.zf = q;
     TRY(dalloc(ctx, &L.zcol, 2 * plane));
-    if (l > 0) { TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.n = q; }
-    if (l > 0 || M->zfast) {
-      TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.x = q;
-      TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.b = q;
+    if (l == 0) {
+      L.x = pcb; L.x2 = pcb + ts * nc; L.b = pcb + 2 * ts * nc;
+      L.r = ffb; L.nz = ffb + ts * nc;
+      continue;
     }
+    TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.r = q;
+    TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.n = q;
+    TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.x = q;
+    TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.b = q;
     if (M->zfast) {
       TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.nz = q;
       TRY(dalloc(ctx, &q, (int64_t)ts * nc)); L.x2 = q;
@@ -223,18 +225,20 @@ void mg_release(chy_ctx *ctx)
   if (!M) return;
   for (int l = 0; l < M->nlev; l++) {
     MgLevel &L = M->lv[l];
-    void *ps[] = {L.r, L.zf, L.zcol, l > 0 ? L.n : nullptr, L.x, L.b, L.nz, L.x2};
-    for (void *p : ps) if (p) (void)hipFree(p);
+    void *own[] = {L.zf, L.zcol}, *coarse[] = {L.r, L.n, L.x, L.b, L.nz, L.x2};
+    for (void *p : own) if (p) (void)hipFree(p);
+    if (l == 0) continue;
+    for (void *p : coarse) if (p) (void)hipFree(p);
   }
-  if (M->tmp) (void)hipFree(M->tmp);
   delete M;
   ctx->mg = nullptr;
 }
 
 int mg_levels(const chy_ctx *ctx) { return ctx->mg ? ((const Mg *)ctx->mg)->nlev : 0; }
 
-// Once per solve: the density of every level and the z-line factors of every
-// level's operator.
+// Once per solve, before the Krylov basis holds anything: the density of every
+// level and the z-line factors of every level's operator (made with x fastest in
+// the basis' first four vectors).
 template <typename T>
 int mg_prepare(chy_ctx *ctx, const T *n)
 {
@@ -246,7 +250,7 @@ int mg_prepare(chy_ctx *ctx, const T *n)
     if (l > 0)
       hipLaunchKernelGGL((k_mg_restrict<T, false>), nb_of(L.g.nc), kBlock, 0, ctx->stream, M->lv[l - 1].g, L.g,
                          (const T *)M->lv[l - 1].n, (T *)L.n);
-    T *zf = M->zfast ? (T *)M->tmp : (T *)L.zf;
+    T *zf = M->zfast ? (T *)ctx->V : (T *)L.zf;
     launch_zline_factor_g<T>(ctx, L.g, L.d, ctx->prm.lhs_type, (const T *)L.n, zf, L.zcol);
     if (M->zfast) {
       const int64_t nc = L.g.nc;

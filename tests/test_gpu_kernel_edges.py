@@ -1,5 +1,6 @@
 """Kernels at the sizes where their tiling can go wrong: block edges,
 remainders, the smallest grids and both sides of each dispatch rule."""
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -394,3 +395,25 @@ def test_ions_are_staged_without_device_memory_to_spare(tmp_path):
     p = subprocess.run([sys.executable, "-c", _NO_STAGE, str(so), here, os.path.join(root, "oracle"),
                         os.path.join(root, "collisional-hybrid_amd")], capture_output=True, text=True, timeout=100)
     assert p.returncode == 0 and "STAGED" in p.stdout, p.stderr[-2000:]
+
+
+# multigrid takes no more device memory than its z-line factors and its coarse
+# levels need: 4 fields of the finest grid and a third of 10 (the coarse levels'
+# nodes), with a third of a field and an allocation granule of 2 MiB for each
+# array to spare
+def test_multigrid_levels_share_the_work_arrays():
+    N = (256, 256, 128)
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def used(pc):
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        before = free.value
+        with context(opts(N, extra=f"-pc_type {pc} -ksp_gmres_restart 2"), capacity=1):
+            assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+            return before - free.value
+
+    used("jacobi")
+    extra = used("mg") - used("jacobi")
+    field = 8 * N[0] * N[1] * N[2]
+    assert extra <= (4 + 10 / 3 + 1 / 3) * field + 64 * 2 ** 21, extra / field
