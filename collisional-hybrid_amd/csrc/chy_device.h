@@ -101,12 +101,32 @@ __host__ __device__ __forceinline__ double div_rn(double a, double d, double rd)
   return __builtin_fma(__builtin_fma(-q, d, a), rd, q);
 }
 
+// The hardware's approximations of 1 / x and 1 / sqrt(x); on the host, where the
+// functions below are tested, the values moved by 2^-24 of themselves
+__host__ __device__ __forceinline__ double rcp_approx(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rcp(x);
+#else
+  return (1.0 + 0x1p-24) / x;
+#endif
+}
+
+__host__ __device__ __forceinline__ double rsq_approx(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_rsq(x);
+#else
+  return (1.0 + 0x1p-24) / __builtin_sqrt(x);
+#endif
+}
+
 // a / b for normal b (not 0) whose quotient neither over- nor underflows: the hardware's
 // reciprocal refined twice, then one exact remainder (the last bit may differ
 // from a / b's where that is a near tie)
-__device__ __forceinline__ double div_normal(double a, double b)
+__host__ __device__ __forceinline__ double div_normal(double a, double b)
 {
-  double y = __builtin_amdgcn_rcp(b);
+  double y = rcp_approx(b);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
   const double q = a * y;
@@ -171,13 +191,9 @@ __host__ __device__ __forceinline__ double log_unit(double u)
 #endif
   if (m < 0.70710678118654752440) { m *= 2.0; e -= 1; }
   const double f = m - 1.0, d = 2.0 + f;
-#if defined(__HIP_DEVICE_COMPILE__)
-  double y = __builtin_amdgcn_rcp(d);
+  double y = rcp_approx(d);
   y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
   y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
-#else
-  const double y = 1.0 / d;
-#endif
   double s = f * y;
   s = __builtin_fma(__builtin_fma(-d, s, f), y, s);
   const double z = s * s;
@@ -200,9 +216,9 @@ __host__ __device__ __forceinline__ double log_unit(double u)
 // sqrt(x) for normal positive x (zero for x = 0): the hardware's reciprocal
 // square root refined as the library does (two residuals from the exact x -
 // g^2), without its scaling for the ends of the exponent range.
-__device__ __forceinline__ double sqrt_normal(double x)
+__host__ __device__ __forceinline__ double sqrt_normal(double x)
 {
-  const double y = __builtin_amdgcn_rsq(x);
+  const double y = rsq_approx(x);
   double g = x * y, h = 0.5 * y;
   const double r = __builtin_fma(-h, g, 0.5);
   g = __builtin_fma(g, r, g);
