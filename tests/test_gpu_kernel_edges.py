@@ -417,3 +417,36 @@ def test_multigrid_levels_share_the_work_arrays():
     extra = used("mg") - used("jacobi")
     field = 8 * N[0] * N[1] * N[2]
     assert extra <= (4 + 10 / 3 + 1 / 3) * field + 64 * 2 ** 21, extra / field
+
+
+# the dot products that come with A z (up to 8 basis vectors, iterations 1 to 8) and
+# their sums in the update (nodes in fours), against the oracle's iterate after
+# as many steps: blocks of columns and groups of planes that are and are not
+# whole.  The least-squares step amplifies the basis' rounding, some 100 ulps, by
+# the conditioning of the preconditioned operator: 2.3e4 for the first, at most
+# 1.2e3 for the others (mixed: 250).  Products that miss one node move an FP64
+# iterate by 2e-6 at least, products that miss a plane or a part of a block any
+# iterate by 1e-2 (computed with a GMRES that leaves them out).
+_DOTS = [((5, 7, 3), "-pc_type jacobi", orc.PC_JACOBI), ((17, 16, 6), "-pc_type zline", orc.PC_ZLINE),
+         ((17, 15, 9), "-pc_type zline -B0x 1e-5 -B0y 2e-5", orc.PC_ZLINE), ((16, 16, 8), "-pc_type fft", orc.PC_FFT),
+         ((19, 14, 5), "-pc_type jacobi -B0x 1e-5 -B0y 2e-5", orc.PC_JACOBI)]
+
+
+@pytest.mark.parametrize("refine", ["NEVER", "ALWAYS"])
+@pytest.mark.parametrize("N,extra,pc,prec,tol", [(*d, "fp64", 1e-9) for d in _DOTS] + [(*d, "mixed", 2e-3) for d in _DOTS[1:4]])
+def test_gmres_iterates_with_the_operators_dot_products(N, extra, pc, prec, tol, refine):
+    with context(opts(N, extra=f"{extra} -ksp_rtol 1e-14 -ksp_inner_rtol 1e-7 -precision {prec} "
+                               f"-ksp_gmres_cgs_refinement_type REFINE_{refine}")) as ctx:
+        g = grid_of(ctx.prm)
+        mom = [m.astype(np.float32).astype(np.float64) for m in _moments(g, np.random.default_rng(19))]
+        ctx.set_moments(vlasov_from(mom))
+        K, b, phis = list(ctx.prm.kappa_e), ctx.compute_rhs(), {}
+        for k in (1, 2, 3, 5, 7, 8, 9, 10):
+            ctx.set_tolerances(max_it=k)
+            ctx.set_potential(np.zeros(g.nc))
+            phis[k], st = ctx.solve_potential()
+            assert (st.iterations, st.outer) == (k, 1)
+    for k, phi in phis.items():
+        ref, its, _, _ = orc.solve(g, K, mom[0], b, pc=pc, rtol=1e-14, max_it=k)
+        assert its == k
+        assert np.abs(phi - ref).max() <= tol * np.abs(ref).max(), k
