@@ -450,3 +450,21 @@ def test_gmres_iterates_with_the_operators_dot_products(N, extra, pc, prec, tol,
         ref, its, _, _ = orc.solve(g, K, mom[0], b, pc=pc, rtol=1e-14, max_it=k)
         assert its == k
         assert np.abs(phi - ref).max() <= tol * np.abs(ref).max(), k
+
+
+# the FP64 push's launch holds 2^24 ions: more take several trips, the last one
+# partly live, with each trip's ions loaded during the one before
+def test_fp64_push_in_several_trips():
+    test_fp64_push_of_any_number_of_ions((64, 64, 64), 2 ** 24 + 40003, 1e3)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_push_of_no_ions(prec):
+    with context(opts((5, 4, 3), extra=f"-precision {prec} -Np 0"), capacity=8) as ctx:
+        none = np.empty(0)
+        ctx.set_particles(none, none, none, none, none, none)
+        ctx.set_potential(np.random.default_rng(24).standard_normal(ctx.nc))
+        st = ctx.update_velocities()
+        ctx.update_positions()
+        assert (st.accepted, st.refused, ctx.num_particles()) == (0, 0, 0)
+        assert not ctx.collect_moments().any()
