@@ -468,3 +468,14 @@ def test_push_of_no_ions(prec):
         ctx.update_positions()
         assert (st.accepted, st.refused, ctx.num_particles()) == (0, 0, 0)
         assert not ctx.collect_moments().any()
+
+
+# the z-line stage on 16 columns where a block takes 32: FP32 columns of 65 to 256
+# planes, and the factors of columns beyond 128 planes in both precisions (the
+# other blocks take 16 columns, and planes with axes of 4, 8, 16.. nodes hold a
+# multiple of 16)
+@pytest.mark.parametrize("prec,base", [("fp64", 1e-11), ("mixed", 2e-5)])
+@pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5"])
+@pytest.mark.parametrize("N", [(4, 4, 128), (4, 4, 256)])
+def test_zline_stage_in_a_part_of_a_block(N, extra, prec, base):
+    test_zline_stage_on_columns_of_any_length(N, extra, prec, base)
