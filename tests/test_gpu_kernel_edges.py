@@ -107,7 +107,7 @@ def test_fft_passes_on_axes_of_any_length(N, extra, prec, base):
 # of the column stencil, and are added in the update's kernel where nodes come
 # in fours: 12 iterations (past 8 vectors) on node counts that are and are not
 # multiples of 4, ragged last blocks, and every kind of row; against a solve
-# that takes a second Gram-Schmidt pass and so the separate kernels.  Two
+# that takes a second Gram-Schmidt pass, and so sums them in a launch.  Two
 # converged solves at this tolerance differ by it times the conditioning of the
 # preconditioned operator (below 100), and by the FP64 residual's rounding.
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
@@ -172,9 +172,9 @@ def test_multigrid_columns_of_any_length(N, extra, prec, tol):
     assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
 
 
-# the z-line stage in segments: full and ragged columns of each segmentation,
-# planes that are no multiple of a block's 16 or 32 columns (x-y axes of a power
-# of two, as the preconditioner needs), and the column walk beyond 256 planes;
+# the z-line stage in segments: full and ragged columns of each segmentation
+# (x-y axes of a power of two, as the preconditioner needs, whose planes here fill
+# the blocks' 16 or 32 columns), and the column walk beyond 256 planes;
 # B along z (the 2-D correction folded in) and oblique (the plain stage)
 @pytest.mark.parametrize("prec,base", [("fp64", 1e-11), ("mixed", 2e-5)])
 @pytest.mark.parametrize("extra", ["", "-B0x 1e-5 -B0y 2e-5"])
@@ -199,8 +199,7 @@ def test_zline_stage_on_columns_of_any_length(N, extra, prec, base):
 
 # host arrays: one block and its neighbours, many ions on a grid whose Krylov
 # basis is too small a scratch for them (one staging piece, and several: 1.2 M
-# ions are 91 MB), and a field of 32 MiB and a bit, which comes back in pinned
-# chunks.  The values only change layout (and type, in mixed mode)
+# ions are 91 MB).  The values only change layout (and type, in mixed mode)
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("N,n", [((3, 3, 3), 1), ((4, 5, 6), 257), ((4, 4, 4), 70000), ((12, 10, 11), 1200000)])
 def test_ions_survive_the_host_round_trip(N, n, prec):
@@ -225,6 +224,7 @@ def test_ions_survive_the_host_round_trip(N, n, prec):
         assert np.array_equal(d[name][back], ref)
 
 
+# a potential of 16 MiB and a bit, and its moments, come back in pinned chunks
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("N", [(3, 3, 3), (7, 5, 9), (128, 128, 129)])
 def test_grid_arrays_survive_the_host_round_trip(N, prec):
@@ -238,9 +238,9 @@ def test_grid_arrays_survive_the_host_round_trip(N, prec):
         assert np.array_equal(ctx.get_potential(), phi)
 
 
-# the FP64 push carries its next ion along: no ion, one, a wave and its
-# neighbours, a block, and more ions than one trip of the largest grid; every
-# wave with and without colliders (nu_in 1e3 and 1e5 s^-1)
+# the FP64 push carries its next ion along: one ion, a wave and its neighbours, a
+# block, and several, all in one trip; waves with few and with many colliders
+# (nu_in 1e3 and 1e5 s^-1)
 @pytest.mark.parametrize("nui", [1e3, 1e5])
 @pytest.mark.parametrize("N,n", [((3, 3, 3), 1), ((5, 4, 3), 63), ((5, 4, 3), 65), ((4, 4, 4), 256), ((7, 5, 6), 1023),
                                  ((20, 20, 20), 40000)])
@@ -596,3 +596,27 @@ def test_a_small_field_comes_back_in_one_blocking_copy():
         get = least(lambda: chybrid.lib().chy_get_potential(ctx._p, out.ctypes.data))
         assert np.array_equal(out, phi)
     assert get <= 1.4 * copy, (get, copy)
+
+
+# the 2-D correction makes one Gram-Schmidt pass, the oracle two: in each of its
+# forms (planes in registers, in LDS and by launches) on densities that leave the
+# second direction nothing but rounding, and on one that varies twentyfold in x
+# and y; tolerances as in the test of any plane
+@pytest.mark.parametrize("prec,base", [("fp64", 1e-12), ("mixed", 2e-5)])
+@pytest.mark.parametrize("contrast", [0.0, 0.001, 0.95])
+@pytest.mark.parametrize("N", [(16, 16, 8), (8, 64, 8), (64, 64, 4)])
+def test_two_level_correction_at_any_contrast(N, contrast, prec, base):
+    rng = np.random.default_rng(27)
+    with context(opts(N, extra=f"-pc_type fft2 -precision {prec}")) as ctx:
+        g = grid_of(ctx.prm)
+        wave = np.sin(2 * np.pi * np.arange(N[0]) / N[0]) * np.cos(2 * np.pi * np.arange(N[1]) / N[1])[:, None]
+        n = (1 + contrast * np.broadcast_to(wave, N[::-1]).ravel()).astype(np.float32).astype(np.float64)
+        ctx.set_moments(vlasov_from([n] + 3 * [np.zeros(g.nc)]))
+        r = rng.standard_normal(g.nc)
+        r -= r.mean()
+        z = ctx.pc_apply(r)
+        K = list(ctx.prm.kappa_e)
+    tol = base + 16 * 2.0 ** -52 * (3 + K[2] ** 2) / (1 - np.cos(2 * np.pi / max(N)))
+    ref = orc.pc_apply(g, K, n, r, orc.PC_FFT2)
+    z, ref = z - z.mean(), ref - ref.mean()
+    assert np.abs(z - ref).max() <= tol * np.abs(ref).max()
