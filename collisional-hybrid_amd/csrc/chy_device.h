@@ -121,9 +121,10 @@ __host__ __device__ __forceinline__ double rsq_approx(double x)
 #endif
 }
 
-// a / b for normal b (not 0) whose quotient neither over- nor underflows: the hardware's
-// reciprocal refined twice, then one exact remainder (the last bit may differ
-// from a / b's where that is a near tie)
+// a / b for normal b (not 0) whose quotient neither over- nor underflows: two
+// Newton-Raphson steps y += y (1 - b y) on the hardware's reciprocal, and the
+// quotient a y corrected by its exact remainder, as in div_rn (the last bit may
+// differ from a / b's where that is a near tie)
 __host__ __device__ __forceinline__ double div_normal(double a, double b)
 {
   double y = rcp_approx(b);
@@ -175,11 +176,13 @@ __host__ __device__ __forceinline__ void sincos2pi(double u, double &s, double &
   c = ((q + 1) & 2) ? -cn : cn;
 }
 
-// log(u) for normal u in (0, 1): u = 2^e m, m in [1/sqrt 2, sqrt 2), f = m - 1,
-// s = f / (2 + f), log m = f - (f^2/2 - s (f^2/2 + R)), R the atanh series
-// 2/3 s^2 + 2/5 s^4 + ... (to s^18: below 3e-17 of the logarithm), log 2 in two
-// parts of which the first has few enough bits for e, and e log 2 + f - f^2/2 in
-// two parts: rounded to nearest but for 0.7 % of the arguments.
+// log(u) for normal u in (0, 1): u = 2^e m, m in [1/sqrt 2, sqrt 2), and with f =
+// m - 1, s = f / (2 + f) = (m - 1) / (m + 1) the series log m = 2 atanh s = 2 s + s
+// R, R = 2/3 s^2 + 2/5 s^4 + ... (Abramowitz and Stegun, 4.1.27; to s^18: below
+// 3e-17 of the logarithm).  Its leading term is not exact: since s (2 + f) = f,
+// with h = f^2 / 2, 2 s = f - s f = f - h + s h, whose large terms are.  log 2 is
+// in two parts of which the first has few enough bits for e, and e log 2 + f - h
+// in two parts: rounded to nearest but for 0.7 % of the arguments.
 __host__ __device__ __forceinline__ double log_unit(double u)
 {
   int e;
@@ -213,9 +216,12 @@ __host__ __device__ __forceinline__ double log_unit(double u)
   return t2 + (t2l + (t1l + __builtin_fma(s, h + R, __builtin_fma(ed, 4.7493250390316726e-07, -hl))));
 }
 
-// sqrt(x) for normal positive x (zero for x = 0): the hardware's reciprocal
-// square root refined as the library does (two residuals from the exact x -
-// g^2), without its scaling for the ends of the exponent range.
+// sqrt(x) for normal positive x, 0 for all others, NaN among them (under the
+// kinematics' roots rounding may leave a little less than 0; an ion's NaN is
+// seen where its state is stored): Goldschmidt's coupled iteration for g = sqrt x
+// and h = 1 / (2 sqrt x) from the hardware's reciprocal root, one step (Goldschmidt,
+// "Applications of division by convergence", 1964), then g twice corrected by
+// its exact remainder, g += h (x - g^2) (Markstein).
 __host__ __device__ __forceinline__ double sqrt_normal(double x)
 {
   const double y = rsq_approx(x);

@@ -2207,9 +2207,11 @@ __global__ __launch_bounds__(NC * SG) void k_zline_seg(Grid g, const T *__restri
 // - A x), the residual never stored: 4 to 6 us on 96 x 80 x 50 and its coarse
 // levels (FP32), where with x fastest it took a residual pass (4 to 6 us) and a
 // solve (16.6 us walking 96 x 80 columns, 4.6 us on fewer).  A preconditioner
-// application there went from 65 launches to 43.  Whole solves: 96 x 80 x 50
-// mixed 26.1 -> 14.6 ms, 64 x 48 x 40 FP64 21.7 -> 12.8, 160 x 144 x 100 mixed
-// 8.9 -> 5.7, 256^3 mixed 22.7 -> 17.9.  What is left is latency: one launch
+// application there went from 65 launches to 38, 339 -> 149 us.  Whole solves
+// with a run's noise, to 1e-10 (mixed) and 1e-11, B oblique: 96 x 80 x 50 mixed
+// 29.3 -> 12.4 ms, 64 x 48 x 40 FP64 23.9 -> 10.4, 160 x 144 x 100 mixed 89.7 ->
+// 38.8; B along z: 160 x 144 x 100 mixed 10.3 -> 4.8, 256^3 mixed 26.0 -> 16.1
+// (all of the solver's changes in them).  What is left is latency: one launch
 // after another on grids that a chip of 256 CUs does in a microsecond or two.
 // (All sweeps of the coarsest level in one workgroup, in LDS and registers,
 // took 27 to 52 us against 8 launches of 4 to 5: the scans' instructions
@@ -2928,7 +2930,12 @@ void launch_zline_factor_g(chy_ctx *ctx, const Grid &g, const double d[3], int l
                      zbuf + nc, zbuf + 2 * nc, zbuf + 3 * nc, colbuf, colbuf + plane);
 }
 
-// res = b - A(n) x on grid g with spacings d, precision T (multigrid levels)
+// res = b - A(n) x on grid g with spacings d, precision T (multigrid levels of
+// columns beyond kMgMaxPlanes).  Where the column stencil does not take a grid, the
+// tiles do also on small planes: a thread a node is level with them on thin ones
+// and slower on others (twelve iterations, ms, tiles / nodes: FP64 36 x 4 x 20000
+// 513 / 514, 16 x 16 x 36000 1936 / 1933, 64 x 64 x 600 55.2 / 57.0, 128 x 128 x
+// 1000 129 / 149; mixed 461 / 461, 1786 / 1783, 41.5 / 41.7, 91.5 / 103)
 template <typename T>
 void launch_residual_g(chy_ctx *ctx, const Grid &g, const double d[3], int lhs_type, const T *n, const T *b,
                        const T *x, T *res)
