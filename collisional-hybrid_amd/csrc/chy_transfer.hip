@@ -166,7 +166,7 @@ static int moments_copy(chy_ctx *ctx, double *v, bool in)
     }
   }
   CHY_HIP(hipGetLastError());
-  CHY_HIP(hipStreamSynchronize(ctx->stream));
+  if (in) CHY_HIP(hipStreamSynchronize(ctx->stream));  // (copies to the host are complete)
   return CHY_OK;
 }
 
